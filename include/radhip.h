@@ -248,7 +248,7 @@ int rad_debug_bins(rad_ctx *ctx, uint32_t *out_or_null, uint32_t *ntiles, uint32
  * spill region, [6] triangle-faces queued for clipping, [7] nonzero if an
  * earlier pass overflowed.  Capacities: out_caps (optional, 3 entries) gets
  * the spill capacity, the bin-entry capacity and the clip-queue capacity.
- * A pass of 16 or more slots renders as two halves, each with these
+ * A large pass renders as two halves, each with these
  * capacities: [3], [5] and [6] are then the fuller half's, [4] the sum. */
 int rad_debug_counters(rad_ctx *ctx, uint32_t *out8, uint32_t *out_caps_or_null);
 

@@ -4,7 +4,8 @@
 // sequence of device kernels on the context stream with no host
 // synchronisation between passes: select -> prepare -> clear -> raster setup
 // -> raster tiles -> reduce -> shoot; the raster stages of a pass of 16 or
-// more slots run as two halves on the context's two streams.
+// more slots and 8,192 or more bins run as two halves on the context's two
+// streams.
 #include <cstddef>
 #include <hip/hip_runtime.h>
 
@@ -101,9 +102,13 @@ void record(rad_ctx *c, size_t idx)
         (void)hipEventRecord(c->ev[idx], c->st);
 }
 
-// A pass of 16 or more slots renders as two halves side by side, except a
-// timed one (stage events bracket whole stages).
-static bool split_render(const rad_ctx *c, uint32_t k) { return k >= kSplitMin && !c->timing; }
+// A pass of kSplitMin or more slots and kSplitBins or more bins renders as
+// two halves side by side, except a timed one (stage events bracket whole
+// stages).
+static bool split_render(const rad_ctx *c, uint32_t k)
+{
+    return k >= kSplitMin && k * c->bb.ntiles >= kSplitBins && !c->timing;
+}
 
 // First slot of the second half of a split pass.
 static uint32_t split_at(uint32_t k) { return k / 2; }
@@ -148,7 +153,7 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
                         ids || fq ? nullptr : c->ff, fq ? c->ffq : nullptr, hits, c->counters,
                         c->pk.slot_w, c->pk.slot_dffo, c->fblk, c->K, st);
     };
-    // A pass of 16 or more slots renders as two halves side by side: the
+    // A large pass renders as two halves side by side (split_render): the
     // halves share no bins, records, list entries or counters, so the item
     // buffers and F rows are those of one launch over all slots.  Timed
     // passes stay whole so that the stage events bracket every kernel.
@@ -298,8 +303,6 @@ int set_tiles(rad_ctx *c, uint32_t T, uint32_t small_px)
     if (c->st)
         (void)hipStreamSynchronize(c->st);
     c->bb.tshift = T == 8 ? 3 : (T == 16 ? 4 : 5);
-    if (!c->bb.setup_group)
-        c->bb.setup_group = c->K >= 8 ? 8u : c->K;
     c->bb.ntx = ntx;
     c->bb.nty = nty;
     c->bb.ntiles = ntx * nty;
@@ -550,6 +553,10 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     // spill region; bin entries: three per record slot
     c->bb.nblk = nblk ? nblk : 1;
     c->bb.nz = K <= 4 ? 5u : 1u;
+    c->bb.setup_group = 8;
+    while (c->bb.setup_group > 1 &&
+           (uint64_t)c->bb.nblk * c->bb.nz * K < (uint64_t)kSetupGroups * c->bb.setup_group)
+        c->bb.setup_group /= 2;
     uint64_t regions = (uint64_t)c->bb.nblk * K * c->bb.nz * kRecsPerBlock;
     uint64_t spill = regions / 8 + 65536;
     if (regions + kCntBlocks * spill > (1ull << 31))

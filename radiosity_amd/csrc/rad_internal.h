@@ -55,6 +55,21 @@ enum {
 // queue and list area; the sticky flag lives in the first block.
 constexpr int kCntBlocks = 2;
 constexpr uint32_t kSplitMin = 16; // smallest pass rendered as two halves
+// ... and the fewest bins (slots x tiles): the halves overlap each other's
+// tails, which pays for the two streams' fork and join (5-12 us per edge)
+// only where the tile kernel runs long.  A pass of 64 shooters at hemicube 256
+// (12,288 bins), whole against halves: 50,000 triangles 262 -> 245 us, 100,000
+// 303 -> 283, 200,000 398 -> 379; at hemicube 128 (3,072 bins) 194 both ways;
+// 32 shooters at hemicube 256 (6,144) 277 -> 279; 20 at hemicube 128 247 -> 263;
+// 16 at hemicube 64 82 -> 93.
+constexpr uint32_t kSplitBins = 8192;
+// Workgroups the setup and the bin fill should have before each walks more
+// than one shooter slot (then up to 8, which reads the vertices once per 8
+// shooters).  About five per CU are resident; walking 8 slots whatever the
+// scene left most CUs idle below 200,000 triangles.  A pass of 64 shooters,
+// hemicube 128: 16,384 triangles 155 us at 8 slots a workgroup (512
+// workgroups), 122 us at 2 (2,048); 200,000 triangles (50,000 pairs) keep 8.
+constexpr uint32_t kSetupGroups = 1200;
 
 // Control block of a context (u32 words on the device), written by the
 // shoot kernels and read by the pass gate in k_prepare_clear:

@@ -28,6 +28,7 @@
 // which is the fragment GL_LESS keeps when triangles are drawn in id order
 // (Main.cpp:1104, DrawPatchLook Main.cpp:720).
 #include "rad_internal.h"
+#include "rad_topk.h"
 
 #include <hip/hip_runtime.h>
 
@@ -2528,120 +2529,6 @@ __device__ static inline void count_pass(uint32_t *__restrict__ ctl, uint32_t n)
     *(unsigned long long *)(ctl + kCtlShotLo) += n;
 }
 
-// Lane exchanges of the top-K networks without ds_bpermute: lane i gets the
-// value of lane i ^ M, from DPP lane moves (strides 1, 2, 4, 8 inside a row
-// of 16 lanes) and the gfx950 row and half-wave swaps (16, 32).
-template <int M> __device__ __forceinline__ uint32_t lane_xor(uint32_t x)
-{
-    const int lane = threadIdx.x & 63;
-    const int xi = (int)x;
-    if constexpr (M == 1) {
-        return (uint32_t)__builtin_amdgcn_update_dpp(xi, xi, 0xB1, 0xF, 0xF, false); // quad_perm 1,0,3,2
-    } else if constexpr (M == 2) {
-        return (uint32_t)__builtin_amdgcn_update_dpp(xi, xi, 0x4E, 0xF, 0xF, false); // quad_perm 2,3,0,1
-    } else if constexpr (M == 4) {
-        const int up = __builtin_amdgcn_update_dpp(xi, xi, 0x104, 0xF, 0xF, false); // row_shl:4, lane i + 4
-        const int dn = __builtin_amdgcn_update_dpp(xi, xi, 0x114, 0xF, 0xF, false); // row_shr:4, lane i - 4
-        return (uint32_t)((lane & 4) ? dn : up);
-    } else if constexpr (M == 8) {
-        return (uint32_t)__builtin_amdgcn_update_dpp(xi, xi, 0x128, 0xF, 0xF, false); // row_ror:8
-    } else if constexpr (M == 16) {
-        // odd rows of the first operand swap with even rows of the second:
-        // r[0] holds rows (0, 0, 2, 2) of x, r[1] rows (1, 1, 3, 3)
-        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
-        return (lane & 16) ? r[0] : r[1];
-    } else {
-        static_assert(M == 32, "lane_xor strides 1 .. 32");
-        // the upper half of the first operand swaps with the lower half of
-        // the second: r[0] holds x's lower half twice, r[1] its upper half
-        const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
-        return (lane & 32) ? r[0] : r[1];
-    }
-}
-
-template <int M> __device__ __forceinline__ uint64_t lane_xor_u64(uint64_t v)
-{
-    return ((uint64_t)lane_xor<M>((uint32_t)(v >> 32)) << 32) | lane_xor<M>((uint32_t)v);
-}
-
-// The value of lane 63 - i: each row mirrored (row_mirror), then rows
-// r and 3 - r exchanged.
-__device__ __forceinline__ uint64_t lane_reverse_u64(uint64_t v)
-{
-    const int lo = __builtin_amdgcn_update_dpp((int)v, (int)v, 0x140, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp((int)(v >> 32), (int)(v >> 32), 0x140, 0xF, 0xF, false);
-    const uint64_t m = ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
-    return lane_xor_u64<32>(lane_xor_u64<16>(m));
-}
-
-// A wave-uniform lane's value (lane src, a constant).
-__device__ __forceinline__ uint64_t lane_read_u64(uint64_t v, int src)
-{
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, src);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), src);
-    return ((uint64_t)hi << 32) | lo;
-}
-
-// One compare-exchange step of a bitonic network at lane stride M.
-template <int M> __device__ __forceinline__ uint64_t bitonic_step(uint64_t v, bool take_max)
-{
-    const uint64_t o = lane_xor_u64<M>(v);
-    return take_max ? (v > o ? v : o) : (v < o ? v : o);
-}
-
-__device__ __forceinline__ uint64_t wave_sort_desc(uint64_t v)
-{
-    const int lane = threadIdx.x & 63;
-    // stage `size`: lanes in blocks of size sort descending where
-    // lane & size == 0; a step at stride m keeps the max in the lower lane
-    // of a pair when that block is descending
-#define RAD_SORT_STEP(size_, m_) \
-    v = bitonic_step<m_>(v, ((lane & (m_)) == 0) == ((lane & (size_)) == 0));
-    RAD_SORT_STEP(2, 1)
-    RAD_SORT_STEP(4, 2) RAD_SORT_STEP(4, 1)
-    RAD_SORT_STEP(8, 4) RAD_SORT_STEP(8, 2) RAD_SORT_STEP(8, 1)
-    RAD_SORT_STEP(16, 8) RAD_SORT_STEP(16, 4) RAD_SORT_STEP(16, 2) RAD_SORT_STEP(16, 1)
-    RAD_SORT_STEP(32, 16) RAD_SORT_STEP(32, 8) RAD_SORT_STEP(32, 4) RAD_SORT_STEP(32, 2)
-    RAD_SORT_STEP(32, 1)
-    RAD_SORT_STEP(64, 32) RAD_SORT_STEP(64, 16) RAD_SORT_STEP(64, 8) RAD_SORT_STEP(64, 4)
-    RAD_SORT_STEP(64, 2) RAD_SORT_STEP(64, 1)
-#undef RAD_SORT_STEP
-    return v;
-}
-
-// top and b sorted descending over the lanes: the top 64 of both, sorted.
-__device__ __forceinline__ uint64_t wave_merge_desc(uint64_t top, uint64_t b)
-{
-    const int lane = threadIdx.x & 63;
-    const uint64_t r = lane_reverse_u64(b);
-    uint64_t v = top > r ? top : r;
-    v = bitonic_step<32>(v, (lane & 32) == 0);
-    v = bitonic_step<16>(v, (lane & 16) == 0);
-    v = bitonic_step<8>(v, (lane & 8) == 0);
-    v = bitonic_step<4>(v, (lane & 4) == 0);
-    v = bitonic_step<2>(v, (lane & 2) == 0);
-    v = bitonic_step<1>(v, (lane & 1) == 0);
-    return v;
-}
-
-// The sorted 64-key lists of the workgroup's waves (top) merged pairwise
-// through wl; wave 0 returns the 64 largest keys of all of them.  Every
-// thread of the workgroup calls it.
-__device__ static uint64_t merge_wave_lists(uint64_t top, uint64_t (*wl)[64])
-{
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    wl[w][lane] = top;
-    for (int h = nw >> 1; h >= 1; h >>= 1) {
-        __syncthreads();
-        if (w < h)
-            top = wave_merge_desc(wl[w][lane], wl[w + h][lane]);
-        __syncthreads();
-        if (w < h)
-            wl[w][lane] = top;
-    }
-    return top;
-}
-
 // The 64 largest keys of the sorted 64-key lists [l0, l1) by the
 // workgroup's waves: each wave merges every nw-th list, loading 16 of them
 // at a time (a list whose largest key is not above the 64th of the wave's
@@ -3464,105 +3351,182 @@ size_t topk_cand_half(uint32_t npatch, uint32_t k)
 // ModelContainer.cpp:263-298 simulated exactly by one workgroup.  The
 // list's last (smallest) key never decreases during the scan, so a chunk's
 // candidates can be prefiltered in parallel against the value at the chunk
-// start; the survivors are then inserted one by one in index order by lane 0
-// with the list's push_back / stable sort / reverse / truncate semantics:
-// every run of equal keys reverses its order and the new element goes
-// first among its equals.
-__global__ __launch_bounds__(256) void k_select_reference(const float *__restrict__ unshot,
-                                                          uint32_t npatch, uint32_t k,
-                                                          uint32_t *__restrict__ shooters,
-                                                          uint32_t *__restrict__ nshoot)
+// start; the survivors are then inserted one by one in index order by the
+// first wavefront with the list's push_back / stable sort / reverse /
+// truncate semantics: every run of equal keys reverses its order and the new
+// element goes first among its equals.
+//
+// Serial by its nature (an insertion decides the next test), so what counts
+// is the time of one insertion: the list is held one entry per lane (R per
+// lane beyond 64), every entry finds its new place from ballots of the run
+// starts, the list is permuted through LDS, and the next candidate the list
+// takes is found by one ballot.  772 patches, K = 10: 16 us, where one lane
+// moving the entries one by one through LDS took 180.
+constexpr uint32_t kRefThreads = 1024;
+
+template <int R>
+__device__ static inline void reference_insert(float (&key)[R], uint32_t (&id)[R], uint32_t &n,
+                                               uint32_t k, float ek, uint32_t eid, float *lk,
+                                               uint32_t *li)
 {
-    __shared__ uint32_t tid_[RAD_MAX_K + 1], tmp_id[RAD_MAX_K + 1];
-    __shared__ float tkey[RAD_MAX_K + 1], tmp_key[RAD_MAX_K + 1];
-    __shared__ uint32_t cand[256];
-    __shared__ uint32_t ncand, n;
-    if (threadIdx.x == 0)
-        n = 0;
-    __syncthreads();
-    for (uint32_t base = 0; base < npatch; base += blockDim.x) {
-        float back = n ? tkey[n - 1] : 0.0f;
-        bool empty = n == 0;
-        if (threadIdx.x == 0)
-            ncand = 0;
-        __syncthreads();
-        uint32_t j = base + threadIdx.x;
-        float e = 0.f;
-        bool c = false;
-        if (j < npatch) {
-            float u0 = unshot[3 * (size_t)j], u1 = unshot[3 * (size_t)j + 1],
-                  u2 = unshot[3 * (size_t)j + 2];
-            e = u0 * u0 + u1 * u1 + u2 * u2;
-            c = (empty && j == base) || (e > 0 && back <= e);
+    const uint32_t lane = threadIdx.x & 63u;
+    uint64_t head[R];
+    uint32_t p = 0; // the new element's place: after every larger key
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t i = (uint32_t)r * 64u + lane;
+        float prev = __shfl_up(key[r], 1, 64);
+        if (r > 0 && lane == 0)
+            prev = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(key[r ? r - 1 : 0]), 63));
+        head[r] = __ballot(i < n && (i == 0 || key[r] != prev));
+        p += (uint32_t)__popcll(__ballot(i < n && key[r] > ek));
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t i = (uint32_t)r * 64u + lane;
+        const uint64_t upto = (2ull << lane) - 1ull;
+        // the entry's run of equal keys [g0, g1), reversed
+        uint32_t g0 = 0, g1 = n;
+        bool found = false;
+#pragma unroll
+        for (int q = r; q >= 0; --q) {
+            const uint64_t m = q == r ? head[q] & upto : head[q];
+            if (!found && m) {
+                g0 = (uint32_t)q * 64u + 63u - (uint32_t)__clzll(m);
+                found = true;
+            }
         }
-        // compact candidates in index order with a ballot per wave
-        uint64_t m = __ballot(c);
-        __shared__ uint32_t wcnt[4];
-        int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        found = false;
+#pragma unroll
+        for (int q = r; q < R; ++q) {
+            const uint64_t m = q == r ? head[q] & ~upto : head[q];
+            if (!found && m) {
+                g1 = (uint32_t)q * 64u + (uint32_t)__ffsll((long long)m) - 1u;
+                found = true;
+            }
+        }
+        const uint32_t to = g0 + g1 - 1u - i + (key[r] <= ek ? 1u : 0u);
+        if (i < n && to < k) {
+            lk[to] = key[r];
+            li[to] = id[r];
+        }
+    }
+    if (lane == 0 && p < k) {
+        lk[p] = ek;
+        li[p] = eid;
+    }
+    n = n < k ? n + 1u : k;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        key[r] = lk[r * 64 + (int)lane];
+        id[r] = li[r * 64 + (int)lane];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int R>
+__global__ __launch_bounds__(kRefThreads) void k_select_reference(
+    const float *__restrict__ unshot, uint32_t npatch, uint32_t k, uint32_t *__restrict__ shooters,
+    uint32_t *__restrict__ nshoot)
+{
+    __shared__ float lk[64 * R], ck[kRefThreads];
+    __shared__ uint32_t li[64 * R], ci[kRefThreads];
+    __shared__ uint32_t wcnt[kRefThreads / 64];
+    __shared__ float sback;
+    __shared__ uint32_t sn;
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    float key[R]; // the list, in the first wavefront
+    uint32_t id[R], n = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        key[r] = 0.0f;
+        id[r] = 0u;
+    }
+    if (threadIdx.x < 64 * R) {
+        lk[threadIdx.x] = 0.0f;
+        li[threadIdx.x] = 0u;
+    }
+    if (threadIdx.x == 0) {
+        sback = 0.0f;
+        sn = 0u;
+    }
+    auto energy = [&](uint32_t j) {
+        if (j >= npatch)
+            return 0.0f;
+        const float u0 = unshot[3 * (size_t)j], u1 = unshot[3 * (size_t)j + 1],
+                    u2 = unshot[3 * (size_t)j + 2];
+        return u0 * u0 + u1 * u1 + u2 * u2;
+    };
+    float e = energy(threadIdx.x);
+    __syncthreads();
+    for (uint32_t base = 0; base < npatch; base += kRefThreads) {
+        const uint32_t j = base + threadIdx.x;
+        const bool c = j < npatch && ((sn == 0 && j == base) || (e > 0 && sback <= e));
+        // the candidates in index order
+        const uint64_t m = __ballot(c);
         if (lane == 0)
-            wcnt[w] = __popcll(m);
+            wcnt[w] = (uint32_t)__popcll(m);
         __syncthreads();
-        uint32_t off = 0;
-        for (int q = 0; q < w; ++q)
-            off += wcnt[q];
-        if (c)
-            cand[off + __popcll(m & ((1ull << lane) - 1))] = j;
-        if (threadIdx.x == 0)
-            ncand = wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
+        uint32_t off = 0, total = 0;
+        for (uint32_t q = 0; q < kRefThreads / 64; ++q) {
+            off += q < w ? wcnt[q] : 0u;
+            total += wcnt[q];
+        }
+        if (c) {
+            const uint32_t o = off + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            ci[o] = j;
+            ck[o] = e;
+        }
+        e = energy(base + kRefThreads + threadIdx.x); // the next chunk's
         __syncthreads();
-        if (threadIdx.x == 0) {
-            for (uint32_t q = 0; q < ncand; ++q) {
-                uint32_t pi = cand[q];
-                float u0 = unshot[3 * (size_t)pi], u1 = unshot[3 * (size_t)pi + 1],
-                      u2 = unshot[3 * (size_t)pi + 2];
-                float ek = u0 * u0 + u1 * u1 + u2 * u2;
-                if (!(n == 0 || (ek > 0 && tkey[n - 1] <= ek)))
-                    continue;
-                // result: groups in descending key order; each existing group
-                // reversed; the new element first in its group
-                uint32_t m2 = 0;
-                bool placed = false;
-                uint32_t g0 = 0;
-                while (g0 < n || !placed) {
-                    if (!placed && (g0 >= n || tkey[g0] <= ek)) {
-                        // groups with key > ek are done; the new element's group
-                        tmp_id[m2] = pi;
-                        tmp_key[m2] = ek;
-                        ++m2;
-                        placed = true;
-                        continue;
-                    }
-                    uint32_t g1 = g0;
-                    while (g1 < n && tkey[g1] == tkey[g0])
-                        ++g1;
-                    for (uint32_t q2 = g1; q2 > g0; --q2) {
-                        tmp_id[m2] = tid_[q2 - 1];
-                        tmp_key[m2] = tkey[q2 - 1];
-                        ++m2;
-                    }
-                    g0 = g1;
+        if (w == 0 && total) {
+            // 64 candidates at a time, one per lane: the next one the list
+            // takes is the first lane left whose key reaches its back
+            float back = sback;
+            for (uint32_t q0 = 0; q0 < total; q0 += 64u) {
+                const bool in = q0 + lane < total;
+                const float ek = in ? ck[q0 + lane] : 0.0f;
+                const uint32_t ei = in ? ci[q0 + lane] : 0u;
+                uint64_t left = __ballot(in);
+                while (true) {
+                    const uint64_t m = left & __ballot(n == 0 || (ek > 0 && back <= ek));
+                    if (!m)
+                        break;
+                    const int l = __ffsll((long long)m) - 1;
+                    left = m & (m - 1u);
+                    reference_insert<R>(
+                        key, id, n, k,
+                        __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ek), l)),
+                        (uint32_t)__builtin_amdgcn_readlane((int)ei, l), lk, li);
+                    back = lk[n - 1u];
                 }
-                if (m2 > k)
-                    m2 = k;
-                for (uint32_t q2 = 0; q2 < m2; ++q2) {
-                    tid_[q2] = tmp_id[q2];
-                    tkey[q2] = tmp_key[q2];
-                }
-                n = m2;
+            }
+            if (lane == 0) {
+                sback = back;
+                sn = n;
             }
         }
         __syncthreads();
     }
-    for (uint32_t i = threadIdx.x; i < k; i += blockDim.x)
-        shooters[i] = i < n ? tid_[i] : 0u;
+    for (uint32_t i = threadIdx.x; i < k; i += kRefThreads)
+        shooters[i] = i < sn ? li[i] : 0u;
     if (threadIdx.x == 0)
-        *nshoot = n;
+        *nshoot = sn;
 }
 
 void launch_select_reference(const float *unshot, uint32_t npatch, uint32_t k, uint32_t *shooters,
                              uint32_t *nshoot, hipStream_t st)
 {
-    k_select_reference<<<1, 256, 0, st>>>(unshot, npatch, k, shooters, nshoot);
+    static_assert(RAD_MAX_K <= 256, "four list entries per lane");
+    if (k <= 64)
+        k_select_reference<1><<<1, kRefThreads, 0, st>>>(unshot, npatch, k, shooters, nshoot);
+    else
+        k_select_reference<4><<<1, kRefThreads, 0, st>>>(unshot, npatch, k, shooters, nshoot);
 }
 
 } // namespace rad

@@ -8,31 +8,67 @@
 // the shoot kernel applies a scene's slots to that scene's receivers.  One
 // pass is therefore one launch of each kernel for all scenes together.
 #include "rad_internal.h"
+#include "rad_topk.h"
 
 namespace rad {
 
 // Per-scene selection: one workgroup per scene.  FP64 residual
 // sum_A (r+g+b)(unshot) / den; a scene at or below the target is done (the
 // pass it finished in is kept); otherwise its k shooters are the top-k by
-// A_i (r+g+b) with ties to the lower index, found by k rounds of a block
-// max over packed keys (power bits << 32 | ~index), each round below the
-// previous key.  Zero-power patches are never chosen.
-__global__ __launch_bounds__(256) void k_pack_select(
+// A_i (r+g+b) with ties to the lower index.  Zero-power patches are never
+// chosen.
+//
+// One pass over the scene's patches gives the residual and the 64 largest
+// packed keys (power bits << 32 | ~index): each wavefront keeps a sorted
+// list, one key per lane, that takes the keys above its k-th, then the lists
+// merge pairwise.  32 rooms of 500-20,000 patches wanting up to 10 shooters:
+// 23 us, where a block maximum per shooter, each over the whole scene
+// again, took 158.  Shooters past the 64th (a scene may ask for up to 256)
+// are still found by rounds of block maxima below the previous key.
+constexpr uint32_t kPackSelThreads = 1024;
+
+__global__ __launch_bounds__(kPackSelThreads) void k_pack_select(
     const uint32_t *__restrict__ sc_pbeg, const uint32_t *__restrict__ sc_slots,
     const double *__restrict__ sc_den, const float *__restrict__ unshot,
     const float *__restrict__ area, const uint32_t *__restrict__ pass, double target,
     uint32_t kmax, uint32_t *__restrict__ sc_done, double *__restrict__ sc_res,
     uint32_t *__restrict__ sc_nsel, uint32_t *__restrict__ sc_shot, uint32_t *__restrict__ cand)
 {
-    __shared__ double dred[4];
-    __shared__ uint64_t kred[4];
+    constexpr uint32_t NW = kPackSelThreads / 64;
+    __shared__ double dred[NW];
+    __shared__ uint64_t wl[NW][64];
+    __shared__ uint64_t last;
     const uint32_t sc = blockIdx.x;
     const uint32_t pb = sc_pbeg[sc], pe = sc_pbeg[sc + 1];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    auto key_of = [](float p, uint32_t j) {
+        return p > 0.0f ? ((uint64_t)__float_as_uint(p) << 32) | (uint64_t)(~j) : 0ull;
+    };
     double num = 0.0;
-    for (uint32_t j = pb + threadIdx.x; j < pe; j += blockDim.x) {
-        const float *u = unshot + 3 * (size_t)j;
-        num += (double)area[j] * ((double)u[0] + (double)u[1] + (double)u[2]);
+    const uint32_t k = sc_slots[sc] < kmax ? sc_slots[sc] : kmax;
+    const int kl = (int)(k < 64u ? k : 64u);
+    uint64_t top = 0, thr = 0; // thr: the list's kl-th key
+    constexpr int kLoads = 4; // batches of a wavefront loaded at once
+    for (uint32_t b = pb + (uint32_t)w * 64u; b < pe; b += kLoads * kPackSelThreads) {
+        float u0[kLoads], u1[kLoads], u2[kLoads], ar[kLoads];
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q) {
+            const uint32_t j = b + (uint32_t)q * kPackSelThreads + (uint32_t)lane;
+            const bool in = j < pe;
+            const float *u = unshot + 3 * (size_t)(in ? j : pb);
+            u0[q] = in ? u[0] : 0.0f;
+            u1[q] = in ? u[1] : 0.0f;
+            u2[q] = in ? u[2] : 0.0f;
+            ar[q] = in ? area[j] : 0.0f;
+        }
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q) {
+            const uint32_t j = b + (uint32_t)q * kPackSelThreads + (uint32_t)lane;
+            num += (double)ar[q] * ((double)u0[q] + (double)u1[q] + (double)u2[q]);
+            const uint64_t key = key_of(ar[q] * (u0[q] + u1[q] + u2[q]), j);
+            if (__ballot(key > thr))
+                wave_take_desc(top, thr, key, kl);
+        }
     }
     for (int o = 32; o > 0; o >>= 1)
         num += __shfl_down(num, o, 64);
@@ -40,7 +76,10 @@ __global__ __launch_bounds__(256) void k_pack_select(
         dred[w] = num;
     __syncthreads();
     const double den = sc_den[sc];
-    const double res = den > 0.0 ? (dred[0] + dred[1] + dred[2] + dred[3]) / den : 0.0;
+    double sum = 0.0;
+    for (uint32_t q = 0; q < NW; ++q)
+        sum += dred[q];
+    const double res = den > 0.0 ? sum / den : 0.0;
     const bool done = sc_done[sc] != 0xFFFFFFFFu || res <= target;
     __syncthreads();
     if (done) {
@@ -52,37 +91,44 @@ __global__ __launch_bounds__(256) void k_pack_select(
         }
         return;
     }
-    const uint32_t k = sc_slots[sc] < kmax ? sc_slots[sc] : kmax;
-    uint64_t prev = ~0ull;
+    top = merge_wave_lists(top, wl);
     uint32_t nsel = 0;
-    for (uint32_t r = 0; r < k; ++r) {
-        uint64_t best = 0;
-        for (uint32_t j = pb + threadIdx.x; j < pe; j += blockDim.x) {
-            const float *u = unshot + 3 * (size_t)j;
-            float p = area[j] * (u[0] + u[1] + u[2]);
-            if (!(p > 0.0f))
-                continue;
-            uint64_t key = ((uint64_t)__float_as_uint(p) << 32) | (uint64_t)(~j);
-            if (key < prev && key > best)
-                best = key;
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            uint64_t v = __shfl_down(best, o, 64);
-            best = v > best ? v : best;
-        }
-        if (lane == 0)
-            kred[w] = best;
+    if (w == 0) {
+        const bool ok = (uint32_t)lane < k && top != 0;
+        if (ok)
+            cand[(size_t)sc * kmax + (uint32_t)lane] = ~(uint32_t)(top & 0xFFFFFFFFull);
+        nsel = (uint32_t)__popcll(__ballot(ok));
+        if (lane == 63)
+            last = top;
+    }
+    if (k > 64) {
         __syncthreads();
-        uint64_t b = kred[0];
-        for (int q = 1; q < 4; ++q)
-            b = kred[q] > b ? kred[q] : b;
-        __syncthreads();
-        if (b == 0)
-            break;
-        if (threadIdx.x == 0)
-            cand[(size_t)sc * kmax + r] = ~(uint32_t)(b & 0xFFFFFFFFull);
-        prev = b;
-        ++nsel;
+        uint64_t prev = last; // 0: fewer than 64 patches have power
+        for (uint32_t r = 64; r < k && prev; ++r) {
+            uint64_t best = 0;
+            for (uint32_t j = pb + threadIdx.x; j < pe; j += kPackSelThreads) {
+                const float *u = unshot + 3 * (size_t)j;
+                const uint64_t key = key_of(area[j] * (u[0] + u[1] + u[2]), j);
+                if (key < prev && key > best)
+                    best = key;
+            }
+            for (int o = 32; o > 0; o >>= 1) {
+                uint64_t v = __shfl_down(best, o, 64);
+                best = v > best ? v : best;
+            }
+            __syncthreads(); // wl is free (the merge, or the previous round)
+            if (lane == 0)
+                wl[0][w] = best;
+            __syncthreads();
+            uint64_t b = 0;
+            for (uint32_t q = 0; q < NW; ++q)
+                b = wl[0][q] > b ? wl[0][q] : b;
+            if (b && threadIdx.x == 0) {
+                cand[(size_t)sc * kmax + r] = ~(uint32_t)(b & 0xFFFFFFFFull);
+                ++nsel;
+            }
+            prev = b;
+        }
     }
     if (threadIdx.x == 0) {
         sc_res[sc] = res;
@@ -282,10 +328,13 @@ __global__ __launch_bounds__(256) void k_pack_shoot(
 void launch_pack_select(const PackBuffers &pk, const float *unshot, const float *area,
                         hipStream_t st)
 {
-    k_pack_select<<<pk.nscene, 256, 0, st>>>(pk.sc_pbeg, pk.sc_slots, pk.sc_den, unshot, area,
+    k_pack_select<<<pk.nscene, kPackSelThreads, 0, st>>>(pk.sc_pbeg, pk.sc_slots, pk.sc_den, unshot, area,
                                              pk.pass, pk.target, pk.kmax, pk.sc_done, pk.sc_res,
                                              pk.sc_nsel, pk.sc_shot, pk.cand);
-    k_pack_slots<<<1, 1024, 0, st>>>(pk.nscene, pk.sc_tbeg, pk.sc_pbeg, pk.sc_nsel, pk.sc_shot,
+    // one thread per scene: the kernel's sums and scans over the workgroup
+    // take barriers by its size (32 scenes: 11 us with 1,024 threads)
+    const uint32_t nt = pk.nscene >= 1024 ? 1024u : (pk.nscene + 63u) / 64u * 64u;
+    k_pack_slots<<<1, nt, 0, st>>>(pk.nscene, pk.sc_tbeg, pk.sc_pbeg, pk.sc_nsel, pk.sc_shot,
                                      pk.cand, pk.kmax, pk.K, pk.sc_slot_beg, pk.shooters,
                                      pk.slot_tbeg, pk.slot_tcnt, pk.slot_pbeg, pk.sc_w, pk.sc_dffo,
                                      pk.slot_w, pk.slot_dffo, pk.nshoot, pk.pass);

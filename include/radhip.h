@@ -57,7 +57,8 @@ typedef struct rad_config {
     uint32_t mode;            /* RAD_MODE_* */
     uint32_t select;          /* RAD_SELECT_* */
     uint32_t small_tri_px;    /* raster tuning: triangle pixels in a tile drawn by one lane (0: 64) */
-    uint32_t tile_px;         /* raster tuning: screen tile side 8, 16 or 32 (0: auto) */
+    uint32_t tile_px;         /* raster tuning: screen tile side 8, 16 or 32 of the binned
+                                 rasterizer (0: auto; small passes are then drawn without bins) */
     uint32_t graph_passes;    /* rad_step replays this many passes as one captured
                                  HIP graph (0: plain launches) */
 } rad_config;
@@ -228,7 +229,8 @@ int rad_face_mvps(rad_ctx *ctx, uint32_t patch, float *out80);
  * rad_step/rad_run, measured with HIP events on the context stream:
  * out[0] select, [1] prepare+clear, [2] raster setup, [3] binning (scan +
  * fill), [4] tile raster with the fused ProcessHemicube, [5] shoot; also the
- * number of timed passes. */
+ * number of timed passes.  A pass drawn without bins (small passes, tile_px 0)
+ * is [4] as a whole; its [2] and [3] are 0. */
 int rad_kernel_times(rad_ctx *ctx, int enable, double *out6, uint64_t *npasses);
 
 /* Device time (ms, HIP events) of the last standalone ProcessHemicube
@@ -267,7 +269,8 @@ int rad_debug_pool(rad_ctx *ctx, uint32_t cap, uint32_t *out4_or_null);
  * spread evenly over the patches (render + reduce, no shooting, state
  * unchanged; the device selection is overwritten) for each screen tile
  * side {16, 32} (and 8 for K <= 2) and in-lane triangle limit
- * {16, 32, 48, 64, 128, 256}, and keeps the fastest pair.  No counterpart in the
+ * {16, 32, 48, 64, 128, 256}, and keeps the fastest pair (a context that draws
+ * its passes without bins goes on so if that is faster than every pair).  No counterpart in the
  * reference (its GL driver rasterizes). */
 #define RAD_TUNE_MAX 18
 typedef struct rad_tune_result {

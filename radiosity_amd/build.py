@@ -33,6 +33,7 @@ HIPFLAGS = [f"--offload-arch={ARCH}", "-munsafe-fp-atomics",
 SOURCES = [
     # (source, compiled as HIP)
     ("rad_kernels.hip", True),
+    ("rad_direct.hip", True),
     ("rad_gather.hip", True),
     ("rad_pack.hip", True),
     ("rad_ingest.hip", True),

@@ -102,12 +102,24 @@ void record(rad_ctx *c, size_t idx)
         (void)hipEventRecord(c->ev[idx], c->st);
 }
 
+// Whether a pass of k slots takes the direct rasterizer (never when the
+// caller chose the binned one's tile side, itself or by rad_autotune), and
+// its tile side.
+static bool use_direct(const rad_ctx *c, uint32_t k, uint32_t *T)
+{
+    // nblk: the largest scene's triangles / 256, rounded up
+    const uint32_t ntri = c->pk.nscene ? c->bb.nblk * 256u : c->ntri;
+    return c->auto_tile && direct_wins(k, c->g.W, ntri, T);
+}
+
 // A pass of kSplitMin or more slots and kSplitBins or more bins renders as
 // two halves side by side, except a timed one (stage events bracket whole
 // stages).
 static bool split_render(const rad_ctx *c, uint32_t k)
 {
-    return k >= kSplitMin && k * c->bb.ntiles >= kSplitBins && !c->timing;
+    uint32_t T;
+    return k >= kSplitMin && k * c->bb.ntiles >= kSplitBins && !c->timing &&
+           !use_direct(c, k, &T);
 }
 
 // First slot of the second half of a split pass.
@@ -160,7 +172,42 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
     // With shoot_half, the first half's F rows are shot on the context
     // stream as soon as its tiles are done, while the second half still
     // renders; the caller shoots the second half.
-    if (split_render(c, k)) {
+    uint32_t T;
+    c->last_direct = use_direct(c, k, &T);
+    c->last_k = k;
+    if (c->last_direct) {
+        for (int j = 0; j < 2; ++j)
+            record(c, evbase + 3 + j);
+        DirectArgs d{};
+        d.W = c->g.W;
+        d.RES = c->g.RES;
+        d.nslot = k;
+        d.ntri = c->ntri;
+        d.rowlen = c->rowlen;
+        d.small_px = c->small_px;
+        d.fstride = c->K;
+        d.nshoot = c->nshoot;
+        d.tri = c->tri;
+        d.mvp = c->mvp;
+        d.dff = c->pk.slot_w ? c->pk.dffs : c->dff;
+        d.tsph = c->tsph;
+        d.clu = c->clu;
+        d.tri_patch = c->tri_patch;
+        d.slot_tbeg = c->pk.slot_tbeg;
+        d.slot_tcnt = c->pk.slot_tcnt;
+        d.slot_cbeg = c->pk.slot_cbeg;
+        d.slot_pbeg = c->pk.slot_pbeg;
+        d.slot_w = c->pk.slot_w;
+        d.slot_dffo = c->pk.slot_dffo;
+        d.out_ids = ids;
+        d.out_depth = depth;
+        d.ff = ids || fq ? nullptr : c->ff;
+        d.ffq = fq ? c->ffq : nullptr;
+        d.hits = hits;
+        d.counters = c->counters;
+        d.fblk = d.ff ? c->fblk : nullptr;
+        launch_direct(d, T, c->st);
+    } else if (split_render(c, k)) {
         HIPCHK(c, hipEventRecord(c->ev_fork, c->st));
         HIPCHK(c, hipStreamWaitEvent(c->st2, c->ev_fork, 0));
         for (int j = 0; j < 3; ++j) {
@@ -405,6 +452,7 @@ int rad_create(const rad_config *cfg, rad_ctx **out)
     if (hipGetDeviceProperties(&prop, c->device) == hipSuccess && prop.multiProcessorCount > 0)
         ncu = prop.multiProcessorCount;
     c->sel_blocks = ncu * 2;
+    c->auto_tile = cfg->tile_px == 0;
     // screen tiles: 32x32 when enough hemicubes fill the GPU, else 16x16
     // (32x32 also when a hemicube would have more tiles than the bins hold)
     uint32_t T = cfg->tile_px ? cfg->tile_px : (c->K >= 4 ? 32u : 16u);
@@ -432,7 +480,7 @@ void rad_destroy(rad_ctx *c)
     if (c->st2)
         (void)hipStreamSynchronize(c->st2);
     drop_graph(c);
-    void *ptrs[] = {c->tri,  c->tri_patch, c->tsph, c->frames, c->refl,     c->area,   c->emis,
+    void *ptrs[] = {c->tri,  c->tri_patch, c->tsph, c->clu, c->frames, c->refl,     c->area,   c->emis,
                     c->unshot, c->shot,   c->ff,  c->fblk,   c->hits,     c->dff,    c->item_ids,
                     c->item_depth, c->ffq, c->runs_slots, c->runs_offs, c->trip_h, c->trip_i,
                     c->trip_e,
@@ -443,7 +491,7 @@ void rad_destroy(rad_ctx *c)
                     c->pk.sc_slot_beg, c->pk.sc_nsel, c->pk.sc_done, c->pk.sc_den, c->pk.sc_res,
                     c->pk.sc_shot,
                     c->pk.cand, c->pk.patch_scene, c->pk.pass, c->pk.slot_tbeg, c->pk.slot_tcnt,
-                    c->pk.slot_pbeg, c->pk.sc_w, c->pk.sc_dffo, c->pk.slot_w, c->pk.slot_dffo,
+                    c->pk.slot_pbeg, c->pk.slot_cbeg, c->pk.sc_w, c->pk.sc_dffo, c->pk.slot_w, c->pk.slot_dffo,
                     c->pk.dffs, c->patch_quad, c->quad_pbeg, c->quad_nbr, c->qval,
                     c->viewfr, c->view_sh, c->pool};
     for (void *p : ptrs)
@@ -495,7 +543,7 @@ void pack_free(rad_ctx *c)
     PackBuffers &p = c->pk;
     void *ptrs[] = {p.sc_tbeg, p.sc_pbeg, p.sc_slots, p.sc_slot_beg, p.sc_nsel, p.sc_done, p.sc_den,
                     p.sc_res,  p.sc_shot, p.cand,    p.patch_scene, p.pass,     p.slot_tbeg,
-                    p.slot_tcnt, p.slot_pbeg, p.sc_w, p.sc_dffo, p.slot_w, p.slot_dffo, p.dffs};
+                    p.slot_tcnt, p.slot_pbeg, p.slot_cbeg, p.sc_w, p.sc_dffo, p.slot_w, p.slot_dffo, p.dffs};
     for (void *q : ptrs)
         dfree(q);
     c->pk = PackBuffers{};
@@ -538,6 +586,7 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     size_t K = c->K;
     if ((rc = dalloc(c, &c->tri, (size_t)ntri * 9)) || (rc = dalloc(c, &c->tri_patch, ntri)) ||
         (rc = dalloc(c, &c->tsph, ntri)) ||
+        (rc = dalloc(c, &c->clu, cluster_words(ntri, 0))) ||
         (rc = dalloc(c, &c->frames, (size_t)npatch * 9)) || (rc = dalloc(c, &c->refl, (size_t)npatch * 3)) ||
         (rc = dalloc(c, &c->area, npatch)) || (rc = dalloc(c, &c->emis, (size_t)npatch * 3)) ||
         (rc = dalloc(c, &c->unshot, (size_t)npatch * 3)) || (rc = dalloc(c, &c->shot, (size_t)npatch * 3)) ||
@@ -616,6 +665,7 @@ int upload_copy(rad_ctx *c, const float *tri_xyz, const uint32_t *tri_patch, uin
     HIPCHK(c, hipMemcpy(c->tri, planes.data(), planes.size() * sizeof(float), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->tri_patch, tri_patch, (size_t)ntri * 4, hipMemcpyHostToDevice));
     launch_tri_sphere(c->tri, ntri, c->tsph, c->st);
+    launch_clusters(c->tri, ntri, nullptr, 0, c->clu, c->st);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpy(c->frames, frames, (size_t)npatch * 36, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->refl, refl, (size_t)npatch * 12, hipMemcpyHostToDevice));
@@ -1022,6 +1072,9 @@ static int step_impl(rad_ctx *c, uint32_t passes)
         for (; passes >= G; passes -= G)
             HIPCHK(c, hipGraphLaunch(c->gexec, c->st));
         c->rendered = false;
+        uint32_t T;
+        c->last_direct = use_direct(c, c->K, &T);
+        c->last_k = c->K;
     }
     for (uint32_t p = 0; p < passes; ++p)
         if ((rc = one_pass(c, true, (size_t)p * 7)))
@@ -1312,6 +1365,8 @@ int rad_autotune(rad_ctx *c, uint32_t passes, rad_tune_result *out)
     }
     bool timing = c->timing;
     c->timing = false;
+    const bool was_auto = c->auto_tile;
+    c->auto_tile = false; // the candidates are the binned rasterizer's
     // K shooters spread evenly over the patch list: early in a solve the
     // selection holds only the few emitters, which is no sample of the work
     std::vector<uint32_t> spread(c->K);
@@ -1356,6 +1411,24 @@ int rad_autotune(rad_ctx *c, uint32_t passes, rad_tune_result *out)
             }
         }
     }
+    // a context that may draw directly goes on doing so where that is faster
+    // still than the best candidate
+    uint32_t Td;
+    c->auto_tile = was_auto;
+    if (rc == RAD_OK && use_direct(c, c->K, &Td)) {
+        rc = render_pass(c, c->K, 0, nullptr, nullptr, nullptr); // warm
+        (void)hipEventRecord(e0, c->st);
+        for (uint32_t p = 0; p < passes && rc == RAD_OK; ++p)
+            rc = render_pass(c, c->K, 0, nullptr, nullptr, nullptr);
+        (void)hipEventRecord(e1, c->st);
+        float ms = 0.f;
+        if (rc == RAD_OK && (hipEventSynchronize(e1) != hipSuccess ||
+                             hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
+            rc = fail(c, RAD_E_HIP, "autotune timing");
+        c->auto_tile = r.best_ms == 0.0 || ms / passes < r.best_ms;
+    } else {
+        c->auto_tile = false;
+    }
     c->timing = timing;
     c->rendered = false;
     (void)hipEventDestroy(e0);
@@ -1365,6 +1438,8 @@ int rad_autotune(rad_ctx *c, uint32_t passes, rad_tune_result *out)
     if (rc == RAD_OK && r.tile_px == 0)
         rc = fail(c, RAD_E_LIMIT, "autotune: every candidate overflowed the bins");
     int rc2 = set_tiles(c, rc == RAD_OK ? r.tile_px : T0, rc == RAD_OK ? r.small_tri_px : S0);
+    if (rc)
+        c->auto_tile = was_auto;
     if (rc)
         return rc;
     if (rc2)
@@ -1435,6 +1510,23 @@ int rad_debug_bins(rad_ctx *c, uint32_t *out, uint32_t *ntiles, uint32_t *tile_p
         *ntiles = c->bb.ntiles;
     if (tile_px)
         *tile_px = 1u << c->bb.tshift;
+    if (out && c->last_direct && c->npatch) {
+        // the last pass had no bins: count its records into them now (its
+        // MVPs and shooter count still stand), with counters of their own
+        uint32_t *cnt = nullptr;
+        int rc;
+        if ((rc = dalloc(c, &cnt, kCntN * kCntBlocks)))
+            return rc;
+        launch_clear(c->K, c->bb.count, c->bb.ntiles, nullptr, nullptr, 0, 0, cnt, c->bb.ent_cap,
+                     c->st);
+        launch_raster_setup(c->g, 0, c->last_k, 0, c->tri, c->tsph, c->tri_patch, c->ntri, c->mvp,
+                            c->nshoot, c->bb, cnt, c->pk.slot_tbeg, c->pk.slot_tcnt, c->pk.slot_w,
+                            c->st);
+        const hipError_t e = hipStreamSynchronize(c->st);
+        dfree(cnt);
+        HIPCHK(c, e);
+        c->last_direct = false;
+    }
     if (out)
         HIPCHK(c, hipMemcpy(out, c->bb.count, (size_t)c->K * c->bb.ntiles * 4, hipMemcpyDeviceToHost));
     return RAD_OK;
@@ -1977,7 +2069,9 @@ int rad_pack_upload(rad_ctx *c, uint32_t nscene, const uint32_t *scene_tri_beg,
         (rc = dalloc(c, &p.sc_shot, S)) ||
         (rc = dalloc(c, &p.cand, S * kmax)) || (rc = dalloc(c, &p.patch_scene, npatch)) ||
         (rc = dalloc(c, &p.pass, 1)) || (rc = dalloc(c, &p.slot_tbeg, c->K)) ||
-        (rc = dalloc(c, &p.slot_tcnt, c->K)) || (rc = dalloc(c, &p.slot_pbeg, c->K))) {
+        (rc = dalloc(c, &p.slot_tcnt, c->K)) || (rc = dalloc(c, &p.slot_pbeg, c->K)) ||
+        (rc = dalloc(c, &p.slot_cbeg, c->K)) ||
+        (rc = dalloc(c, &c->clu, cluster_words(ntri, nscene)))) {
         // the F rows are sized for the largest scene, not for a plain scene
         pack_free(c);
         return drop_scene(c, rc);
@@ -2005,6 +2099,10 @@ int rad_pack_upload(rad_ctx *c, uint32_t nscene, const uint32_t *scene_tri_beg,
     set(p.slot_tbeg, 0, c->K * 4);
     set(p.slot_tcnt, 0, c->K * 4);
     set(p.slot_pbeg, 0, c->K * 4);
+    set(p.slot_cbeg, 0, c->K * 4);
+    launch_clusters(c->tri, ntri, p.sc_tbeg, nscene, c->clu, c->st);
+    if (e == hipSuccess)
+        e = hipGetLastError();
     if (e != hipSuccess) {
         pack_free(c);
         return drop_scene(c, fail(c, RAD_E_HIP, std::string("pack upload: ") +
@@ -2308,6 +2406,7 @@ int rad_scene_ingest(rad_ctx *c, const float *quads, uint32_t nface, const float
                       c->tri_patch, c->frames, c->refl, c->area, c->emis, c->unshot, c->shot,
                       c->patch_quad, c->quad_pbeg, c->quad_nbr, c->st);
         launch_tri_sphere(c->tri, nt, c->tsph, c->st);
+        launch_clusters(c->tri, nt, nullptr, 0, c->clu, c->st);
         e = hipGetLastError();
     }
     if (e == hipSuccess)

@@ -32,6 +32,7 @@ struct rad_ctx {
     float *tri = nullptr;          // 9 planes of ntri
     uint32_t *tri_patch = nullptr; // ntri
     float4 *tsph = nullptr;        // ntri bounding spheres (centre, radius)
+    float4 *clu = nullptr;         // bounds of the runs of 64 and 16 triangles
     float *frames = nullptr;       // npatch*9
     float *refl = nullptr;         // npatch*3
     float *area = nullptr;         // npatch
@@ -78,6 +79,9 @@ struct rad_ctx {
     uint32_t pool_cap = rad::kPoolCap;
     uint32_t small_px = 16;        // in-lane rasterization limit (pixels of a tile)
     int sel_blocks = 1024;
+    bool auto_tile = true;         // no tile side chosen: small passes are drawn directly
+    bool last_direct = false;      // the last pass was, over last_k slots
+    uint32_t last_k = 0;
     bool rendered = false;        // item_ids hold the item buffer of the last render
     uint32_t rendered_k = 0;
 

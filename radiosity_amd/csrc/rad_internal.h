@@ -128,6 +128,7 @@ struct PackBuffers {
     uint32_t *patch_scene = nullptr;                 // npatch
     uint32_t *pass = nullptr;                        // passes selected so far
     uint32_t *slot_tbeg = nullptr, *slot_tcnt = nullptr, *slot_pbeg = nullptr; // K
+    uint32_t *slot_cbeg = nullptr;                   // first cluster of the slot's scene
     // scenes at their own hemicube resolution (rad_pack_hemicubes; null: all
     // at the context's): per scene W and offset of its ΔFF table in dffs,
     // the same per slot of the pass
@@ -251,6 +252,30 @@ uint32_t shoot_lists(uint32_t npatch, bool pooled = false);
 void launch_residual(const float *unshot, const float *area, const float *emis,
                      uint32_t npatch, double *partials, uint32_t *counter, double *resid,
                      int nblocks, hipStream_t st);
+
+// Launchers implemented in rad_direct.hip: the clusters of a scene (or of
+// the nscene scenes of a pack), and a pass's whole rasterization (shooter
+// slots [0, nslot), of which those below *nshoot are drawn) in one launch
+// from the prepared MVPs: out_ids != null writes the item buffer, else the
+// tiles are reduced into ff (with its F-block flags fblk, nullable) or, when
+// it is given, the fixed-point rows ffq, and into hits (nullable).
+struct DirectArgs {
+    uint32_t W, RES, nslot, ntri, rowlen, small_px, tshift, fstride;
+    const uint32_t *nshoot;
+    const float *tri, *mvp, *dff;
+    const float4 *tsph, *clu;
+    const uint32_t *tri_patch;
+    const uint32_t *slot_tbeg, *slot_tcnt, *slot_cbeg, *slot_pbeg, *slot_w, *slot_dffo;
+    uint32_t *out_ids;
+    float *out_depth, *ff;
+    unsigned long long *ffq;
+    uint32_t *hits, *counters, *fblk;
+};
+size_t cluster_words(uint32_t ntri, uint32_t nscene);
+void launch_clusters(const float *tri, uint32_t ntri, const uint32_t *sc_tbeg, uint32_t nscene,
+                     float4 *clu, hipStream_t st);
+bool direct_wins(uint32_t k, uint32_t W, uint32_t ntri, uint32_t *T);
+void launch_direct(const DirectArgs &args, uint32_t T, hipStream_t st);
 
 // Launchers implemented in rad_pack.hip.
 void launch_pack_select(const PackBuffers &pk, const float *unshot, const float *area,

@@ -181,7 +181,8 @@ __global__ __launch_bounds__(1024) void k_pack_slots(
     const uint32_t *__restrict__ cand, uint32_t kmax, uint32_t K,
     uint32_t *__restrict__ sc_slot_beg, uint32_t *__restrict__ shooters,
     uint32_t *__restrict__ slot_tbeg, uint32_t *__restrict__ slot_tcnt,
-    uint32_t *__restrict__ slot_pbeg, const uint32_t *__restrict__ sc_w,
+    uint32_t *__restrict__ slot_pbeg, uint32_t *__restrict__ slot_cbeg,
+    const uint32_t *__restrict__ sc_w,
     const uint32_t *__restrict__ sc_dffo, uint32_t *__restrict__ slot_w,
     uint32_t *__restrict__ slot_dffo, uint32_t *__restrict__ nshoot, uint32_t *__restrict__ pass)
 {
@@ -254,6 +255,7 @@ __global__ __launch_bounds__(1024) void k_pack_slots(
                 slot_tbeg[slot] = sc_tbeg[s];
                 slot_tcnt[slot] = sc_tbeg[s + 1] - sc_tbeg[s];
                 slot_pbeg[slot] = sc_pbeg[s];
+                slot_cbeg[slot] = sc_tbeg[s] / 64u + s;
                 if (sc_w) {
                     slot_w[slot] = sc_w[s];
                     slot_dffo[slot] = sc_dffo[s];
@@ -336,7 +338,8 @@ void launch_pack_select(const PackBuffers &pk, const float *unshot, const float 
     const uint32_t nt = pk.nscene >= 1024 ? 1024u : (pk.nscene + 63u) / 64u * 64u;
     k_pack_slots<<<1, nt, 0, st>>>(pk.nscene, pk.sc_tbeg, pk.sc_pbeg, pk.sc_nsel, pk.sc_shot,
                                      pk.cand, pk.kmax, pk.K, pk.sc_slot_beg, pk.shooters,
-                                     pk.slot_tbeg, pk.slot_tcnt, pk.slot_pbeg, pk.sc_w, pk.sc_dffo,
+                                     pk.slot_tbeg, pk.slot_tcnt, pk.slot_pbeg, pk.slot_cbeg,
+                                     pk.sc_w, pk.sc_dffo,
                                      pk.slot_w, pk.slot_dffo, pk.nshoot, pk.pass);
 }
 

@@ -217,7 +217,7 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
         if (shoot_half)
             launch_shoot(c->cfg.mode, c->K, c->shooters, c->nshoot, c->snap, c->ff, c->fblk,
                          c->refl, c->area, c->npatch, c->unshot, c->shot, c->ctl, 0, split_at(k),
-                         false, nullptr, nullptr, c->st);
+                         false, nullptr, nullptr, 0, c->st);
         HIPCHK(c, hipEventRecord(c->ev_join, c->st2));
         HIPCHK(c, hipStreamWaitEvent(c->st, c->ev_join, 0));
     } else {
@@ -269,19 +269,23 @@ int select_dev(rad_ctx *c, uint32_t k)
         return check_launch(c, "select");
     }
     if (c->cfg.select == RAD_SELECT_REFERENCE)
-        launch_select_reference(c->unshot, c->npatch, k, c->shooters, c->nshoot, c->st);
+        launch_select_reference(c->unshot, c->npatch, k, c->shooters, c->nshoot, nullptr, c->ctl,
+                                c->st);
     else
         launch_select_topk(c->cfg.select, c->unshot, c->area, c->emis, c->npatch, k, c->shooters,
                            c->nshoot, c->cand, nullptr, nullptr, c->resid, c->st);
     return check_launch(c, "select");
 }
 
-// Whether a pass's last shoot can leave the next POWER selection's
-// per-workgroup lists (top-K of 2 .. 64, one merge level for the lists).
+// Whether a pass's last shoot can leave the next selection's keys: each
+// workgroup's largest for one shooter, its list of 64 for POWER passes of
+// 2 .. 64 (one merge level for the lists).
 static bool fused_select(const rad_ctx *c)
 {
-    return !c->pk.nscene && c->cfg.select == RAD_SELECT_POWER && c->K > 1 && c->K <= 64 &&
-           shoot_lists(c->npatch) <= 256;
+    if (c->pk.nscene)
+        return false;
+    return c->K == 1 || (c->cfg.select == RAD_SELECT_POWER && c->K <= 64 &&
+                         shoot_lists(c->npatch) <= 256);
 }
 
 // One pass: select, render, shoot.  chain_in: the previous pass already
@@ -297,13 +301,24 @@ int one_pass(rad_ctx *c, bool do_select, size_t evbase, bool chain_in = false,
              bool chain_out = false, uint32_t target = 0, bool relist = false)
 {
     int rc;
+    const NextPass np{c->K,    c->shooters, c->nshoot,   c->frames,
+                      c->snap, c->mvp,      c->bb.count, (size_t)c->K * c->bb.ntiles,
+                      c->counters, c->bb.ent_cap};
+    bool prepared = chain_in;
     record(c, evbase + 0);
     if (c->pk.nscene) {
         launch_pack_select(c->pk, c->unshot, c->area, c->st);
         if ((rc = check_launch(c, "pack select")))
             return rc;
-    } else if (do_select && !chain_in && (rc = select_dev(c, c->K)) != RAD_OK) {
-        return rc;
+    } else if (do_select && !chain_in) {
+        // the list selection, one workgroup, prepares its pass itself when
+        // no F rows need clearing
+        prepared = c->K > 1 && c->cfg.select == RAD_SELECT_REFERENCE && !c->ff_dirty && !c->timing;
+        if (prepared)
+            launch_select_reference(c->unshot, c->npatch, c->K, c->shooters, c->nshoot, &np,
+                                    c->ctl, c->st);
+        else if ((rc = select_dev(c, c->K)) != RAD_OK)
+            return rc;
     }
     record(c, evbase + 1);
     // the first half of a split pass is shot before the second finishes
@@ -311,7 +326,7 @@ int one_pass(rad_ctx *c, bool do_select, size_t evbase, bool chain_in = false,
     // comes after both halves)
     const bool half = !c->pk.nscene && !c->det && split_render(c, c->K);
     if ((rc = render_pass(c, c->K, evbase, nullptr, nullptr, nullptr, nullptr, nullptr, half,
-                          chain_in)) != RAD_OK)
+                          prepared)) != RAD_OK)
         return rc;
     if (c->pk.nscene)
         launch_pack_shoot(c->pk, c->cfg.mode, c->snap, c->ff, c->rowlen, c->refl, c->area,
@@ -321,14 +336,16 @@ int one_pass(rad_ctx *c, bool do_select, size_t evbase, bool chain_in = false,
                      c->det ? nullptr : c->fblk, c->refl, c->area, c->npatch, c->unshot,
                      c->shot, c->ctl, half ? split_at(c->K) : 0u, c->K, true,
                      chain_out ? c->cand : nullptr,
-                     chain_out && chain_in && !relist ? c->pool : nullptr, c->st);
+                     chain_out && chain_in && !relist && c->K > 1 ? c->pool : nullptr,
+                     chain_out && c->K == 1 ? 1u + c->cfg.select : 0u, c->st);
     if (chain_out) {
-        const NextPass np{c->K,    c->shooters, c->nshoot,   c->frames,
-                          c->snap, c->mvp,      c->bb.count, (size_t)c->K * c->bb.ntiles,
-                          c->counters, c->bb.ent_cap};
-        launch_next_pass(c->cand, shoot_lists(c->npatch, chain_in && !relist), np, c->unshot,
-                         c->area, c->npatch,
-                         c->ctl, c->pool, !chain_in || relist, target, c->pool_cap, c->st);
+        if (c->K == 1)
+            launch_next_top1(c->cfg.select, c->cand, shoot_lists(c->npatch, true), np, c->unshot,
+                             c->ctl, c->st);
+        else
+            launch_next_pass(c->cand, shoot_lists(c->npatch, chain_in && !relist), np, c->unshot,
+                             c->area, c->npatch, c->ctl, c->pool, !chain_in || relist, target,
+                             c->pool_cap, c->st);
     }
     c->ff_dirty = 0; // the shoot kernels zero the entries they read
     record(c, evbase + 6);
@@ -994,6 +1011,27 @@ static int ensure_events(rad_ctx *c, size_t n)
     return RAD_OK;
 }
 
+// n passes in a row.  Nothing else touches the state between them, so every
+// pass but the last selects and prepares its successor.  Every kPoolRearm
+// passes (from the first) a pass's shoot leaves lists and the next selection
+// arms the pool from them.  Armed after pass p's shoot, the pool serves the
+// selections of passes p + 2 .. q (q: the pass before the next such shoot's
+// successor, at most n - 1); each pass shoots K keys at or above the bound
+// while the others only grow (all additions are of non-negative terms), so
+// (q - p) K keys at or above it keep every pool at K or more.  Whatever the
+// bound, a pool is used only when it holds K keys.
+static int chained_passes(rad_ctx *c, uint32_t n)
+{
+    const bool fuse = fused_select(c);
+    int rc = RAD_OK;
+    for (uint32_t p = 0; p < n && rc == RAD_OK; ++p) {
+        const uint32_t q = std::min(kPoolRearm * (p / kPoolRearm + 1), n - 1);
+        rc = one_pass(c, true, 0, fuse && p > 0, fuse && p + 1 < n,
+                      fuse && q >= p + 2 ? (q - p) * c->K : 0u, p % kPoolRearm == 0);
+    }
+    return rc;
+}
+
 // Captures graph_passes passes (kernels only: every clear in a pass is a
 // kernel, no memset or copy node) into one executable graph.
 static int capture_graph(rad_ctx *c, uint32_t n)
@@ -1001,23 +1039,7 @@ static int capture_graph(rad_ctx *c, uint32_t n)
     drop_graph(c);
     hipGraph_t graph = nullptr;
     HIPCHK(c, hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
-    int rc = RAD_OK;
-    // inside a replay nothing else touches the state between passes, so
-    // every pass but the last selects and prepares its successor.  Every
-    // kPoolRearm passes (from the first) a pass's shoot leaves lists and the
-    // next selection arms the pool from them.  Armed after pass p's shoot,
-    // the pool serves the selections of passes p + 2 .. q (q: the pass
-    // before the next such shoot's successor, at most n - 1); each pass
-    // shoots K keys at or above the bound while the others only grow (all
-    // additions are of non-negative terms), so (q - p) K keys at or above
-    // it keep every pool at K or more.  Whatever the bound, a pool is used
-    // only when it holds K keys.
-    const bool fuse = fused_select(c);
-    for (uint32_t p = 0; p < n && rc == RAD_OK; ++p) {
-        const uint32_t q = std::min(kPoolRearm * (p / kPoolRearm + 1), n - 1);
-        rc = one_pass(c, true, 0, fuse && p > 0, fuse && p + 1 < n,
-                      fuse && q >= p + 2 ? (q - p) * c->K : 0u, p % kPoolRearm == 0);
-    }
+    const int rc = chained_passes(c, n);
     hipError_t e = hipStreamEndCapture(c->st, &graph);
     if (rc)
         return rc;
@@ -1076,10 +1098,12 @@ static int step_impl(rad_ctx *c, uint32_t passes)
         c->last_direct = use_direct(c, c->K, &T);
         c->last_k = c->K;
     }
+    if (!c->timing) // timed passes stay whole: their stages are bracketed
+        return chained_passes(c, passes);
     for (uint32_t p = 0; p < passes; ++p)
         if ((rc = one_pass(c, true, (size_t)p * 7)))
             return rc;
-    return c->timing ? add_stage_times(c, passes) : RAD_OK;
+    return add_stage_times(c, passes);
 }
 
 int rad_step(rad_ctx *c, uint32_t passes)

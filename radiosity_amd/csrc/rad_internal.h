@@ -148,8 +148,6 @@ void launch_select_topk(uint32_t rule, const float *unshot, const float *area,
                         uint32_t *nshoot, uint64_t *cand, double *partials,
                         uint32_t *counter, double *resid, hipStream_t st);
 size_t topk_cand_half(uint32_t npatch, uint32_t k);
-void launch_select_reference(const float *unshot, uint32_t npatch, uint32_t k,
-                             uint32_t *shooters, uint32_t *nshoot, hipStream_t st);
 void launch_prepare(const Geometry &g, uint32_t K, const uint32_t *shooters,
                     const uint32_t *nshoot, const float *frames, const float *unshot,
                     float *snap, float *mvp, hipStream_t st);
@@ -210,6 +208,11 @@ struct NextPass {
     uint32_t *counters;
     uint32_t ent_cap;
 };
+// With np (its frames, snapshots, MVPs, bins and counters) the selection
+// also prepares the pass.
+void launch_select_reference(const float *unshot, uint32_t npatch, uint32_t k, uint32_t *shooters,
+                             uint32_t *nshoot, const NextPass *np, const uint32_t *ctl,
+                             hipStream_t st);
 // Candidate pool of a chained POWER selection (device memory).  When armed,
 // a pass's last shoot keeps every receiver whose key is at least tau:
 // count keys, the first kPoolCap of them in keys (one global atomic per
@@ -236,7 +239,12 @@ void launch_shoot(uint32_t mode, uint32_t K, const uint32_t *shooters,
                   const uint32_t *nshoot, const float *snap, float *ff, uint32_t *fblk,
                   const float *refl, const float *area, uint32_t npatch, float *unshot,
                   float *shot, uint32_t *ctl, uint32_t sbeg, uint32_t send, bool last,
-                  uint64_t *lists, SelPool *pool, hipStream_t st);
+                  uint64_t *lists, SelPool *pool, uint32_t top1, hipStream_t st);
+// With top1 = 1 + rule (passes of one shooter) the last shoot leaves each
+// workgroup's largest key in lists instead (as many as shoot_lists(npatch,
+// true)), and launch_next_top1 selects and prepares the next pass from them.
+void launch_next_top1(uint32_t rule, const uint64_t *keys, uint32_t nkeys, const NextPass &np,
+                      const float *unshot, const uint32_t *ctl, hipStream_t st);
 // The selection and preparation of a pass after one whose last shoot left
 // lists or pooled (pool->armed, unless lists_only).  From lists, with
 // target != 0, it arms the pool for the shoots that follow: tau is set so

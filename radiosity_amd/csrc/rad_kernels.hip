@@ -1939,6 +1939,16 @@ __device__ static void write_shooters(uint64_t top, uint32_t k, uint32_t *__rest
         *nshoot = (uint32_t)__popcll(m);
 }
 
+__device__ static inline uint64_t wave_max_u64(uint64_t v)
+{
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        uint64_t o = __shfl_xor(v, d);
+        v = o > v ? o : v;
+    }
+    return v;
+}
+
 // Main.cpp:1251-1295 for all receivers at once: one thread per receiver j
 // accumulates the contributions of the pass's shooters, then the shooters
 // move their snapshot from unshot to shot.  Every nonzero F entry it reads
@@ -1949,7 +1959,8 @@ __device__ static void write_shooters(uint64_t top, uint32_t k, uint32_t *__rest
 // per-workgroup lists k_topk64_scan would make from the stored state, so
 // the next pass's selection only merges them; or, with the pool armed, it
 // adds every receiver whose key is at least the pool's tau to the pool
-// instead.  NT threads per workgroup: 1,024 with lists (one merge
+// instead; with top1 != 0 (one shooter per pass) each workgroup leaves its
+// largest key of rule top1 - 1 in lists[blockIdx.x].  NT threads per workgroup: 1,024 with lists (one merge
 // level for up to 262,144 receivers); 256 without lists, and with lists
 // when the pool is expected (then lists, left only when the pool is not
 // armed, cover 256 receivers each).
@@ -1967,7 +1978,7 @@ __global__ __launch_bounds__(NT) void k_shoot(uint32_t mode, const uint32_t *__r
                                                float *__restrict__ shot, uint32_t *__restrict__ ctl,
                                                uint32_t sbeg, uint32_t send, uint32_t last,
                                                uint64_t *__restrict__ lists,
-                                               SelPool *__restrict__ pool)
+                                               SelPool *__restrict__ pool, uint32_t top1)
 {
     __shared__ uint32_t sid[RAD_MAX_K];
     __shared__ float sc[RAD_MAX_K * 4];
@@ -2094,13 +2105,27 @@ __global__ __launch_bounds__(NT) void k_shoot(uint32_t mode, const uint32_t *__r
     }
     if (!lists)
         return;
-    // sel_key(RAD_SELECT_POWER) of the state just stored
+    // sel_key of the state just stored
     uint64_t key = 0ull;
-    if (live) {
+    if (live && top1 == 1u + RAD_SELECT_REFERENCE) {
+        key = ((uint64_t)__float_as_uint(u0 * u0 + u1 * u1 + u2 * u2) << 32) | j;
+    } else if (live) {
         float e = area[j] * (u0 + u1 + u2);
         if (!(e > 0.0f))
             e = 0.0f;
         key = ((uint64_t)__float_as_uint(e) << 32) | (0xFFFFFFFFu - j);
+    }
+    if (top1) {
+        key = wave_max_u64(key);
+        if (lane == 0)
+            wl[0][w] = key;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (uint32_t q = 1; q < NT / 64; ++q)
+                key = wl[0][q] > key ? wl[0][q] : key;
+            lists[blockIdx.x] = key;
+        }
+        return;
     }
     if (pooled) {
         // every receiver whose key is at least tau (a positive power) goes
@@ -2149,17 +2174,17 @@ void launch_shoot(uint32_t mode, uint32_t K, const uint32_t *shooters, const uin
                   const float *snap, float *ff, uint32_t *fblk, const float *refl,
                   const float *area, uint32_t npatch, float *unshot, float *shot, uint32_t *ctl,
                   uint32_t sbeg, uint32_t send, bool last, uint64_t *lists, SelPool *pool,
-                  hipStream_t st)
+                  uint32_t top1, hipStream_t st)
 {
-    if (lists && !pool)
+    if (lists && !pool && !top1)
         k_shoot<kShootListThreads><<<shoot_lists(npatch, false), kShootListThreads, 0, st>>>(
             mode, shooters, nshoot, snap, ff, fblk, K, refl, area, npatch, unshot, shot, ctl,
-            sbeg, send, last ? 1u : 0u, lists, nullptr);
+            sbeg, send, last ? 1u : 0u, lists, nullptr, 0u);
     else
         k_shoot<256><<<(npatch + 255) / 256, 256, 0, st>>>(mode, shooters, nshoot, snap, ff, fblk,
                                                           K, refl, area, npatch, unshot, shot,
                                                           ctl, sbeg, send, last ? 1u : 0u, lists,
-                                                          pool);
+                                                          pool, top1);
 }
 
 __device__ static inline uint64_t sel_key(uint32_t rule, const float *unshot, const float *area,
@@ -2404,21 +2429,50 @@ __device__ static inline uint32_t sel_decode(uint32_t rule, uint64_t key)
     return 0xFFFFFFFFu - (uint32_t)key;
 }
 
+// The start of the pass after one whose shoot left each workgroup's largest
+// key: the single shooter and what k_prepare_clear does, as k_next_pass.
+__global__ __launch_bounds__(1024) void k_next_top1(uint32_t rule, const uint64_t *__restrict__ keys,
+                                                    uint32_t nkeys, NextPass np,
+                                                    const float *__restrict__ unshot,
+                                                    const uint32_t *__restrict__ ctl)
+{
+    __shared__ uint64_t wl[16];
+    __shared__ uint32_t ssel, sn;
+    const uint32_t t = threadIdx.x;
+    const uint32_t stop = ctl[kCtlStop];
+    uint64_t best = 0;
+    for (uint32_t i = t; i < nkeys; i += blockDim.x)
+        best = keys[i] > best ? keys[i] : best;
+    best = wave_max_u64(best);
+    if ((t & 63u) == 0)
+        wl[t >> 6] = best;
+    __syncthreads();
+    if (t == 0) {
+        for (uint32_t q = 1; q < 16; ++q)
+            best = wl[q] > best ? wl[q] : best;
+        ssel = sel_decode(rule, best);
+        sn = stop ? 0u : 1u;
+        np.shooters[0] = ssel;
+        *np.nshoot = sn;
+    }
+    __syncthreads();
+    if (t < 5)
+        prepare_item(t, 1u, &ssel, &sn, np.frames, unshot, np.snap, np.mvp, nullptr);
+    clear_range(t, blockDim.x, np.bin_count, np.nbins, nullptr, nullptr, 0, np.counters,
+                np.ent_cap);
+}
+
+void launch_next_top1(uint32_t rule, const uint64_t *keys, uint32_t nkeys, const NextPass &np,
+                      const float *unshot, const uint32_t *ctl, hipStream_t st)
+{
+    k_next_top1<<<1, 1024, 0, st>>>(rule, keys, nkeys, np, unshot, ctl);
+}
+
 template <typename T> __device__ static inline T wave_sum(T v)
 {
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1)
         v += __shfl_xor(v, d);
-    return v;
-}
-
-__device__ static inline uint64_t wave_max_u64(uint64_t v)
-{
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-        uint64_t o = __shfl_xor(v, d);
-        v = o > v ? o : v;
-    }
     return v;
 }
 
@@ -2795,10 +2849,12 @@ __device__ static inline void reference_insert(float (&key)[R], uint32_t (&id)[R
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// np.K != 0: the workgroup also does k_prepare_clear's work for the pass (no
+// F rows or hits to clear), one dependent launch less.
 template <int R>
 __global__ __launch_bounds__(kRefThreads) void k_select_reference(
     const float *__restrict__ unshot, uint32_t npatch, uint32_t k, uint32_t *__restrict__ shooters,
-    uint32_t *__restrict__ nshoot)
+    uint32_t *__restrict__ nshoot, NextPass np, const uint32_t *__restrict__ ctl)
 {
     __shared__ float lk[64 * R], ck[kRefThreads];
     __shared__ uint32_t li[64 * R], ci[kRefThreads];
@@ -2881,18 +2937,32 @@ __global__ __launch_bounds__(kRefThreads) void k_select_reference(
     }
     for (uint32_t i = threadIdx.x; i < k; i += kRefThreads)
         shooters[i] = i < sn ? li[i] : 0u;
+    if (np.K) {
+        __syncthreads(); // every thread has read sn
+        if (threadIdx.x == 0 && ctl[kCtlStop])
+            sn = 0u; // the stop gate of k_prepare_clear
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < np.K * 5; i += kRefThreads)
+            prepare_item(i, np.K, li, &sn, np.frames, unshot, np.snap, np.mvp, nullptr);
+        clear_range(threadIdx.x, kRefThreads, np.bin_count, np.nbins, nullptr, nullptr, 0,
+                    np.counters, np.ent_cap);
+    }
     if (threadIdx.x == 0)
         *nshoot = sn;
 }
 
 void launch_select_reference(const float *unshot, uint32_t npatch, uint32_t k, uint32_t *shooters,
-                             uint32_t *nshoot, hipStream_t st)
+                             uint32_t *nshoot, const NextPass *np, const uint32_t *ctl,
+                             hipStream_t st)
 {
     static_assert(RAD_MAX_K <= 256, "four list entries per lane");
+    const NextPass p = np ? *np : NextPass{};
     if (k <= 64)
-        k_select_reference<1><<<1, kRefThreads, 0, st>>>(unshot, npatch, k, shooters, nshoot);
+        k_select_reference<1><<<1, kRefThreads, 0, st>>>(unshot, npatch, k, shooters, nshoot, p,
+                                                         ctl);
     else
-        k_select_reference<4><<<1, kRefThreads, 0, st>>>(unshot, npatch, k, shooters, nshoot);
+        k_select_reference<4><<<1, kRefThreads, 0, st>>>(unshot, npatch, k, shooters, nshoot, p,
+                                                         ctl);
 }
 
 } // namespace rad

@@ -80,3 +80,33 @@ def test_pack_selection_equals_plain(rad, slots):
     q.set_state(u, z, u)
     q.step(2)
     assert res[0] == pytest.approx(q.residual(), rel=1e-12)
+
+
+@pytest.mark.parametrize("K,graph,select", [(1, 0, 0), (1, 0, 1), (1, 5, 0), (1, 5, 1), (3, 0, 0),
+                                            (7, 4, 0), (24, 0, 1), (64, 0, 1), (70, 0, 1)])
+def test_passes_in_a_row_equal_single_passes(rad, K, graph, select):
+    """A call of several passes selects and prepares each from what the one
+    before left; single-pass calls select from the stored state.  With
+    fixed-point form factors the states agree bit for bit, stopped cycles
+    (whose later passes shoot nobody) included."""
+    sc = rad.Scene.boxes(nboxes=12, room=(7.0, 3.0, 7.0), target_tris=3000, nlights=6, seed=4)
+    say(f"passes in a row K={K} graph={graph} select={select}")
+    out = []
+    for one in (False, True):
+        s = rad.Solver(hemicube=32, hemicubes=K, graph_passes=0 if one else graph, select=select)
+        s.set_deterministic(True)
+        s.upload(sc)
+        for _ in range(2):
+            if one:
+                for _ in range(11):
+                    s.step(1)
+            else:
+                s.step(11)
+        s.finish()
+        out.append(s.state() + (s.shot_count(),))
+        st = s.run_cycle(4, 1e9) if not one else None
+        if st:
+            assert st.passes == 1 and st.stopped == 1
+    for a, b in zip(out[0][:2], out[1][:2]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    assert out[0][2] == out[1][2]

@@ -88,6 +88,18 @@ void dfree(void *p)
         (void)hipFree(p);
 }
 
+void gather_free(rad_ctx *c)
+{
+    GatherWs &w = c->gw;
+    void *ptrs[] = {w.yp, w.E, w.B, w.rv, w.out, w.xhi, w.xlo, w.parts};
+    for (void *q : ptrs)
+        dfree(q);
+    for (hipEvent_t e : w.ev)
+        if (e)
+            (void)hipEventDestroy(e);
+    c->gw = GatherWs{};
+}
+
 int check_launch(rad_ctx *c, const char *what)
 {
     hipError_t e = hipGetLastError();
@@ -497,6 +509,7 @@ void rad_destroy(rad_ctx *c)
     if (c->st2)
         (void)hipStreamSynchronize(c->st2);
     drop_graph(c);
+    gather_free(c);
     void *ptrs[] = {c->tri,  c->tri_patch, c->tsph, c->clu, c->frames, c->refl,     c->area,   c->emis,
                     c->unshot, c->shot,   c->ff,  c->fblk,   c->hits,     c->dff,    c->item_ids,
                     c->item_depth, c->ffq, c->runs_slots, c->runs_offs, c->trip_h, c->trip_i,
@@ -596,6 +609,7 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     (void)hipStreamSynchronize(c->st);
     drop_graph(c);
     pack_free(c);
+    gather_free(c);
     c->nquad = 0;
     c->ntri = c->npatch = 0;
     c->hash_valid = false;
@@ -1609,20 +1623,29 @@ int need_dense(rad_ctx *c)
     return RAD_OK;
 }
 
-// Work buffers of one gather call (R columns, rp = 16 * tiles).
+// One gather call (R columns, rp = 16 * tiles): its work buffers, which
+// belong to the context.
 struct GatherBufs {
-    uint32_t rt = 1, rp = 16, S = 1, nblk = 1024;
+    uint32_t rt = 1, rp = 16, S = 1, nblk = 1;
     GemmSplit ks1{}, ks2{}; // k slices of the single-half and two-half products
     float *yp = nullptr, *E = nullptr, *B = nullptr, *rv = nullptr, *out = nullptr;
     uint16_t *xhi = nullptr, *xlo = nullptr;
     double *parts = nullptr;
-    ~GatherBufs()
-    {
-        void *p[] = {yp, E, B, rv, out, xhi, xlo, parts};
-        for (void *q : p)
-            dfree(q);
-    }
 };
+
+// A work buffer of at least n elements (contents undefined).
+template <typename T> int ws_get(rad_ctx *c, T **p, size_t *cap, size_t n, T **out)
+{
+    if (n > *cap) {
+        *cap = 0;
+        int rc;
+        if ((rc = dalloc(c, p, n)))
+            return rc;
+        *cap = n;
+    }
+    *out = *p;
+    return RAD_OK;
+}
 
 int gather_alloc(rad_ctx *c, GatherBufs &g, uint32_t R)
 {
@@ -1633,17 +1656,21 @@ int gather_alloc(rad_ctx *c, GatherBufs &g, uint32_t R)
     HIPCHK(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device));
     g.ks1 = gemm_split(g.rt, false, c->npad, g.S, ncu > 0 ? (uint32_t)ncu : 1u);
     g.ks2 = gemm_split(g.rt, true, c->npad, g.S, ncu > 0 ? (uint32_t)ncu : 1u);
+    g.nblk = gather_blocks(R, c->npad);
     const uint32_t planes = std::max(g.S, std::max(g.ks1.S2, g.ks2.S2));
     size_t plane = (size_t)g.rp * c->npad;
+    GatherWs &w = c->gw;
     int rc;
-    if ((rc = dalloc(c, &g.yp, plane * planes)) || (rc = dalloc(c, &g.E, plane)) ||
-        (rc = dalloc(c, &g.B, plane)) || (rc = dalloc(c, &g.rv, plane)) ||
-        (rc = dalloc(c, &g.out, (size_t)R * c->npatch)) || (rc = dalloc(c, &g.xhi, plane)) ||
-        (rc = dalloc(c, &g.xlo, plane)) || (rc = dalloc(c, &g.parts, g.nblk)))
+    if ((rc = ws_get(c, &w.yp, &w.nyp, plane * planes, &g.yp)) ||
+        (rc = ws_get(c, &w.E, &w.nE, plane, &g.E)) || (rc = ws_get(c, &w.B, &w.nB, plane, &g.B)) ||
+        (rc = ws_get(c, &w.rv, &w.nrv, plane, &g.rv)) ||
+        (rc = ws_get(c, &w.out, &w.nout, (size_t)R * c->npatch, &g.out)) ||
+        (rc = ws_get(c, &w.xhi, &w.nxhi, plane, &g.xhi)) ||
+        (rc = ws_get(c, &w.xlo, &w.nxlo, plane, &g.xlo)) ||
+        (rc = ws_get(c, &w.parts, &w.nparts, (size_t)g.nblk, &g.parts)))
         return rc;
-    HIPCHK(c, hipMemsetAsync(g.E, 0, plane * 4, c->st));
-    HIPCHK(c, hipMemsetAsync(g.B, 0, plane * 4, c->st));
-    HIPCHK(c, hipMemsetAsync(g.rv, 0, plane * 4, c->st));
+    // the products read X whole: its padding is zero.  The vectors' padding is
+    // loaded with the rows beside it, but no result uses it.
     HIPCHK(c, hipMemsetAsync(g.xhi, 0, plane * 2, c->st));
     HIPCHK(c, hipMemsetAsync(g.xlo, 0, plane * 2, c->st));
     return RAD_OK;
@@ -1809,6 +1836,7 @@ int rad_dense_release(rad_ctx *c)
     if (!c)
         return RAD_E_ARG;
     (void)hipStreamSynchronize(c->st);
+    gather_free(c);
     dfree(c->fhi);
     dfree(c->flo);
     c->fhi = c->flo = nullptr;
@@ -1875,7 +1903,7 @@ int rad_gather_solve(rad_ctx *c, const float *rhs, uint32_t R, const rad_gather_
     launch_pad_columns(R, P, N, g.out, g.E, nullptr, nullptr, c->st);
     // B = 0, r = E; denominator sum_i A_i sum_r |E_ir|
     launch_gather_update(0, g.yp, g.ks1, g.rp, R, P, N, g.E, c->refl, c->area, g.rv, g.B, g.xhi,
-                         g.xlo, g.parts, g.nblk, c->st);
+                         g.xlo, g.parts, c->st);
     if ((rc = check_launch(c, "gather init")))
         return rc;
     double den = 0.0, num = 0.0;
@@ -1886,10 +1914,10 @@ int rad_gather_solve(rad_ctx *c, const float *rhs, uint32_t R, const rad_gather_
     rad_gather_stats st{};
     // events around the first sweep product and the residual product of
     // each step (device time of the two product kernels)
-    hipEvent_t ev[4] = {};
+    hipEvent_t *const ev = c->gw.ev;
     bool have_ev = true;
-    for (hipEvent_t &e : ev)
-        have_ev = have_ev && hipEventCreate(&e) == hipSuccess;
+    for (int k = 0; k < 4; ++k)
+        have_ev = have_ev && (ev[k] || hipEventCreate(&ev[k]) == hipSuccess);
     double t_sweep = 0.0, t_res = 0.0;
     while (res > target && outer < max_outer) {
         // correction d = r + diag(rho) M_bf16 d, `inner` sweeps from d = r,
@@ -1901,7 +1929,7 @@ int rad_gather_solve(rad_ctx *c, const float *rhs, uint32_t R, const rad_gather_
             if (s == 0 && have_ev)
                 (void)hipEventRecord(ev[1], c->st);
             launch_gather_update(s + 1 == inner ? 2 : 1, g.yp, g.ks1, g.rp, R, P, N, g.E, c->refl,
-                                 c->area, g.rv, g.B, g.xhi, g.xlo, g.parts, g.nblk, c->st);
+                                 c->area, g.rv, g.B, g.xhi, g.xlo, g.parts, c->st);
         }
         sweeps += inner;
         // residual r = E + diag(rho) M B - B from both halves, FP64 sums
@@ -1911,7 +1939,7 @@ int rad_gather_solve(rad_ctx *c, const float *rhs, uint32_t R, const rad_gather_
         if (have_ev)
             (void)hipEventRecord(ev[3], c->st);
         launch_gather_update(3, g.yp, g.ks2, g.rp, R, P, N, g.E, c->refl, c->area, g.rv, g.B, g.xhi,
-                             g.xlo, g.parts, g.nblk, c->st);
+                             g.xlo, g.parts, c->st);
         if ((rc = check_launch(c, "gather step")) || (rc = sum_parts(c, g, &num)))
             break;
         if (have_ev) {
@@ -1926,9 +1954,6 @@ int rad_gather_solve(rad_ctx *c, const float *rhs, uint32_t R, const rad_gather_
             st.history[outer] = res;
         ++outer;
     }
-    for (hipEvent_t e : ev)
-        if (e)
-            (void)hipEventDestroy(e);
     if (rc)
         return rc;
     st.sweep_ms = outer ? t_sweep / outer : 0.0;

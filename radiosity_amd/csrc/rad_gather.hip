@@ -479,54 +479,114 @@ __device__ __forceinline__ void block_sum_store(double v, double *parts)
 //  kOut     out = B + r
 enum { kInit = 0, kInner = 1, kLast = 2, kResid = 3 };
 
+// Bound by the S partial planes it reads (50 MB per sweep of 8,192 rows and
+// 192 columns): four consecutive rows per lane with 16-byte accesses, the
+// column from the grid (no division), and the partial sums of a lane loaded
+// four planes at a time before they are added in slice order.  That sweep's
+// update takes 13 us (3.9 TB/s); one element per lane and trip, with a 64-bit division
+// each, took 24.
+template <int KIND>
 __global__ __launch_bounds__(256) void k_gather_update(
-    int kind, const float *__restrict__ yp, GemmSplit ks, uint32_t rp, uint32_t R, uint32_t npad,
+    const float *__restrict__ yp, GemmSplit ks, uint32_t rp, uint32_t R, uint32_t npad,
     uint32_t n, const float *__restrict__ E, const float *__restrict__ refl,
     const float *__restrict__ area, float *__restrict__ rv, float *__restrict__ B,
     uint16_t *__restrict__ xhi, uint16_t *__restrict__ xlo, double *__restrict__ parts)
 {
     double acc = 0.0;
-    size_t total = (size_t)R * npad;
-    size_t stride = (size_t)gridDim.x * blockDim.x;
-    size_t plane = (size_t)rp * npad;
-    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < total; e += stride) {
-        uint32_t r = (uint32_t)(e / npad), i = (uint32_t)(e - (size_t)r * npad);
-        if (i >= n)
-            continue;
-        if (kind == kInit) {
-            float v = E[e];
-            rv[e] = v;
-            B[e] = 0.0f;
-            xhi[e] = bf16_rne(v);
-            acc += (double)area[i] * fabs((double)v);
+    const size_t plane = (size_t)rp * npad;
+    const uint32_t i = (blockIdx.x * 256u + threadIdx.x) * 4u;
+    const bool in = i < n;
+    // rsplit is a multiple of a workgroup's rows: a lane's rows lie on one side
+    const uint32_t S = i < ks.rsplit ? ks.S : ks.S2;
+    for (uint32_t r = blockIdx.y; in && r < R; r += gridDim.y) {
+        const size_t e = (size_t)r * npad + i;
+        if constexpr (KIND == kInit) {
+            const f32x4 v = *(const f32x4 *)(E + e);
+            *(f32x4 *)(rv + e) = v;
+            *(f32x4 *)(B + e) = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q)
+                if (i + q < n) {
+                    xhi[e + q] = bf16_rne(v[q]);
+                    acc += (double)area[i + q] * fabs((double)v[q]);
+                }
             continue;
         }
-        float y = 0.0f;
-        const uint32_t S = i < ks.rsplit ? ks.S : ks.S2;
-        for (uint32_t s = 0; s < S; ++s)
-            y += yp[s * plane + e];
-        float rho = refl[(size_t)i * 3 + r % 3];
-        if (kind == kResid) {
-            double res = (double)E[e] + (double)rho * (double)y - (double)B[e];
-            float rf = (float)res;
-            rv[e] = rf;
-            xhi[e] = bf16_rne(rf);
-            acc += (double)area[i] * fabs(res);
-        } else {
-            float d = rv[e] + rho * y;
-            if (kind == kInner) {
-                xhi[e] = bf16_rne(d);
+        f32x4 y = {0.f, 0.f, 0.f, 0.f};
+        for (uint32_t s = 0; s < S; s += 4) {
+            f32x4 p[4];
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q)
+                if (s + q < S)
+                    p[q] = *(const f32x4 *)(yp + (s + q) * plane + e);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q)
+                if (s + q < S)
+                    y += p[q];
+        }
+        const f32x4 old = *(const f32x4 *)(KIND == kResid ? B + e : rv + e);
+        const f32x4 ev = KIND == kResid ? *(const f32x4 *)(E + e) : f32x4{0.f, 0.f, 0.f, 0.f};
+        const f32x4 bv = KIND == kLast ? *(const f32x4 *)(B + e) : f32x4{0.f, 0.f, 0.f, 0.f};
+        f32x4 out = {0.f, 0.f, 0.f, 0.f};
+        uint16_t h[4] = {0, 0, 0, 0}, l[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            if (i + q >= n)
+                continue;
+            const float rho = refl[(size_t)(i + q) * 3 + r % 3];
+            if constexpr (KIND == kResid) {
+                const double res =
+                    (double)ev[q] + (double)rho * (double)y[q] - (double)old[q];
+                out[q] = (float)res;
+                h[q] = bf16_rne(out[q]);
+                acc += (double)area[i + q] * fabs(res);
             } else {
-                float b = B[e] + d;
-                B[e] = b;
-                uint16_t h = bf16_rne(b);
-                xhi[e] = h;
-                xlo[e] = bf16_rne(b - bf16_val(h));
+                const float d = old[q] + rho * y[q];
+                if constexpr (KIND == kInner) {
+                    h[q] = bf16_rne(d);
+                } else {
+                    out[q] = bv[q] + d;
+                    h[q] = bf16_rne(out[q]);
+                    l[q] = bf16_rne(out[q] - bf16_val(h[q]));
+                }
             }
         }
+        // rows past n hold zeros in X (the padding of the product) and
+        // nothing that is read in the vectors
+        *(uint2 *)(xhi + e) = uint2{h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16)};
+        if constexpr (KIND == kResid)
+            *(f32x4 *)(rv + e) = out;
+        if constexpr (KIND == kLast) {
+            *(f32x4 *)(B + e) = out;
+            *(uint2 *)(xlo + e) =
+                uint2{l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16)};
+        }
     }
-    if (kind == kInit || kind == kResid)
-        block_sum_store(acc, parts);
+    if constexpr (KIND == kInit || KIND == kResid) {
+        __shared__ double red[4];
+        for (int o = 32; o > 0; o >>= 1)
+            acc += __shfl_down(acc, o, 64);
+        if ((threadIdx.x & 63) == 0)
+            red[threadIdx.x >> 6] = acc;
+        __syncthreads();
+        if (threadIdx.x == 0)
+            parts[blockIdx.y * gridDim.x + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+    }
+}
+
+// Columns of the grid: all of them, or as many as make about 2,048 workgroups.
+static dim3 gather_grid(uint32_t R, uint32_t npad)
+{
+    const uint32_t bx = (npad + 1023u) / 1024u;
+    uint32_t by = 2048u / bx;
+    by = by < 1u ? 1u : by > R ? R : by;
+    return dim3(bx, by);
+}
+
+uint32_t gather_blocks(uint32_t R, uint32_t npad)
+{
+    const dim3 g = gather_grid(R, npad);
+    return g.x * g.y;
 }
 
 __global__ void k_gather_out(uint32_t R, uint32_t npad, uint32_t n, const float *__restrict__ B,
@@ -839,10 +899,26 @@ void launch_gemm(uint32_t rt, bool split, const uint16_t *fhi, const uint16_t *f
 void launch_gather_update(int kind, const float *yp, GemmSplit ks, uint32_t rp, uint32_t R,
                           uint32_t npad, uint32_t n, const float *E, const float *refl,
                           const float *area, float *rv, float *B, uint16_t *xhi, uint16_t *xlo,
-                          double *parts, uint32_t nblocks, hipStream_t st)
+                          double *parts, hipStream_t st)
 {
-    k_gather_update<<<nblocks, 256, 0, st>>>(kind, yp, ks, rp, R, npad, n, E, refl, area, rv, B,
-                                             xhi, xlo, parts);
+    const dim3 g = gather_grid(R, npad);
+    switch (kind) {
+    case kInit:
+        k_gather_update<kInit><<<g, 256, 0, st>>>(yp, ks, rp, R, npad, n, E, refl, area, rv, B,
+                                                  xhi, xlo, parts);
+        break;
+    case kInner:
+        k_gather_update<kInner><<<g, 256, 0, st>>>(yp, ks, rp, R, npad, n, E, refl, area, rv, B,
+                                                   xhi, xlo, parts);
+        break;
+    case kLast:
+        k_gather_update<kLast><<<g, 256, 0, st>>>(yp, ks, rp, R, npad, n, E, refl, area, rv, B,
+                                                  xhi, xlo, parts);
+        break;
+    default:
+        k_gather_update<kResid><<<g, 256, 0, st>>>(yp, ks, rp, R, npad, n, E, refl, area, rv, B,
+                                                   xhi, xlo, parts);
+    }
 }
 
 void launch_gather_out(uint32_t R, uint32_t npad, uint32_t n, const float *B, const float *rv,

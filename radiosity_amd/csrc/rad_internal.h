@@ -326,10 +326,12 @@ GemmSplit gemm_split(uint32_t rt, bool split, uint32_t npad, uint32_t S, uint32_
 void launch_gemm(uint32_t rt, bool split, const uint16_t *fhi, const uint16_t *flo,
                  const uint16_t *xhi, const uint16_t *xlo, uint32_t npad, GemmSplit ks,
                  float *yp, hipStream_t st);
+// Workgroups (and partial sums) of a launch_gather_update over R columns.
+uint32_t gather_blocks(uint32_t R, uint32_t npad);
 void launch_gather_update(int kind, const float *yp, GemmSplit ks, uint32_t rp, uint32_t R,
                           uint32_t npad, uint32_t n, const float *E, const float *refl,
                           const float *area, float *rv, float *B, uint16_t *xhi, uint16_t *xlo,
-                          double *parts, uint32_t nblocks, hipStream_t st);
+                          double *parts, hipStream_t st);
 // FP64 residual check of a gather solution against rendered FP32 rows
 // (shooting layout), one pass of k rows at a time; R <= kCheckMaxR (16).
 void launch_check_accum(const float *ff, uint32_t k, uint32_t row0, uint32_t rowlen, uint32_t n,

@@ -170,7 +170,8 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
                                 c->nshoot, c->bb, c->counters, c->pk.slot_tbeg,
                                 c->pk.slot_tcnt, c->pk.slot_w, st);
         else if (j == 1)
-            launch_bin(s0, s1, h, c->nshoot, c->bb, c->counters, st);
+            launch_bin(c->g, s0, s1, h, c->tri, c->tri_patch, c->ntri, c->mvp, c->bb, c->counters,
+                       c->pk.slot_w, st);
         else
             launch_tile(c->g, s0, s1, h, c->nshoot, c->bb, c->small_px, ids, depth,
                         c->pk.slot_w ? c->pk.dffs : c->dff, c->rowlen, c->pk.slot_pbeg,
@@ -365,6 +366,21 @@ int one_pass(rad_ctx *c, bool do_select, size_t evbase, bool chain_in = false,
     return check_launch(c, "shoot");
 }
 
+// The bins' lists: room for 16 times the records per bin of a scene spread
+// evenly over the tiles, within 4 GiB in all.  A fuller bin is drawn from its
+// slot's records without a list (k_tile_raster), so the size is no limit.
+int bin_lists(rad_ctx *c)
+{
+    const uint64_t ntri = (uint64_t)c->bb.nblk * 256;
+    uint32_t cap = 256;
+    while (cap < 65536 && (uint64_t)cap * c->bb.ntiles < 16 * ntri)
+        cap *= 2;
+    while (cap > 256 && (uint64_t)c->bb.nbins * cap > (1ull << 30))
+        cap /= 2;
+    c->bb.bin_cap = cap;
+    return dalloc(c, &c->bb.list, (size_t)c->bb.nbins * cap);
+}
+
 // Screen tile side T (8, 16, 32) and the in-lane triangle limit; (re)sizes
 // the per-(shooter, tile) bin arrays.
 int set_tiles(rad_ctx *c, uint32_t T, uint32_t small_px)
@@ -388,10 +404,11 @@ int set_tiles(rad_ctx *c, uint32_t T, uint32_t small_px)
     drop_graph(c);
     size_t nbins = (size_t)c->K * c->bb.ntiles;
     int rc;
-    if ((rc = dalloc(c, &c->bb.count, nbins)) || (rc = dalloc(c, &c->bb.start, nbins)) ||
-        (rc = dalloc(c, &c->bb.fill, nbins)) || (rc = dalloc(c, &c->bb.order, nbins)))
+    c->bb.nbins = (uint32_t)nbins;
+    if ((rc = dalloc(c, &c->bb.count, nbins)) ||
+        (rc = dalloc(c, &c->bb.order, nbins * kBinClasses)))
         return rc;
-    return RAD_OK;
+    return c->npatch ? bin_lists(c) : RAD_OK;
 }
 
 int need_scene(rad_ctx *c)
@@ -515,7 +532,7 @@ void rad_destroy(rad_ctx *c)
                     c->item_depth, c->ffq, c->runs_slots, c->runs_offs, c->trip_h, c->trip_i,
                     c->trip_e,
                     c->mvp,  c->snap,     c->shooters, c->nshoot, c->counters, c->ctl, c->sel,
-                    c->resid, c->bb.recs, c->bb.count, c->bb.start, c->bb.fill,
+                    c->resid, c->bb.recs, c->bb.count,
                     c->bb.list, c->bb.blk_nrec, c->bb.bbox, c->bb.clipq, c->cand, c->parts, c->bb.order,
                     c->fhi,  c->flo,      c->pk.sc_tbeg, c->pk.sc_pbeg, c->pk.sc_slots,
                     c->pk.sc_slot_beg, c->pk.sc_nsel, c->pk.sc_done, c->pk.sc_den, c->pk.sc_res,
@@ -644,14 +661,13 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     c->bb.spill_base = (uint32_t)regions;
     c->bb.spill_cap = (uint32_t)spill;
     c->bb.clip_cap = (uint32_t)(spill / 2);
-    c->bb.clip_blocks = 512;
+    c->bb.clip_blocks = 128;
     uint64_t went = 2 * (regions + spill);
     c->bb.ent_cap = (uint32_t)(went > 0xF0000000ull ? 0xF0000000ull : went);
-    // each half of a split pass has its own spill region, list area and
-    // clipping queue
+    // each half of a split pass has its own spill region and clipping queue
     const uint64_t nrec = regions + kCntBlocks * spill;
     if ((rc = dalloc(c, &c->bb.recs, nrec)) || (rc = dalloc(c, &c->bb.bbox, nrec)) ||
-        (rc = dalloc(c, &c->bb.list, (size_t)kCntBlocks * c->bb.ent_cap)) ||
+        (rc = bin_lists(c)) || (rc = dalloc(c, &c->bb.pool, (size_t)kCntBlocks * c->bb.ent_cap)) ||
         (rc = dalloc(c, &c->bb.blk_nrec, (size_t)c->bb.nblk * K * c->bb.nz)) ||
         (rc = dalloc(c, &c->bb.clipq, (size_t)kCntBlocks * c->bb.clip_cap)) ||
         (rc = dalloc(c, &c->cand, 2 * topk_cand_half(npatch, c->K))))
@@ -1514,13 +1530,13 @@ int rad_debug_counters(rad_ctx *c, uint32_t *out8, uint32_t *caps)
 {
     if (!c || !out8)
         return RAD_E_ARG;
-    static_assert(kCntN == 8, "eight pass counters");
+    static_assert(kCntClass == 8, "eight pass counters");
     HIPCHK(c, hipStreamSynchronize(c->st));
     uint32_t cnt[kCntN * kCntBlocks];
     HIPCHK(c, hipMemcpy(cnt, c->counters, sizeof(cnt), hipMemcpyDeviceToHost));
     // the halves of a split pass: flags OR, unknown ids add up, and the
     // fill levels are the fuller half's (each half has the capacities)
-    for (int i = 0; i < kCntN; ++i) {
+    for (int i = 0; i < kCntClass; ++i) {
         out8[i] = 0;
         for (int h = 0; h < kCntBlocks; ++h) {
             const uint32_t v = cnt[h * kCntN + i];
@@ -1560,13 +1576,19 @@ int rad_debug_bins(rad_ctx *c, uint32_t *out, uint32_t *ntiles, uint32_t *tile_p
         launch_raster_setup(c->g, 0, c->last_k, 0, c->tri, c->tsph, c->tri_patch, c->ntri, c->mvp,
                             c->nshoot, c->bb, cnt, c->pk.slot_tbeg, c->pk.slot_tcnt, c->pk.slot_w,
                             c->st);
+        launch_bin(c->g, 0, c->last_k, 0, c->tri, c->tri_patch, c->ntri, c->mvp, c->bb, cnt,
+                   c->pk.slot_w, c->st);
         const hipError_t e = hipStreamSynchronize(c->st);
         dfree(cnt);
         HIPCHK(c, e);
         c->last_direct = false;
     }
-    if (out)
-        HIPCHK(c, hipMemcpy(out, c->bb.count, (size_t)c->K * c->bb.ntiles * 4, hipMemcpyDeviceToHost));
+    if (out) {
+        const size_t n = (size_t)c->K * c->bb.ntiles;
+        HIPCHK(c, hipMemcpy(out, c->bb.count, n * 4, hipMemcpyDeviceToHost));
+        for (size_t i = 0; i < n; ++i)
+            out[i] &= ~kBinSeen;
+    }
     return RAD_OK;
 }
 

@@ -48,11 +48,29 @@ enum {
     kCntSpill = 5,    // records in the spill region
     kCntClip = 6,     // triangle-face jobs queued for clipping
     kCntSticky = 7,   // some earlier pass overflowed (cleared by the host only)
-    kCntN = 8
+    kCntFacts = 4,    // a BinFacts begins here
+    kCntClass = 8,    // bins of each size class of the launch order
+    kCntPool = 30,    // entries reserved in the pool of whole lists
+    kCntN = 32
 };
+constexpr uint32_t kBinClasses = 8;     // size classes of the launch order
+constexpr uint32_t kBinSeen = 0x80000000u; // in a bin's count: summed into kCntEntries
+constexpr uint32_t kSplitRecs = 1536;   // records from which a bin is drawn as quadrants
+// What the tile kernel reads beside its arguments: counters of the pass, and
+// what only a bin fuller than its list needs.
+struct BinFacts {
+    uint32_t unknown, nspill, nclip, sticky; // counters 4 .. 7
+    uint32_t cls[kBinClasses];
+    const uint32_t *blk_nrec;
+    uint32_t *pool, *pool_used;
+    uint32_t nreg, spill_base, spill_cap, pool_cap, split_cap, pad;
+};
+static_assert((kCntFacts + 4) == kCntClass && kCntFacts * 4 + sizeof(BinFacts) <= kCntPool * 4 &&
+                  kCntFacts % 2 == 0 && kCntN % 2 == 0,
+              "its place among the counters");
 // A pass may render as two halves on two streams (slots [0, k/2) and
-// [k/2, k)), each with its own block of kCntN counters, spill region, clip
-// queue and list area; the sticky flag lives in the first block.
+// [k/2, k)), each with its own block of kCntN counters, spill region and
+// clip queue; the sticky flag lives in the first block.
 constexpr int kCntBlocks = 2;
 constexpr uint32_t kSplitMin = 16; // smallest pass rendered as two halves
 // ... and the fewest bins (slots x tiles): the halves overlap each other's
@@ -63,7 +81,7 @@ constexpr uint32_t kSplitMin = 16; // smallest pass rendered as two halves
 // 32 shooters at hemicube 256 (6,144) 277 -> 279; 20 at hemicube 128 247 -> 263;
 // 16 at hemicube 64 82 -> 93.
 constexpr uint32_t kSplitBins = 8192;
-// Workgroups the setup and the bin fill should have before each walks more
+// Workgroups the setup should have before each walks more
 // than one shooter slot (then up to 8, which reads the vertices once per 8
 // shooters).  About five per CU are resident; walking 8 slots whatever the
 // scene left most CUs idle below 200,000 triangles.  A pass of 64 shooters,
@@ -87,11 +105,13 @@ enum {
 // Bins of the sort-middle rasterizer: one per (shooter slot, tile).
 struct BinBuffers {
     RasterRec *recs;       // nblk*K regions of kRecsPerBlock, then kCntBlocks spill regions of spill_cap
-    uint64_t *bbox;        // texel bbox per record slot, read by the bin fill
+    uint64_t *bbox;        // texel bbox per record slot, of which the lists are made
     uint32_t *blk_nrec;    // records per (shooter, setup block)
-    uint32_t *count, *start, *fill;
-    uint32_t *list;        // kCntBlocks list areas of ent_cap entries
-    uint32_t *order;       // bins by descending size class (tile launch order)
+    uint32_t *count;       // records per bin
+    uint32_t *list;        // bin_cap record slots per bin
+    uint32_t *pool;        // kCntBlocks areas of ent_cap entries: lists of fuller bins
+    uint32_t *order;       // kBinClasses queues of nbins bins (tile launch order)
+    uint32_t nbins, bin_cap;
     uint32_t nblk;         // setup blocks per shooter and face group (256 triangles each)
     uint32_t nz;           // face groups: 5 (one face per block, small K) or 1
     uint32_t spill_base, spill_cap, ent_cap;
@@ -163,19 +183,19 @@ void launch_clear(uint32_t K, uint32_t *bin_count, uint32_t ntiles, float *ff, u
                   uint32_t ff_rows, uint32_t rowlen, uint32_t *counters, uint32_t ent_cap,
                   hipStream_t st);
 // Binned render of the shooter slots [s0, s1) (of which those below nshoot
-// are drawn) in three launches: setup (records + bin counts), bin (scan +
-// fill), tile (LDS depth test; out_ids != null writes the item buffer, ff or
-// ffq != null reduces into F rows and hits).  h selects the counter block,
-// spill region, clip queue and list area (0, or 1 for the second half of a
-// split pass).
+// are drawn) in three launches: setup (records and bins), bin (launch order
+// of the bins, clipped triangles), tile (LDS depth test; out_ids != null
+// writes the item buffer, ff or ffq != null reduces into F rows and hits).  h selects the counter block,
+// spill region and clip queue (0, or 1 for the second half of a split pass).
 void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h,
                          const float *tri, const float4 *tsph, const uint32_t *tri_patch,
                          uint32_t ntri, const float *mvp, const uint32_t *nshoot,
                          const BinBuffers &bb, uint32_t *counters, const uint32_t *slot_tbeg,
                          const uint32_t *slot_tcnt, const uint32_t *slot_w, hipStream_t st);
 void launch_tri_sphere(const float *tri, uint32_t ntri, float4 *sph, hipStream_t st);
-void launch_bin(uint32_t s0, uint32_t s1, uint32_t h, const uint32_t *nshoot,
-                const BinBuffers &bb, uint32_t *counters, hipStream_t st);
+void launch_bin(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const float *tri,
+                const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const BinBuffers &bb,
+                uint32_t *counters, const uint32_t *slot_w, hipStream_t st);
 void launch_tile(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const uint32_t *nshoot,
                  const BinBuffers &bb, uint32_t small_px, uint32_t *out_ids, float *out_depth,
                  const float *dff, uint32_t rowlen, const uint32_t *slot_pbeg, float *ff,

@@ -12,10 +12,9 @@
 //                  counts and pass counters reset, F rows zeroed unless the
 //                  previous shoot left them zero
 //   k_raster_setup one lane per (triangle, shooter) over the five faces:
-//                  cull, transform, clip, snap; records counted into tile bins
-//   k_setup_clipped  the few triangle-faces that cross the near plane or the
-//                  guard band
-//   k_bin_scan / k_bin_fill   bin offsets and record lists
+//                  cull, transform, snap; records into the tiles' lists
+//   k_order_clip   the launch order of the tiles; the few triangle-faces that
+//                  cross the near plane or the guard band
 //   k_tile_raster  one workgroup per (shooter, tile): depth test in LDS, then
 //                  the tile's item buffer out or ProcessHemicube fused
 //   k_reduce       ProcessHemicube over a whole item buffer (wave-level
@@ -259,9 +258,10 @@ __device__ static void clear_range(size_t i, size_t stride, uint32_t *__restrict
         for (int h = 0; h < kCntBlocks; ++h)
             bad = bad || counters[h * kCntN + kCntOverflow] != 0 ||
                   counters[h * kCntN + kCntEntries] > ent_cap;
-        for (int k = 0; k < kCntN * kCntBlocks; ++k)
-            if (k != kCntSticky)
-                counters[k] = 0;
+        for (int h = 0; h < kCntBlocks; ++h)
+            for (int k = 0; k < kCntN; ++k)
+                if (h || k != kCntSticky)
+                    counters[h * kCntN + k] = 0;
         if (bad)
             counters[kCntSticky] = 1;
     }
@@ -348,11 +348,11 @@ void launch_clear(uint32_t K, uint32_t *bin_count, uint32_t ntiles, float *ff, u
 // ---------------------------------------------------------------- rasterizer
 // Sort-middle rasterizer.
 //  k_raster_setup  one lane per (triangle, shooter), looping over the five
-//                  faces: cull, transform, clip, snap; every surviving
-//                  (sub-)triangle becomes a RasterRec and is counted in the
-//                  bins of the screen tiles its bbox touches
-//  k_bin_scan      exclusive scan of the bin counts
-//  k_bin_fill      record indices into their bins
+//                  faces: cull, transform, snap; every surviving triangle
+//                  becomes a RasterRec and is listed in the bins of the
+//                  screen tiles its bbox touches
+//  k_order_clip    the bins by size, for the launch order of the tiles; the
+//                  triangles to clip, as records of their own
 //  k_tile_raster   one workgroup per tile: depth test in LDS with 64-bit
 //                  atomicMin, then either writes the tile's ids and depths
 //                  (item buffer out) or reduces it into form factors
@@ -369,32 +369,48 @@ struct BinCtx {
     uint2 *clipq;          // (triangle, shooter * 8 + face) jobs that need clipping
     uint32_t clip_cap;
     uint32_t ntx, ntiles, tshift; // tiles per row, per hemicube, log2(tile side)
+    uint32_t *list;        // bin_cap entries (record slots) per bin
+    uint32_t bin_cap;
 };
 
-// Emits a snapped triangle (face-local coordinates) as a record into the
-// block's region (spill region when full) and counts it in the LDS
-// histogram of the tiles its texel bbox touches.
-__device__ static void emit_tri(const SV &a, const SV &b, const SV &c, uint32_t id,
-                                const FaceView &fv, uint32_t s, int face, const BinCtx &bc)
+// Record r into the list of a bin at place pos (bins hold bin_cap entries;
+// the tile kernel draws a fuller one from the records themselves).
+__device__ static inline void list_put(const BinCtx &bc, uint32_t s, uint32_t tile, uint32_t pos,
+                                       uint32_t r)
+{
+    if (pos < bc.bin_cap)
+        bc.list[((size_t)s * bc.ntiles + tile) * bc.bin_cap + pos] = r;
+}
+
+// A record of a triangle and the tiles [g0, g1] x [h0, h1] of its texel bbox.
+struct Placed {
+    uint32_t r, g0, g1, h0, h1;
+};
+
+// The record of a snapped triangle (face-local coordinates) into the block's
+// region or, when that is full (or for a clipped triangle), into the spill
+// region: 0 no record, 1 region, 2 spill.
+__device__ static inline int place_tri(const SV &a, const SV &b, const SV &c, uint32_t id,
+                                       const FaceView &fv, uint32_t s, int face, const BinCtx &bc,
+                                       Placed &p)
 {
     int64_t area2;
     int32_t ix0, iy0, ix1, iy1;
     if (!snapped_bbox(a, b, c, fv.sx0, fv.sy0, fv.sx1, fv.sy1, area2, ix0, iy0, ix1, iy1))
-        return;
+        return 0;
     uint32_t slot = bc.lnrec ? atomicAdd(bc.lnrec, 1u) : kRecsPerBlock;
-    uint32_t r;
     bool local = slot < kRecsPerBlock;
     if (local) {
-        r = bc.region + slot;
+        p.r = bc.region + slot;
     } else {
         if (bc.lnrec)
             atomicSub(bc.lnrec, 1u);
         uint32_t q = atomicAdd(&bc.counters[kCntSpill], 1u);
         if (q >= bc.spill_cap) {
             atomicOr(&bc.counters[kCntOverflow], 1u);
-            return;
+            return 0;
         }
-        r = bc.spill_base + q;
+        p.r = bc.spill_base + q;
     }
     RasterRec rr;
     make_record(a, b, c, area2, id, rr);
@@ -402,25 +418,45 @@ __device__ static void emit_tri(const SV &a, const SV &b, const SV &c, uint32_t 
     rr.pad = 0u;
     // bbox in texel coordinates of the hemicube slab
     int32_t tx0 = fv.vpx + ix0, tx1 = fv.vpx + ix1, ty0 = fv.vpy + iy0, ty1 = fv.vpy + iy1;
-    bc.recs[r] = rr;
-    bc.bbox[r] = (uint64_t)(uint16_t)tx0 | ((uint64_t)(uint16_t)ty0 << 16) |
-                 ((uint64_t)(uint16_t)tx1 << 32) | ((uint64_t)(uint16_t)ty1 << 48);
-    uint32_t g0 = (uint32_t)tx0 >> bc.tshift, g1 = (uint32_t)tx1 >> bc.tshift;
-    uint32_t h0 = (uint32_t)ty0 >> bc.tshift, h1 = (uint32_t)ty1 >> bc.tshift;
-    if (local) {
-        for (uint32_t gy = h0; gy <= h1; ++gy)
-            for (uint32_t gx = g0; gx <= g1; ++gx)
-                atomicAdd(&bc.lcnt[gy * bc.ntx + gx], 1u);
-    } else {
-        uint32_t *cnt = bc.bin_count + (size_t)s * bc.ntiles;
-        for (uint32_t gy = h0; gy <= h1; ++gy)
-            for (uint32_t gx = g0; gx <= g1; ++gx)
-                atomicAdd(&cnt[gy * bc.ntx + gx], 1u);
-    }
+    bc.recs[p.r] = rr;
+    bc.bbox[p.r] = (uint64_t)(uint16_t)tx0 | ((uint64_t)(uint16_t)ty0 << 16) |
+                   ((uint64_t)(uint16_t)tx1 << 32) | ((uint64_t)(uint16_t)ty1 << 48);
+    p.g0 = (uint32_t)tx0 >> bc.tshift;
+    p.g1 = (uint32_t)tx1 >> bc.tshift;
+    p.h0 = (uint32_t)ty0 >> bc.tshift;
+    p.h1 = (uint32_t)ty1 >> bc.tshift;
+    return local ? 1 : 2;
+}
+
+// A spill record straight into the list of tile b of slot s.
+__device__ static inline void bin_spilled(const BinCtx &bc, uint32_t s, uint32_t b, uint32_t r)
+{
+    const uint32_t pos = atomicAdd(&bc.bin_count[(size_t)s * bc.ntiles + b], 1u);
+    if (pos & kBinSeen) // k_order_clip has summed the counts
+        atomicAdd(&bc.counters[kCntEntries], 1u);
+    list_put(bc, s, b, pos & ~kBinSeen, r);
+}
+
+// place_tri, and a region record counted in the LDS histogram of its tiles.
+__device__ static void emit_tri(const SV &a, const SV &b, const SV &c, uint32_t id,
+                                const FaceView &fv, uint32_t s, int face, const BinCtx &bc)
+{
+    Placed p;
+    const int where = place_tri(a, b, c, id, fv, s, face, bc, p);
+    if (where == 0)
+        return;
+    for (uint32_t gy = p.h0; gy <= p.h1; ++gy)
+        for (uint32_t gx = p.g0; gx <= p.g1; ++gx) {
+            const uint32_t t = gy * bc.ntx + gx;
+            if (where == 1)
+                atomicAdd(&bc.lcnt[t], 1u);
+            else
+                bin_spilled(bc, s, t, p.r);
+        }
 }
 
 // Exact per-face pipeline of one triangle up to the record.  Triangles that
-// need clipping (near plane or guard band) are queued for k_setup_clipped.
+// need clipping (near plane or guard band) are queued for k_order_clip.
 // mm: the face's MVP, scis: face_scissor_clip of the face.
 __device__ static inline void setup_face(const float *mm, float4 scis, const float (&vx)[3][3],
                                          uint32_t W, uint32_t s, int face, uint32_t id,
@@ -443,47 +479,6 @@ __device__ static inline void setup_face(const float *mm, float4 scis, const flo
     float halfW = 0.5f * (float)W;
     SV a = project(poly[0], halfW), b = project(poly[1], halfW), c = project(poly[2], halfW);
     emit_tri(a, b, c, id, fv, s, face, bc);
-}
-
-// Queued (triangle, shooter, face) jobs that cross the near plane or the
-// guard band, one per wavefront (a 64-thread workgroup): lanes 0 .. 2
-// transform their vertex as transform3 does, the wavefront clips, and the fan
-// triangles (0, k, k + 1) are emitted by lanes k = 1 .. n - 2 at once; records
-// go to the spill region.
-__global__ __launch_bounds__(64) void k_setup_clipped(uint32_t W, const float *__restrict__ tri,
-                                                       const uint32_t *__restrict__ tri_patch,
-                                                       uint32_t ntri, const float *__restrict__ mvp,
-                                                       BinCtx bc,
-                                                       const uint32_t *__restrict__ slot_w)
-{
-    __shared__ CV4 lp[kClipMax];
-    const uint32_t lane = threadIdx.x;
-    const uint32_t n = min(bc.counters[kCntClip], bc.clip_cap);
-    for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
-        const uint2 job = bc.clipq[q];
-        const uint32_t t = job.x, s = job.y >> 3;
-        const int face = (int)(job.y & 7u);
-        CV4 v;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            v.c[c] = 0.0f;
-        if (lane < 3) {
-            const float x = tri[(size_t)(3 * lane + 0) * ntri + t];
-            const float y = tri[(size_t)(3 * lane + 1) * ntri + t];
-            const float z = tri[(size_t)(3 * lane + 2) * ntri + t];
-            const float *mm = mvp + (size_t)s * kShooterStride + face * 16;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                v.c[r] = mm[0 * 4 + r] * x + mm[1 * 4 + r] * y + mm[2 * 4 + r] * z + mm[3 * 4 + r];
-        }
-        const uint32_t Ws = slot_w ? slot_w[s] : W;
-        FaceView fv = face_view((int32_t)Ws, face);
-        const int np = clip_polygon_wave(v, lp, &bc.counters[kCntOverflow]);
-        SV a, b, cc;
-        if (np >= 3 && clip_fan(v, np, 0.5f * (float)Ws, a, b, cc))
-            emit_tri(a, b, cc, tri_patch[t] + 1u, fv, s, face, bc);
-        __syncthreads(); // lp is the next job's
-    }
 }
 
 __device__ static uint32_t cull_faces(const float *__restrict__ sm, const float (&vx)[3][3],
@@ -519,12 +514,26 @@ void launch_tri_sphere(const float *tri, uint32_t ntri, float4 *sph, hipStream_t
         k_tri_sphere<<<(ntri + 255) / 256, 256, 0, st>>>(tri, ntri, sph);
 }
 
+// Tile columns [g0, g1] and rows [h0, h1] of a record's texel bbox.
+__device__ static inline void unpack_bbox(uint64_t v, uint32_t tshift, uint32_t &g0,
+                                          uint32_t &g1, uint32_t &h0, uint32_t &h1)
+{
+    g0 = (uint32_t)(v & 0xFFFFu) >> tshift;
+    h0 = (uint32_t)((v >> 16) & 0xFFFFu) >> tshift;
+    g1 = (uint32_t)((v >> 32) & 0xFFFFu) >> tshift;
+    h1 = (uint32_t)(v >> 48) >> tshift;
+}
+
 // One workgroup per (256 triangles, shooter[, face]).  Phase 1: one lane
 // per triangle runs the conservative culls (cull_faces) and queues the
 // surviving (triangle, face) pairs in LDS; phase 2: the lanes take the queue
 // so the exact pipeline runs with every lane busy.  Records go to the block's
-// own region (LDS slot counter) and are counted in an LDS tile histogram,
-// flushed with one global atomic per touched tile.  Triangles are stored as 9
+// own region (LDS slot counter) and are counted in an LDS tile histogram;
+// phase 3 reserves their places in the tiles' lists with one returning global
+// atomic per touched tile and writes them there, which took the place of a
+// scan over all bins and a fill kernel that read the bboxes back: over
+// 200,000 triangles at hemicube 256 a pass of one shooter takes 109 us
+// instead of 125, one of 64 shooters 343 instead of 376.  Triangles are stored as 9
 // planes of ntri floats (v0.x, v0.y, ..., v2.z) so consecutive lanes load
 // consecutive addresses.
 // In a packed launch slot s draws only its scene's triangles
@@ -583,7 +592,7 @@ __global__ __launch_bounds__(256) void k_raster_setup(uint32_t W, const float *_
             ++nsh;
         }
         if (tl0 >= tc) {
-            // beyond the slots' scene: empty regions for the bin fill
+            // beyond the slots' scene: empty regions
             if (threadIdx.x < nsh)
                 blk_nrec[rbof(s + threadIdx.x)] = 0u;
             g += nsh;
@@ -655,15 +664,31 @@ __global__ __launch_bounds__(256) void k_raster_setup(uint32_t W, const float *_
                        tb + tl0 + tl, b2);
         }
         __syncthreads();
-        // flush: one global atomic per touched tile, and the regions' record counts
-        for (uint32_t sh = 0; sh < nsh; ++sh) {
-            uint32_t *cnt = bc.bin_count + (size_t)(s + sh) * bc.ntiles;
-            for (uint32_t i = threadIdx.x; i < bc.ntiles; i += blockDim.x)
-                if (lcnt[sh * bc.ntiles + i])
-                    atomicAdd(&cnt[i], lcnt[sh * bc.ntiles + i]);
-        }
+        // the records into their tiles' lists: one returning global atomic per
+        // touched tile reserves the entries, whose first place takes the
+        // count's place in LDS ...
+        uint32_t *const cnt = bc.bin_count + (size_t)s * bc.ntiles;
+        for (uint32_t i = threadIdx.x; i < nsh * bc.ntiles; i += blockDim.x)
+            if (lcnt[i])
+                lcnt[i] = atomicAdd(&cnt[i], lcnt[i]);
         if (threadIdx.x < nsh)
             blk_nrec[rbof(s + threadIdx.x)] = lnrec2[threadIdx.x];
+        __syncthreads();
+        // ... and every record counts on from it
+        const uint32_t e1 = lnrec2[0], e2 = e1 + lnrec2[1], e3 = e2 + lnrec2[2],
+                       e4 = e3 + lnrec2[3];
+        for (uint32_t f = threadIdx.x; f < e4; f += blockDim.x) {
+            const uint32_t sh = (f >= e1 ? 1u : 0u) + (f >= e2 ? 1u : 0u) + (f >= e3 ? 1u : 0u);
+            const uint32_t q = f - (sh == 0 ? 0u : sh == 1 ? e1 : sh == 2 ? e2 : e3);
+            const uint32_t r = rbof(s + sh) * kRecsPerBlock + q;
+            uint32_t g0, g1, h0, h1;
+            unpack_bbox(bc.bbox[r], bc.tshift, g0, g1, h0, h1);
+            for (uint32_t gy = h0; gy <= h1; ++gy)
+                for (uint32_t gx = g0; gx <= g1; ++gx) {
+                    const uint32_t b = gy * bc.ntx + gx;
+                    list_put(bc, s + sh, b, atomicAdd(&lcnt[sh * bc.ntiles + b], 1u), r);
+                }
+        }
         g += nsh;
     }
 }
@@ -732,261 +757,160 @@ __device__ static uint32_t cull_faces(const float *__restrict__ sm, const float 
     return mask;
 }
 
-// Exclusive scan of n bin counts by one block of 1024 threads; writes start
-// offsets, resets the fill counters and stores the total in
-// counters[kCntEntries].  The counts go through LDS in chunks of
-// kScanChunk: every thread issues its kScanPer coalesced loads at once, then
-// scans kScanPer contiguous counts from LDS, so a chunk costs one memory
-// latency instead of one per count.
-// Also orders the bins for the tile kernel by descending size class
-// (floor(log2(count)) buckets, a counting sort): the largest bins start
-// first, so the heavy horizon tiles overlap the light ones instead of
-// forming the tail of the launch.  The arrays given start at bin bin0 of the
-// pass (a half-pass scans its own bins); the order holds pass bin numbers.
-constexpr uint32_t kScanPer = 8, kScanChunk = 1024 * kScanPer;
+// The launch order of the bins [bin0, bin0 + n) for the tile kernel, largest
+// first, so that the heavy horizon tiles overlap the light ones instead of
+// forming the tail of the launch: each bin goes to the queue of its size
+// class (queue c at order + c * qstride; a class's counter of the pass
+// counters reserves the places).  Class 0 holds the bins that the tile kernel
+// draws as four quadrants, at most split_cap of them.  A thread's bins, and
+// the bins of neighbouring threads, are far apart on the hemicube: that ran
+// measurably faster in the tile kernel than neighbouring tiles launched
+// together.
+//
+// The workgroups from norder on clip: the queued (triangle, shooter, face)
+// jobs that cross the near plane or the guard band, one per wavefront: lanes
+// 0 .. 2 transform their vertex as transform3 does, the wavefront clips, and
+// the fan triangles (0, k, k + 1) are emitted by lanes k = 1 .. n - 2 at
+// once; records go to the spill region and straight into the lists.  The
+// order may miss their counts: every bin is in it whatever its count.  The
+// entry total misses none: an order workgroup marks the bins it has summed
+// (kBinSeen), and an entry that finds the mark adds itself.
+// Latency-bound: 6 us for one shooter over 200,000 triangles, 16 us for each
+// half of 64 (a scan kernel and a clip kernel took 10 and 21).
+constexpr uint32_t kOrderPer = 4;
 
-__device__ static inline uint32_t size_class(uint32_t c)
+__device__ static inline uint32_t order_class(uint32_t n, uint32_t split_max)
 {
-    return c ? 32u - __clz(c) : 0u;
+    if (n >= kSplitRecs && n <= split_max)
+        return 0u;
+    return n >= 2048u ? 1u : n >= 1024u ? 2u : n >= 512u ? 3u : n >= 256u ? 4u : n >= 128u ? 5u
+           : n >= 64u ? 6u : 7u;
 }
 
-__global__ __launch_bounds__(1024) void k_bin_scan(const uint32_t *__restrict__ cnt,
-                                                   uint32_t *__restrict__ start,
-                                                   uint32_t *__restrict__ fill, uint32_t n,
-                                                   uint32_t *__restrict__ counters,
-                                                   uint32_t *__restrict__ order, uint32_t bin0)
+__global__ __launch_bounds__(256) void k_order_clip(uint32_t norder, uint32_t n, uint32_t bin0,
+                                                    uint32_t split_cap,
+                                                    uint32_t *__restrict__ order,
+                                                    uint32_t qstride, uint32_t W,
+                                                    const float *__restrict__ tri,
+                                                    const uint32_t *__restrict__ tri_patch,
+                                                    uint32_t ntri, const float *__restrict__ mvp,
+                                                    BinCtx bc,
+                                                    const uint32_t *__restrict__ blk_nrec,
+                                                    uint32_t nreg, uint32_t *__restrict__ pool,
+                                                    uint32_t pool_cap,
+                                                    const uint32_t *__restrict__ slot_w)
 {
-    __shared__ uint32_t lc[kScanChunk];
-    __shared__ uint32_t wsum[16];
-    __shared__ uint32_t bucket[33], boff[33];
-    __shared__ uint32_t carry;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    if (tid < 33)
-        bucket[tid] = 0u;
-    if (tid == 0)
-        carry = 0u;
-    __syncthreads();
-    for (uint32_t c0 = 0; c0 < n; c0 += kScanChunk) {
-        uint32_t v[kScanPer];
-#pragma unroll
-        for (uint32_t k = 0; k < kScanPer; ++k) {
-            const uint32_t i = c0 + k * 1024u + tid;
-            v[k] = i < n ? cnt[i] : 0u;
+    __shared__ uint32_t lcls[kBinClasses], gcls[kBinClasses], lsum;
+    __shared__ CV4 lp[4][kClipMax];
+    if (blockIdx.x < norder) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            BinFacts *const f = reinterpret_cast<BinFacts *>(bc.counters + kCntFacts);
+            f->blk_nrec = blk_nrec;
+            f->nreg = nreg;
+            f->spill_base = bc.spill_base;
+            f->spill_cap = bc.spill_cap;
+            f->split_cap = split_cap;
+            f->pool = pool;
+            f->pool_cap = pool_cap;
+            f->pool_used = &bc.counters[kCntPool];
         }
-#pragma unroll
-        for (uint32_t k = 0; k < kScanPer; ++k) {
-            const uint32_t i = c0 + k * 1024u + tid;
-            lc[k * 1024u + tid] = v[k];
-            if (i < n) {
-                fill[i] = 0u;
-                atomicAdd(&bucket[size_class(v[k])], 1u);
-            }
-        }
+        if (threadIdx.x < kBinClasses)
+            lcls[threadIdx.x] = 0u;
+        if (threadIdx.x == 0)
+            lsum = 0u;
         __syncthreads();
-        uint32_t x[kScanPer], sum = 0;
+        const uint32_t split_max = split_cap ? bc.bin_cap : 0u;
+        uint32_t c[kOrderPer], pos[kOrderPer], sum = 0;
 #pragma unroll
-        for (uint32_t k = 0; k < kScanPer; ++k) {
-            x[k] = lc[tid * kScanPer + k];
-            sum += x[k];
+        for (uint32_t k = 0; k < kOrderPer; ++k) {
+            const uint32_t i = (threadIdx.x * kOrderPer + k) * norder + blockIdx.x;
+            const uint32_t m = i < n ? atomicOr(&bc.bin_count[bin0 + i], kBinSeen) : 0u;
+            sum += m;
+            c[k] = order_class(m, split_max);
         }
-        // inclusive scan inside the wave, then over the wave totals
-        uint32_t inc = sum;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            uint32_t o = __shfl_up(inc, d, 64);
-            if (lane >= (uint32_t)d)
-                inc += o;
-        }
-        if (lane == 63)
-            wsum[w] = inc;
-        const uint32_t base = carry;
-        __syncthreads();
-        if (w == 0) {
-            uint32_t y = lane < 16 ? wsum[lane] : 0u, z = y;
-#pragma unroll
-            for (int d = 1; d < 16; d <<= 1) {
-                uint32_t o = __shfl_up(z, d, 64);
-                if (lane >= (uint32_t)d)
-                    z += o;
-            }
-            if (lane < 16)
-                wsum[lane] = z - y; // exclusive prefix of the wave totals
-            if (lane == 15)
-                carry = base + z;
-        }
-        __syncthreads();
-        uint32_t run = base + wsum[w] + inc - sum;
-#pragma unroll
-        for (uint32_t k = 0; k < kScanPer; ++k) {
-            lc[tid * kScanPer + k] = run;
-            run += x[k];
-        }
-        __syncthreads();
-#pragma unroll
-        for (uint32_t k = 0; k < kScanPer; ++k) {
-            const uint32_t i = c0 + k * 1024u + tid;
-            if (i < n)
-                start[i] = lc[k * 1024u + tid];
-        }
-        __syncthreads(); // lc and wsum are reused by the next chunk
-    }
-    if (tid == 0) {
-        counters[kCntEntries] = carry;
-        uint32_t acc = 0;
-        for (int k = 32; k >= 0; --k) {
-            boff[k] = acc;
-            acc += bucket[k];
-        }
-    }
-    __syncthreads();
-    // Each thread ranks a contiguous run of bins, one at a time: consecutive
-    // launches of a class then come from bins about n / 1024 apart (tiles far
-    // apart on the hemicube).  That ran measurably faster in the tile kernel
-    // than neighbouring tiles launched together, and than batching the loads.
-    const uint32_t per = (n + blockDim.x - 1) / blockDim.x;
-    const uint32_t b0 = tid * per, b1 = min(n, b0 + per);
-    for (uint32_t i = b0; i < b1; ++i)
-        order[atomicAdd(&boff[size_class(cnt[i])], 1u)] = bin0 + i;
-}
-
-// Same grid as k_raster_setup: block (blk, s) puts the records of its region
-// into their bins, reserving each bin's range with one global atomic per
-// touched tile.  The extra column blk == nblk handles the spill region.
-__device__ static inline void unpack_bbox(uint64_t v, uint32_t tshift, uint32_t &g0,
-                                          uint32_t &g1, uint32_t &h0, uint32_t &h1)
-{
-    g0 = (uint32_t)(v & 0xFFFFu) >> tshift;
-    h0 = (uint32_t)((v >> 16) & 0xFFFFu) >> tshift;
-    g1 = (uint32_t)((v >> 32) & 0xFFFFu) >> tshift;
-    h1 = (uint32_t)(v >> 48) >> tshift;
-}
-
-// The spill records of shooter slots [s0, s1) into their tiles' lists: one
-// global atomic per entry (records go to the spill region only when a setup
-// block's region is full, which is rare).
-__device__ static void bin_spill(const RasterRec *__restrict__ recs,
-                                 const uint64_t *__restrict__ bbox,
-                                 const uint32_t *__restrict__ counters, uint32_t spill_base,
-                                 uint32_t spill_cap, const uint32_t *__restrict__ start,
-                                 uint32_t *__restrict__ fill, uint32_t *__restrict__ list,
-                                 uint32_t ent_cap, uint32_t ntx, uint32_t ntiles, uint32_t tshift,
-                                 uint32_t s0, uint32_t s1)
-{
-    const uint32_t nsp = min(counters[kCntSpill], spill_cap);
-    for (uint32_t s = s0; s < s1; ++s) {
-        uint32_t *fl = fill + (size_t)s * ntiles;
-        const uint32_t *stt = start + (size_t)s * ntiles;
-        for (uint32_t q = threadIdx.x; q < nsp; q += blockDim.x) {
-            const uint32_t r = spill_base + q;
-            if ((recs[r].sf >> 3) != s)
+        for (uint32_t k = 0; k < kOrderPer; ++k) {
+            const uint32_t i = (threadIdx.x * kOrderPer + k) * norder + blockIdx.x;
+            if (i >= n)
                 continue;
-            uint32_t g0, g1, h0, h1;
-            unpack_bbox(bbox[r], tshift, g0, g1, h0, h1);
-            for (uint32_t gy = h0; gy <= h1; ++gy)
-                for (uint32_t gx = g0; gx <= g1; ++gx) {
-                    const uint32_t b = gy * ntx + gx;
-                    const uint32_t pos = stt[b] + atomicAdd(&fl[b], 1u);
-                    if (pos < ent_cap)
-                        list[pos] = r;
-                }
+            if (c[k] == 0u) {
+                const uint32_t p0 = atomicAdd(&bc.counters[kCntClass], 1u);
+                if (p0 < split_cap)
+                    order[p0] = bin0 + i;
+                else
+                    c[k] = 1u; // beyond the quadrants the launch has room for
+            }
+            if (c[k])
+                pos[k] = atomicAdd(&lcls[c[k]], 1u);
         }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_bin_fill(const RasterRec *__restrict__ recs,
-                                                  const uint64_t *__restrict__ bbox,
-                                                  const uint32_t *__restrict__ blk_nrec,
-                                                  const uint32_t *__restrict__ counters,
-                                                  uint32_t nblk, uint32_t spill_base,
-                                                  uint32_t spill_cap,
-                                                  const uint32_t *__restrict__ start,
-                                                  uint32_t *__restrict__ fill,
-                                                  uint32_t *__restrict__ list, uint32_t ent_cap,
-                                                  uint32_t ntx, uint32_t ntiles, uint32_t tshift,
-                                                  const uint32_t *__restrict__ nshoot,
-                                                  uint32_t group, uint32_t slot0,
-                                                  uint32_t nslot)
-{
-    extern __shared__ uint32_t dyn_lds[];
-    uint32_t *lcnt = dyn_lds, *lbase = dyn_lds + ntiles; // dynamic LDS, 2 x ntiles
-    const uint32_t ns = *nshoot < nslot ? *nshoot : nslot;
-    if (blockIdx.x == nblk) {
-        if (blockIdx.z == 0)
-            bin_spill(recs, bbox, counters, spill_base, spill_cap, start, fill, list, ent_cap, ntx,
-                      ntiles, tshift, (slot0 + blockIdx.y * group), min(ns, (slot0 + blockIdx.y * group) + group));
+        atomicAdd(&lsum, sum);
+        __syncthreads();
+        if (threadIdx.x > 0 && threadIdx.x < kBinClasses && lcls[threadIdx.x])
+            gcls[threadIdx.x] =
+                atomicAdd(&bc.counters[kCntClass + threadIdx.x], lcls[threadIdx.x]);
+        if (threadIdx.x == 0 && lsum)
+            atomicAdd(&bc.counters[kCntEntries], lsum);
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < kOrderPer; ++k) {
+            const uint32_t i = (threadIdx.x * kOrderPer + k) * norder + blockIdx.x;
+            if (i < n && c[k])
+                order[(size_t)c[k] * qstride + gcls[c[k]] + pos[k]] = bin0 + i;
+        }
         return;
     }
-    // The workgroup walks `group` consecutive shooter slots, like the setup.
-    // Each lane holds the bboxes of its kFillPer region slots in registers;
-    // the next slot's count and bboxes are loaded while the current slot is
-    // binned, so a slot costs no load latency of its own.
-    constexpr uint32_t kFillPer = kRecsPerBlock / 256;
-    static_assert(kRecsPerBlock % 256 == 0, "k_bin_fill runs 256 threads per region");
-    uint64_t bv[kFillPer];
-    uint32_t nrec = 0;
-    auto prefetch = [&](uint32_t s) {
-        const uint32_t blk = (s * gridDim.z + blockIdx.z) * nblk + blockIdx.x;
-        nrec = blk_nrec[blk];
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    const uint32_t nj = min(bc.counters[kCntClip], bc.clip_cap);
+    for (uint32_t q = (blockIdx.x - norder) * 4u + wv; q < nj; q += (gridDim.x - norder) * 4u) {
+        const uint2 job = bc.clipq[q];
+        const uint32_t t = job.x, s = job.y >> 3;
+        const int face = (int)(job.y & 7u);
+        CV4 v;
 #pragma unroll
-        for (uint32_t k = 0; k < kFillPer; ++k) {
-            const uint32_t q = threadIdx.x + 256u * k;
-            bv[k] = q < nrec ? bbox[(size_t)blk * kRecsPerBlock + q] : 0ull;
+        for (int c = 0; c < 4; ++c)
+            v.c[c] = 0.0f;
+        if (lane < 3) {
+            const float x = tri[(size_t)(3 * lane + 0) * ntri + t];
+            const float y = tri[(size_t)(3 * lane + 1) * ntri + t];
+            const float z = tri[(size_t)(3 * lane + 2) * ntri + t];
+            const float *mm = mvp + (size_t)s * kShooterStride + face * 16;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                v.c[r] = mm[0 * 4 + r] * x + mm[1 * 4 + r] * y + mm[2 * 4 + r] * z + mm[3 * 4 + r];
         }
-    };
-    if ((slot0 + blockIdx.y * group) < ns)
-        prefetch((slot0 + blockIdx.y * group));
-    for (uint32_t g = 0; g < group; ++g) {
-        const uint32_t s = (slot0 + blockIdx.y * group) + g;
-        if (s >= ns)
-            break;
-        uint32_t *fl = fill + (size_t)s * ntiles;
-        const uint32_t *stt = start + (size_t)s * ntiles;
-        const uint32_t blk = (s * gridDim.z + blockIdx.z) * nblk + blockIdx.x;
-        const uint32_t region = blk * kRecsPerBlock, n = nrec;
-        uint64_t cur[kFillPer];
-#pragma unroll
-        for (uint32_t k = 0; k < kFillPer; ++k)
-            cur[k] = bv[k];
-        if (g + 1 < group && s + 1 < ns)
-            prefetch(s + 1);
-        if (n == 0)
-            continue;
-        __syncthreads(); // the previous slot is done with lcnt / lbase
-        for (uint32_t i = threadIdx.x; i < ntiles; i += blockDim.x)
-            lcnt[i] = 0u;
-        __syncthreads();
-#pragma unroll
-        for (uint32_t k = 0; k < kFillPer; ++k) {
-            if (threadIdx.x + 256u * k >= n)
-                break;
-            uint32_t g0, g1, h0, h1;
-            unpack_bbox(cur[k], tshift, g0, g1, h0, h1);
-            for (uint32_t gy = h0; gy <= h1; ++gy)
-                for (uint32_t gx = g0; gx <= g1; ++gx)
-                    atomicAdd(&lcnt[gy * ntx + gx], 1u);
-        }
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < ntiles; i += blockDim.x) {
-            uint32_t c = lcnt[i];
-            lbase[i] = c ? stt[i] + atomicAdd(&fl[i], c) : 0u;
-            lcnt[i] = 0u;
-        }
-        __syncthreads();
-#pragma unroll
-        for (uint32_t k = 0; k < kFillPer; ++k) {
-            const uint32_t q = threadIdx.x + 256u * k;
-            if (q >= n)
-                break;
-            uint32_t g0, g1, h0, h1;
-            unpack_bbox(cur[k], tshift, g0, g1, h0, h1);
-            for (uint32_t gy = h0; gy <= h1; ++gy)
-                for (uint32_t gx = g0; gx <= g1; ++gx) {
-                    uint32_t b = gy * ntx + gx;
-                    uint32_t pos = lbase[b] + atomicAdd(&lcnt[b], 1u);
-                    if (pos < ent_cap)
-                        list[pos] = region + q;
+        const uint32_t Ws = slot_w ? slot_w[s] : W;
+        FaceView fv = face_view((int32_t)Ws, face);
+        const int np = clip_polygon_wave(v, lp[wv], &bc.counters[kCntOverflow]);
+        SV a, b, cc;
+        Placed p;
+        bool have = false;
+        if (np >= 3 && clip_fan(v, np, 0.5f * (float)Ws, a, b, cc))
+            have = place_tri(a, b, cc, tri_patch[t] + 1u, fv, s, face, bc, p) != 0;
+        // the records' tiles, flattened over the lanes: a list place is a
+        // returning atomic, so one lane walking a large record's tiles would
+        // wait for each
+        const uint64_t em = __ballot(have);
+        for (uint32_t base = 0, total = 64u; base < total; base += 64u) {
+            total = 0;
+            uint32_t r = 0, tile = ~0u;
+            for (uint64_t m = em; m; m &= m - 1) {
+                const int l = __ffsll((long long)m) - 1;
+                auto at = [&](uint32_t x) {
+                    return (uint32_t)__builtin_amdgcn_readlane((int)x, l);
+                };
+                const uint32_t g0 = at(p.g0), nx = at(p.g1) - g0 + 1u;
+                const uint32_t h0 = at(p.h0), ny = at(p.h1) - h0 + 1u;
+                const uint32_t i = base + lane - total;
+                if (base + lane >= total && i < nx * ny) {
+                    r = at(p.r);
+                    tile = (h0 + i / nx) * bc.ntx + g0 + i % nx;
                 }
+                total += nx * ny;
+            }
+            if (tile != ~0u)
+                bin_spilled(bc, s, tile, r);
         }
+        wave_lds_sync(); // lp is the next job's
     }
 }
 
@@ -1004,17 +928,63 @@ __global__ __launch_bounds__(256) void k_bin_fill(const RasterRec *__restrict__ 
 // plane) or is reduced into F rows and hit counts (ff or, in the
 // deterministic mode, its fixed-point rows ffq != null).
 
+// read by scalar loads: nothing writes it during the launch
+using ConstFacts = const __attribute__((address_space(4))) BinFacts *;
+
+// The list of a bin fuller than its list has room for: the workgroup goes
+// over all records of the slot, the regions and the spill region, and writes
+// those that touch the tile at (ox, oy) into the pool, where it reserves the
+// bin's n entries.  *cnt (LDS): how many.
+__device__ static const uint32_t *whole_list(ConstFacts f,
+                                             const RasterRec *__restrict__ recs,
+                                             const uint64_t *__restrict__ bbox, uint32_t s,
+                                             uint32_t n, int32_t ox, int32_t oy, int32_t T,
+                                             uint32_t *cnt, uint32_t *at)
+{
+    const uint32_t me = threadIdx.x;
+    if (me == 0) {
+        *cnt = 0u;
+        *at = atomicAdd(f->pool_used, n);
+    }
+    __syncthreads();
+    const uint32_t used = __builtin_amdgcn_readfirstlane(*at);
+    const uint32_t cap = f->pool_cap, room = cap - min(used, cap);
+    uint32_t *const out = f->pool + (cap - room);
+    auto take = [&](uint32_t r) {
+        const uint64_t v = bbox[r];
+        if ((int32_t)(v & 0xFFFFu) < ox + T && (int32_t)((v >> 16) & 0xFFFFu) < oy + T &&
+            (int32_t)((v >> 32) & 0xFFFFu) >= ox && (int32_t)(v >> 48) >= oy) {
+            const uint32_t q = atomicAdd(cnt, 1u);
+            if (q < room) // always, unless the pass has more entries than it may
+                out[q] = r;
+        }
+    };
+    for (uint32_t b = me >> 6; b < f->nreg; b += kTileThreads / 64u) {
+        const uint32_t reg = s * f->nreg + b, k = f->blk_nrec[reg];
+        for (uint32_t q = me & 63u; q < k; q += 64u)
+            take(reg * kRecsPerBlock + q);
+    }
+    const uint32_t nsp = min((uint32_t)f->nspill, (uint32_t)f->spill_cap);
+    for (uint32_t q = me; q < nsp; q += kTileThreads)
+        if ((recs[f->spill_base + q].sf >> 3) == s)
+            take(f->spill_base + q);
+    __syncthreads();
+    if (me == 0)
+        *cnt = min(*cnt, room);
+    __syncthreads();
+    return out;
+}
+
 template <bool FQ>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_tile_raster(
     uint32_t W, uint32_t TW, uint32_t TH, uint32_t RES, const uint32_t *__restrict__ nshoot,
     const RasterRec *__restrict__ recs, const uint64_t *__restrict__ bbox,
-    const uint32_t *__restrict__ bin_count, const uint32_t *__restrict__ bin_start,
-    const uint32_t *__restrict__ list, uint32_t ent_cap, uint32_t ntx, uint32_t ntiles,
-    uint32_t tshift, uint32_t small_px, uint32_t *__restrict__ out_ids,
+    const uint32_t *__restrict__ bin_count, const uint32_t *__restrict__ list, uint32_t bin_cap,
+    const BinFacts *__restrict__ facts, uint32_t ntx, uint32_t ntiles, uint32_t tshift, uint32_t small_px, uint32_t *__restrict__ out_ids,
     float *__restrict__ out_depth, const float *__restrict__ dff,
     uint32_t rowlen, const uint32_t *__restrict__ slot_pbeg, float *__restrict__ ff,
     unsigned long long *__restrict__ ffq, uint32_t *__restrict__ hits,
-    uint32_t *__restrict__ counters, const uint32_t *__restrict__ order,
+    uint32_t *__restrict__ counters, const uint32_t *__restrict__ order, uint32_t qstride,
     const uint32_t *__restrict__ slot_w, const uint32_t *__restrict__ slot_dffo,
     uint32_t *__restrict__ fblk, uint32_t fstride)
 {
@@ -1034,12 +1004,30 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
     uint32_t *const perm = sh.q.perm;
     uint64_t *const pbb = sh.q.pbb;
     __shared__ uint32_t nbig;
-    const uint32_t bin = order[blockIdx.x];
+    // the workgroup's bin: first the quadrants of the largest (class 0), then
+    // the other classes' queues
+    uint32_t bin, quad = 4u;
+    {
+        const auto cls = ((ConstFacts)facts)->cls;
+        const uint32_t n0 = min((uint32_t)cls[0], (uint32_t)((ConstFacts)facts)->split_cap);
+        uint32_t b = blockIdx.x, c = 0;
+        if (b < 4u * n0) {
+            quad = b & 3u;
+            b >>= 2;
+        } else {
+            b -= 4u * n0;
+            for (c = 1; c < kBinClasses && b >= cls[c]; ++c)
+                b -= cls[c];
+            if (c == kBinClasses)
+                return;
+        }
+        bin = order[(size_t)c * qstride + b];
+    }
     const uint32_t s = bin / ntiles;
     if (s >= *nshoot)
         return;
     const uint32_t tile = bin - s * ntiles;
-    const uint32_t n = bin_count[bin], st0 = bin_start[bin];
+    const uint32_t n = bin_count[bin] & ~kBinSeen;
     // an empty bin adds nothing to the F rows (its texels are background)
     if (n == 0 && !out_ids)
         return;
@@ -1051,40 +1039,59 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
         TH = W + W / 2;
         dff += slot_dffo[s];
     }
+    int32_t ox = (int32_t)((tile % ntx) << tshift), oy = (int32_t)((tile / ntx) << tshift);
+    if (quad < 4u && n > bin_cap) {
+        // the clipped triangles overfilled it since: drawn whole
+        if (quad)
+            return;
+        quad = 4u;
+    }
+    if (quad < 4u) { // a quadrant: a tile of half the side over the same list
+        tshift -= 1;
+        ox += (int32_t)((quad & 1u) << tshift);
+        oy += (int32_t)((quad >> 1) << tshift);
+    }
     const uint32_t T = 1u << tshift, TT = T * T;
-    const int32_t ox = (int32_t)((tile % ntx) << tshift), oy = (int32_t)((tile / ntx) << tshift);
     const int32_t Wi = (int32_t)W;
     const uint32_t me = threadIdx.x;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(me >> 6);
     constexpr uint32_t kNoRec = ~0u;
+    const uint32_t *lst = list + (size_t)bin * bin_cap;
+    uint32_t nl = n;
+    if (__builtin_expect(n > bin_cap, 0)) {
+        lst = whole_list((ConstFacts)facts, recs, bbox, s, n, ox, oy, (int32_t)T, &nbig, perm);
+        nl = __builtin_amdgcn_readfirstlane(nbig);
+        __syncthreads();
+    }
     // Lane me's record of the chunk starting at entry cb.  A chunk of m <
     // 256 records would leave waves idle: its records are dealt to
     // ceil(m / 64) wave sets (one per lane), and the nph = 4 / sets waves of a
     // set each draw row phase ph of its in-lane records (every nph-th bbox
     // row); a full chunk keeps one record per lane, nph = 1.
     auto deal = [&](uint32_t cb, uint32_t &ph, uint32_t &nph) -> uint32_t {
-        const uint32_t m = min(kTileThreads, n - cb);
+        const uint32_t m = min(kTileThreads, nl - cb);
         const uint32_t sets = (m + 63u) >> 6;
         nph = sets >= 3u ? 1u : 4u / sets;
         ph = wv / sets;
         const uint32_t k = (wv - ph * sets) * 64u + (me & 63u);
-        return ph < nph && k < m && st0 + cb + k < ent_cap ? list[st0 + cb + k] : kNoRec;
+        return ph < nph && k < m ? lst[cb + k] : kNoRec;
     };
+
     // A lane's entry of the first chunk (list index and bbox) is fetched
     // while the tile clears; each later chunk's list entries are fetched
     // during the chunk before it.
     uint32_t ph = 0, nph = 1;
-    uint32_t ri = n ? deal(0u, ph, nph) : kNoRec;
+    uint32_t ri = nl ? deal(0u, ph, nph) : kNoRec;
     uint64_t bv = 0;
     if (ri != kNoRec)
         bv = bbox[ri];
     for (uint32_t p = threadIdx.x; p < TT; p += blockDim.x)
         tk[p] = kClearKey;
-    for (uint32_t c0 = 0; c0 < n; c0 += blockDim.x) {
+    for (uint32_t c0 = 0; c0 < nl; c0 += blockDim.x) {
         if (me == 0)
             nbig = 0u;
         uint32_t ph_n = 0, nph_n = 1;
-        const uint32_t rnext = c0 + blockDim.x < n ? deal(c0 + blockDim.x, ph_n, nph_n) : kNoRec;
+        const uint32_t rnext = c0 + blockDim.x < nl ? deal(c0 + blockDim.x, ph_n, nph_n) : kNoRec;
         __syncthreads();
         if (ri != kNoRec) {
             const int32_t ax0 = max((int32_t)(bv & 0xFFFFu), ox);
@@ -1092,7 +1099,9 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
             const int32_t ax1 = min((int32_t)((bv >> 32) & 0xFFFFu), ox + (int32_t)T - 1);
             const int32_t ay1 = min((int32_t)(bv >> 48), oy + (int32_t)T - 1);
             const uint32_t area = (uint32_t)(ax1 - ax0 + 1) * (uint32_t)(ay1 - ay0 + 1);
-            if (area <= small_px) {
+            if (ax1 < ax0 || ay1 < ay0) {
+                // touches other quadrants only
+            } else if (area <= small_px) {
                 const RasterRec r = recs[ri];
                 FaceView fv = face_view(Wi, (int)(r.sf & 7u));
                 draw_lane(r, fv.vpx, fv.vpy, ax0, ax1, ay0, ay1, ox, oy, tshift, tk, ph, nph);
@@ -1223,277 +1232,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
     }
 }
 
-// k_bin_fill for up to 256 * RPT tiles, software-pipelined over the
-// workgroup's shooter slots: the list space of slot g is reserved (one
-// returning global atomic per touched tile) and, while those atomics are in
-// flight, the records of the previous slot are placed; two LDS sets of
-// counts and bases alternate between the slots.  Slots without records are
-// skipped.  The placement is k_bin_fill's: a record's entries go to its
-// tiles' lists at base + rank, rank from an LDS atomic in lane order.
-template <int RPT>
-__global__ __launch_bounds__(256) void k_bin_fill_pipe(const RasterRec *__restrict__ recs,
-                                                       const uint64_t *__restrict__ bbox,
-                                                       const uint32_t *__restrict__ blk_nrec,
-                                                       const uint32_t *__restrict__ counters,
-                                                       uint32_t nblk, uint32_t spill_base,
-                                                       uint32_t spill_cap,
-                                                       const uint32_t *__restrict__ start,
-                                                       uint32_t *__restrict__ fill,
-                                                       uint32_t *__restrict__ list,
-                                                       uint32_t ent_cap, uint32_t ntx,
-                                                       uint32_t ntiles, uint32_t tshift,
-                                                       const uint32_t *__restrict__ nshoot,
-                                                       uint32_t group, uint32_t slot0,
-                                                       uint32_t nslot)
-{
-    extern __shared__ uint32_t dyn_lds[]; // 4 x ntiles: counts and bases, twice
-    constexpr uint32_t kFillPer = kRecsPerBlock / 256;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t ns = *nshoot < nslot ? *nshoot : nslot;
-    const uint32_t sbeg = slot0 + blockIdx.y * group, send = min(ns, sbeg + group);
-    if (blockIdx.x == nblk) { // the last column: the spill records
-        if (blockIdx.z == 0)
-            bin_spill(recs, bbox, counters, spill_base, spill_cap, start, fill, list, ent_cap, ntx,
-                      ntiles, tshift, sbeg, send);
-        return;
-    }
-    auto blk_of = [&](uint32_t sl) { return (sl * gridDim.z + blockIdx.z) * nblk + blockIdx.x; };
-    uint64_t bv[kFillPer];
-    uint32_t nrec = 0;
-    auto prefetch = [&](uint32_t sl) {
-        const uint32_t blk = blk_of(sl);
-        nrec = blk_nrec[blk];
-#pragma unroll
-        for (uint32_t k = 0; k < kFillPer; ++k) {
-            const uint32_t q = tid + 256u * k;
-            bv[k] = q < nrec ? bbox[(size_t)blk * kRecsPerBlock + q] : 0ull;
-        }
-    };
-    // the records of one slot into the lists (bases lb, ranks from lc)
-    auto place = [&](const uint64_t (&v)[kFillPer], uint32_t n, uint32_t region, uint32_t *lc,
-                     const uint32_t *lb) {
-#pragma unroll
-        for (uint32_t k = 0; k < kFillPer; ++k) {
-            const uint32_t q = tid + 256u * k;
-            if (q >= n)
-                break;
-            uint32_t g0, g1, h0, h1;
-            unpack_bbox(v[k], tshift, g0, g1, h0, h1);
-            for (uint32_t gy = h0; gy <= h1; ++gy)
-                for (uint32_t gx = g0; gx <= g1; ++gx) {
-                    const uint32_t b = gy * ntx + gx;
-                    const uint32_t pos = lb[b] + atomicAdd(&lc[b], 1u);
-                    if (pos < ent_cap)
-                        list[pos] = region + q;
-                }
-        }
-    };
-    uint64_t pv[kFillPer];
-    uint32_t pn = 0, pregion = 0, it = 0;
-    if (sbeg < send)
-        prefetch(sbeg);
-    for (uint32_t sl = sbeg; sl < send; ++sl) {
-        const uint32_t n = nrec, region = blk_of(sl) * kRecsPerBlock;
-        uint64_t cur[kFillPer];
-#pragma unroll
-        for (uint32_t k = 0; k < kFillPer; ++k)
-            cur[k] = bv[k];
-        if (sl + 1 < send)
-            prefetch(sl + 1);
-        if (n == 0)
-            continue;
-        uint32_t *lc = dyn_lds + (it & 1u) * 2u * ntiles, *lb = lc + ntiles;
-        uint32_t *pc = dyn_lds + ((it & 1u) ^ 1u) * 2u * ntiles, *pb = pc + ntiles;
-        __syncthreads(); // the slot two back is placed; the previous slot's bases are written
-        for (uint32_t i = tid; i < ntiles; i += 256u)
-            lc[i] = 0u;
-        __syncthreads();
-#pragma unroll
-        for (uint32_t k = 0; k < kFillPer; ++k) {
-            if (tid + 256u * k >= n)
-                break;
-            uint32_t g0, g1, h0, h1;
-            unpack_bbox(cur[k], tshift, g0, g1, h0, h1);
-            for (uint32_t gy = h0; gy <= h1; ++gy)
-                for (uint32_t gx = g0; gx <= g1; ++gx)
-                    atomicAdd(&lc[gy * ntx + gx], 1u);
-        }
-        __syncthreads();
-        // reserve this slot's list space ...
-        uint32_t *fl = fill + (size_t)sl * ntiles;
-        const uint32_t *stt = start + (size_t)sl * ntiles;
-        uint32_t rb[RPT];
-#pragma unroll
-        for (int r = 0; r < RPT; ++r) {
-            const uint32_t i = tid + 256u * (uint32_t)r;
-            const uint32_t c = i < ntiles ? lc[i] : 0u;
-            rb[r] = c ? stt[i] + atomicAdd(&fl[i], c) : 0u;
-            if (i < ntiles)
-                lc[i] = 0u;
-        }
-        // ... while the previous slot's records are placed
-        if (it)
-            place(pv, pn, pregion, pc, pb);
-#pragma unroll
-        for (int r = 0; r < RPT; ++r) {
-            const uint32_t i = tid + 256u * (uint32_t)r;
-            if (i < ntiles)
-                lb[i] = rb[r];
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < kFillPer; ++k)
-            pv[k] = cur[k];
-        pn = n;
-        pregion = region;
-        ++it;
-    }
-    if (it) {
-        __syncthreads();
-        uint32_t *lc = dyn_lds + ((it - 1u) & 1u) * 2u * ntiles;
-        place(pv, pn, pregion, lc, lc + ntiles);
-    }
-}
-
-// k_bin_fill for up to 256 tiles per hemicube, all of a workgroup's shooter
-// slots (at most 8) at once: the region records of every slot are counted
-// per (slot, tile) in LDS, one returning global atomic per touched (slot,
-// tile) reserves the list space (all of a thread's issued before any is
-// used), and the records are placed.  Three barriers and one atomic round
-// trip per workgroup, where walking the slots one by one takes one round
-// trip per slot.  A thread keeps the bboxes of its first kFillKeep records
-// in registers for the placement and loads the others again.
-constexpr uint32_t kFillSlots = 8, kFillTiles = 256, kFillKeep = 4;
-
-__global__ __launch_bounds__(256) void k_bin_fill_all(const RasterRec *__restrict__ recs,
-                                                      const uint64_t *__restrict__ bbox,
-                                                      const uint32_t *__restrict__ blk_nrec,
-                                                      const uint32_t *__restrict__ counters,
-                                                      uint32_t nblk, uint32_t spill_base,
-                                                      uint32_t spill_cap,
-                                                      const uint32_t *__restrict__ start,
-                                                      uint32_t *__restrict__ fill,
-                                                      uint32_t *__restrict__ list,
-                                                      uint32_t ent_cap, uint32_t ntx,
-                                                      uint32_t ntiles, uint32_t tshift,
-                                                      const uint32_t *__restrict__ nshoot,
-                                                      uint32_t group, uint32_t slot0,
-                                                      uint32_t nslot)
-{
-    __shared__ uint32_t lc[kFillSlots * kFillTiles], lb[kFillSlots * kFillTiles];
-    __shared__ uint32_t off[kFillSlots + 1];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t ns = *nshoot < nslot ? *nshoot : nslot;
-    const uint32_t sbeg = slot0 + blockIdx.y * group, send = min(ns, sbeg + group);
-    if (blockIdx.x == nblk) { // the last column: the spill records
-        if (blockIdx.z == 0)
-            bin_spill(recs, bbox, counters, spill_base, spill_cap, start, fill, list, ent_cap, ntx,
-                      ntiles, tshift, sbeg, send);
-        return;
-    }
-    if (sbeg >= send)
-        return;
-    const uint32_t nsl = send - sbeg;
-    auto region = [&](uint32_t sl) {
-        return ((sbeg + sl) * gridDim.z + blockIdx.z) * nblk + blockIdx.x;
-    };
-    if (tid < 64) {
-        // the slots' record counts and their running offsets
-        const uint32_t c = tid < nsl ? blk_nrec[region(tid)] : 0u;
-        uint32_t inc = c;
-#pragma unroll
-        for (int d = 1; d < (int)kFillSlots; d <<= 1) {
-            const uint32_t o = __shfl_up(inc, d, 64);
-            if ((int)tid >= d)
-                inc += o;
-        }
-        if (tid < kFillSlots)
-            off[tid + 1] = inc;
-        if (tid == 0)
-            off[0] = 0u;
-    }
-    for (uint32_t i = tid; i < nsl * ntiles; i += 256u)
-        lc[i] = 0u;
-    __syncthreads();
-    const uint32_t total = off[nsl];
-    // record f of the workgroup: slot sl (off[sl] <= f < off[sl + 1]) and
-    // its index q in the slot's region
-    auto locate = [&](uint32_t f, uint32_t &sl, uint32_t &q) {
-        sl = 0;
-        while (sl + 1 < nsl && f >= off[sl + 1])
-            ++sl;
-        q = f - off[sl];
-    };
-    uint64_t keep[kFillKeep];
-#pragma unroll
-    for (uint32_t k = 0; k < kFillKeep; ++k)
-        keep[k] = 0ull;
-    uint32_t k = 0;
-    for (uint32_t f = tid; f < total; f += 256u, ++k) {
-        uint32_t sl, q;
-        locate(f, sl, q);
-        const uint64_t v = bbox[(size_t)region(sl) * kRecsPerBlock + q];
-#pragma unroll
-        for (uint32_t j = 0; j < kFillKeep; ++j)
-            if (j == k)
-                keep[j] = v;
-        uint32_t g0, g1, h0, h1;
-        unpack_bbox(v, tshift, g0, g1, h0, h1);
-        for (uint32_t gy = h0; gy <= h1; ++gy)
-            for (uint32_t gx = g0; gx <= g1; ++gx)
-                atomicAdd(&lc[sl * ntiles + gy * ntx + gx], 1u);
-    }
-    __syncthreads();
-    // reserve: every count of this thread goes out before any result is used
-    constexpr uint32_t kPer = kFillSlots * kFillTiles / 256u;
-    uint32_t rb[kPer], st[kPer];
-#pragma unroll
-    for (uint32_t r = 0; r < kPer; ++r) {
-        const uint32_t i = tid + 256u * r;
-        const uint32_t c = i < nsl * ntiles ? lc[i] : 0u;
-        const uint32_t bin = sbeg * ntiles + i;
-        rb[r] = c ? atomicAdd(&fill[bin], c) : 0u;
-        st[r] = c ? start[bin] : 0u;
-    }
-#pragma unroll
-    for (uint32_t r = 0; r < kPer; ++r) {
-        const uint32_t i = tid + 256u * r;
-        if (i < nsl * ntiles) {
-            lb[i] = st[r] + rb[r];
-            lc[i] = 0u;
-        }
-    }
-    __syncthreads();
-    k = 0;
-    for (uint32_t f = tid; f < total; f += 256u, ++k) {
-        uint32_t sl, q;
-        locate(f, sl, q);
-        const uint32_t rr = region(sl) * kRecsPerBlock + q;
-        uint64_t v = 0ull;
-        if (k < kFillKeep) {
-#pragma unroll
-            for (uint32_t j = 0; j < kFillKeep; ++j)
-                if (j == k)
-                    v = keep[j];
-        } else {
-            v = bbox[rr];
-        }
-        uint32_t g0, g1, h0, h1;
-        unpack_bbox(v, tshift, g0, g1, h0, h1);
-        for (uint32_t gy = h0; gy <= h1; ++gy)
-            for (uint32_t gx = g0; gx <= g1; ++gx) {
-                const uint32_t b = sl * ntiles + gy * ntx + gx;
-                const uint32_t pos = lb[b] + atomicAdd(&lc[b], 1u);
-                if (pos < ent_cap)
-                    list[pos] = rr;
-            }
-    }
-}
-
-void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h,
-                         const float *tri, const float4 *tsph, const uint32_t *tri_patch,
-                         uint32_t ntri, const float *mvp, const uint32_t *nshoot,
-                         const BinBuffers &bb, uint32_t *counters, const uint32_t *slot_tbeg,
-                         const uint32_t *slot_tcnt, const uint32_t *slot_w, hipStream_t st)
+static BinCtx bin_ctx(const BinBuffers &bb, uint32_t h, uint32_t *counters)
 {
     BinCtx bc;
     bc.recs = bb.recs;
@@ -1510,49 +1249,52 @@ void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h
     bc.ntx = bb.ntx;
     bc.ntiles = bb.ntiles;
     bc.tshift = bb.tshift;
+    bc.list = bb.list;
+    bc.bin_cap = bb.bin_cap;
+    return bc;
+}
+
+void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h,
+                         const float *tri, const float4 *tsph, const uint32_t *tri_patch,
+                         uint32_t ntri, const float *mvp, const uint32_t *nshoot,
+                         const BinBuffers &bb, uint32_t *counters, const uint32_t *slot_tbeg,
+                         const uint32_t *slot_tcnt, const uint32_t *slot_w, hipStream_t st)
+{
     const uint32_t n = s1 - s0;
     uint32_t group = bb.setup_group ? bb.setup_group : 1u;
     if (group > n)
         group = n;
     dim3 grid(bb.nblk, (n + group - 1) / group, bb.nz);
     k_raster_setup<<<grid, 256, 4 * bb.ntiles * sizeof(uint32_t), st>>>(
-        g.W, tri, tsph, tri_patch, ntri, mvp, nshoot, bc, bb.blk_nrec, slot_tbeg, slot_tcnt,
-        slot_w, group, s0, s1);
-    bc.lnrec = nullptr;
-    k_setup_clipped<<<bb.clip_blocks, 64, 0, st>>>(g.W, tri, tri_patch, ntri, mvp, bc, slot_w);
+        g.W, tri, tsph, tri_patch, ntri, mvp, nshoot, bin_ctx(bb, h, counters), bb.blk_nrec,
+        slot_tbeg, slot_tcnt, slot_w, group, s0, s1);
 }
 
-void launch_bin(uint32_t s0, uint32_t s1, uint32_t h, const uint32_t *nshoot,
-                const BinBuffers &bb, uint32_t *counters, hipStream_t st)
+// How many of a launch's nb bins may be drawn as quadrants, those of
+// kSplitRecs records or more: a launch whose bins are all resident at once, or
+// nearly, lasts as long as its fullest bin.  A pass of 64 shooters over 33,000
+// triangles at hemicube 128 (3,072 bins) takes 85.1 us instead of 88.4 and one
+// of 32 over 20,000, deterministic (1,536 bins), 109 instead of 114.  With
+// several times more bins (12,288: 64 shooters at hemicube 256) the largest,
+// started first, end before the others do, and with one hemicube (192) the
+// quadrants' reading of the whole list cost 1 %.  From 1,024 records on, or
+// for more than 1 bin in 16, a pass of 25 shooters over 16,000 triangles lost
+// up to 1 %.
+static uint32_t split_cap(const BinBuffers &bb, uint32_t nb)
 {
-    const uint32_t n = s1 - s0, b0 = s0 * bb.ntiles, nb = n * bb.ntiles;
-    uint32_t *ctr = counters + h * kCntN, *list = bb.list + (size_t)h * bb.ent_cap;
-    const uint32_t spill_base = bb.spill_base + h * bb.spill_cap;
-    k_bin_scan<<<1, 1024, 0, st>>>(bb.count + b0, bb.start + b0, bb.fill + b0, nb, ctr,
-                                   bb.order + b0, b0);
-    uint32_t group = bb.setup_group ? bb.setup_group : 1u;
-    if (group > n)
-        group = n;
-    dim3 grid(bb.nblk + 1, (n + group - 1) / group, bb.nz);
-    if (bb.ntiles > 1024) {
-        k_bin_fill<<<grid, 256, 2 * bb.ntiles * sizeof(uint32_t), st>>>(
-            bb.recs, bb.bbox, bb.blk_nrec, ctr, bb.nblk, spill_base, bb.spill_cap, bb.start,
-            bb.fill, list, bb.ent_cap, bb.ntx, bb.ntiles, bb.tshift, nshoot, group, s0, s1);
-        return;
-    }
-    const size_t lds = 4 * bb.ntiles * sizeof(uint32_t);
-    if (bb.ntiles <= kFillTiles && group <= kFillSlots)
-        k_bin_fill_all<<<grid, 256, 0, st>>>(
-            bb.recs, bb.bbox, bb.blk_nrec, ctr, bb.nblk, spill_base, bb.spill_cap, bb.start,
-            bb.fill, list, bb.ent_cap, bb.ntx, bb.ntiles, bb.tshift, nshoot, group, s0, s1);
-    else if (bb.ntiles <= 256)
-        k_bin_fill_pipe<1><<<grid, 256, lds, st>>>(
-            bb.recs, bb.bbox, bb.blk_nrec, ctr, bb.nblk, spill_base, bb.spill_cap, bb.start,
-            bb.fill, list, bb.ent_cap, bb.ntx, bb.ntiles, bb.tshift, nshoot, group, s0, s1);
-    else
-        k_bin_fill_pipe<4><<<grid, 256, lds, st>>>(
-            bb.recs, bb.bbox, bb.blk_nrec, ctr, bb.nblk, spill_base, bb.spill_cap, bb.start,
-            bb.fill, list, bb.ent_cap, bb.ntx, bb.ntiles, bb.tshift, nshoot, group, s0, s1);
+    return bb.tshift == 5 && nb > 512u && nb <= 4096u ? nb / 16u : 0u;
+}
+
+void launch_bin(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const float *tri,
+                const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const BinBuffers &bb,
+                uint32_t *counters, const uint32_t *slot_w, hipStream_t st)
+{
+    const uint32_t b0 = s0 * bb.ntiles, nb = (s1 - s0) * bb.ntiles;
+    const uint32_t norder = (nb + 256u * kOrderPer - 1) / (256u * kOrderPer);
+    k_order_clip<<<norder + bb.clip_blocks, 256, 0, st>>>(
+        norder, nb, b0, split_cap(bb, nb), bb.order + b0, bb.nbins, g.W, tri, tri_patch, ntri, mvp,
+        bin_ctx(bb, h, counters), bb.blk_nrec, bb.nblk * bb.nz,
+        bb.pool + (size_t)h * bb.ent_cap, bb.ent_cap, slot_w);
 }
 
 void launch_tile(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const uint32_t *nshoot,
@@ -1564,19 +1306,19 @@ void launch_tile(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const 
 {
     const uint32_t nb = (s1 - s0) * bb.ntiles;
     const uint32_t *order = bb.order + (size_t)s0 * bb.ntiles;
-    const uint32_t *list = bb.list + (size_t)h * bb.ent_cap;
+    const uint32_t nwg = nb + 3u * split_cap(bb, nb);
     uint32_t *ctr = counters + h * kCntN;
+    const BinFacts *facts = reinterpret_cast<const BinFacts *>(ctr + kCntFacts);
     if (ffq)
-        k_tile_raster<true><<<nb, kTileThreads, 0, st>>>(
-            g.W, g.TW, g.TH, g.RES, nshoot, bb.recs, bb.bbox, bb.count, bb.start, list,
-            bb.ent_cap, bb.ntx, bb.ntiles, bb.tshift, small_px, out_ids, out_depth, dff, rowlen,
-            slot_pbeg, ff, ffq, hits, ctr, order, slot_w, slot_dffo, nullptr, 0u);
+        k_tile_raster<true><<<nwg, kTileThreads, 0, st>>>(
+            g.W, g.TW, g.TH, g.RES, nshoot, bb.recs, bb.bbox, bb.count, bb.list, bb.bin_cap, facts,
+            bb.ntx, bb.ntiles, bb.tshift, small_px, out_ids, out_depth, dff, rowlen, slot_pbeg, ff,
+            ffq, hits, ctr, order, bb.nbins, slot_w, slot_dffo, nullptr, 0u);
     else
-        k_tile_raster<false><<<nb, kTileThreads, 0, st>>>(
-            g.W, g.TW, g.TH, g.RES, nshoot, bb.recs, bb.bbox, bb.count, bb.start, list,
-            bb.ent_cap, bb.ntx, bb.ntiles, bb.tshift, small_px, out_ids, out_depth, dff, rowlen,
-            slot_pbeg, ff, ffq, hits, ctr, order, slot_w, slot_dffo, ff ? fblk : nullptr,
-            fstride);
+        k_tile_raster<false><<<nwg, kTileThreads, 0, st>>>(
+            g.W, g.TW, g.TH, g.RES, nshoot, bb.recs, bb.bbox, bb.count, bb.list, bb.bin_cap, facts,
+            bb.ntx, bb.ntiles, bb.tshift, small_px, out_ids, out_depth, dff, rowlen, slot_pbeg, ff,
+            ffq, hits, ctr, order, bb.nbins, slot_w, slot_dffo, ff ? fblk : nullptr, fstride);
 }
 
 // Deterministic mode: n fixed-point entries (units of 2^-52) into the float

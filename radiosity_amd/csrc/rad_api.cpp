@@ -166,7 +166,7 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
     // block h on stream st
     auto stage = [&](int j, uint32_t s0, uint32_t s1, uint32_t h, hipStream_t st) {
         if (j == 0)
-            launch_raster_setup(c->g, s0, s1, h, c->tri, c->tsph, c->tri_patch, c->ntri, c->mvp,
+            launch_raster_setup(c->g, s0, s1, h, c->tri, c->tsph, c->tback, c->tri_patch, c->ntri, c->mvp,
                                 c->nshoot, c->bb, c->counters, c->pk.slot_tbeg,
                                 c->pk.slot_tcnt, c->pk.slot_w, st);
         else if (j == 1)
@@ -527,7 +527,7 @@ void rad_destroy(rad_ctx *c)
         (void)hipStreamSynchronize(c->st2);
     drop_graph(c);
     gather_free(c);
-    void *ptrs[] = {c->tri,  c->tri_patch, c->tsph, c->clu, c->frames, c->refl,     c->area,   c->emis,
+    void *ptrs[] = {c->tri,  c->tri_patch, c->tsph, c->tback, c->clu, c->frames, c->refl,     c->area,   c->emis,
                     c->unshot, c->shot,   c->ff,  c->fblk,   c->hits,     c->dff,    c->item_ids,
                     c->item_depth, c->ffq, c->runs_slots, c->runs_offs, c->trip_h, c->trip_i,
                     c->trip_e,
@@ -633,7 +633,7 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     int rc;
     size_t K = c->K;
     if ((rc = dalloc(c, &c->tri, (size_t)ntri * 9)) || (rc = dalloc(c, &c->tri_patch, ntri)) ||
-        (rc = dalloc(c, &c->tsph, ntri)) ||
+        (rc = dalloc(c, &c->tsph, ntri)) || (rc = dalloc(c, &c->tback, ntri)) ||
         (rc = dalloc(c, &c->clu, cluster_words(ntri, 0))) ||
         (rc = dalloc(c, &c->frames, (size_t)npatch * 9)) || (rc = dalloc(c, &c->refl, (size_t)npatch * 3)) ||
         (rc = dalloc(c, &c->area, npatch)) || (rc = dalloc(c, &c->emis, (size_t)npatch * 3)) ||
@@ -649,7 +649,7 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     // records: one region of kRecsPerBlock per (setup block, shooter) plus a
     // spill region; bin entries: three per record slot
     c->bb.nblk = nblk ? nblk : 1;
-    c->bb.nz = K <= 4 ? 5u : 1u;
+    c->bb.nz = K <= 4 && (uint64_t)c->bb.nblk * K < kFaceBlocks ? 5u : 1u;
     c->bb.setup_group = 8;
     while (c->bb.setup_group > 1 &&
            (uint64_t)c->bb.nblk * c->bb.nz * K < (uint64_t)kSetupGroups * c->bb.setup_group)
@@ -711,7 +711,7 @@ int upload_copy(rad_ctx *c, const float *tri_xyz, const uint32_t *tri_patch, uin
             planes[(size_t)k * ntri + t] = tri_xyz[(size_t)t * 9 + k];
     HIPCHK(c, hipMemcpy(c->tri, planes.data(), planes.size() * sizeof(float), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->tri_patch, tri_patch, (size_t)ntri * 4, hipMemcpyHostToDevice));
-    launch_tri_sphere(c->tri, ntri, c->tsph, c->st);
+    launch_tri_sphere(c->tri, ntri, c->tsph, c->tback, c->st);
     launch_clusters(c->tri, ntri, nullptr, 0, c->clu, c->st);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpy(c->frames, frames, (size_t)npatch * 36, hipMemcpyHostToDevice));
@@ -1573,7 +1573,7 @@ int rad_debug_bins(rad_ctx *c, uint32_t *out, uint32_t *ntiles, uint32_t *tile_p
             return rc;
         launch_clear(c->K, c->bb.count, c->bb.ntiles, nullptr, nullptr, 0, 0, cnt, c->bb.ent_cap,
                      c->st);
-        launch_raster_setup(c->g, 0, c->last_k, 0, c->tri, c->tsph, c->tri_patch, c->ntri, c->mvp,
+        launch_raster_setup(c->g, 0, c->last_k, 0, c->tri, c->tsph, c->tback, c->tri_patch, c->ntri, c->mvp,
                             c->nshoot, c->bb, cnt, c->pk.slot_tbeg, c->pk.slot_tcnt, c->pk.slot_w,
                             c->st);
         launch_bin(c->g, 0, c->last_k, 0, c->tri, c->tri_patch, c->ntri, c->mvp, c->bb, cnt,
@@ -2476,7 +2476,7 @@ int rad_scene_ingest(rad_ctx *c, const float *quads, uint32_t nface, const float
         launch_ingest(nface, nq, dfaces, dplan, dcol, dem, dsh, (uint32_t)mode, nt, c->tri,
                       c->tri_patch, c->frames, c->refl, c->area, c->emis, c->unshot, c->shot,
                       c->patch_quad, c->quad_pbeg, c->quad_nbr, c->st);
-        launch_tri_sphere(c->tri, nt, c->tsph, c->st);
+        launch_tri_sphere(c->tri, nt, c->tsph, c->tback, c->st);
         launch_clusters(c->tri, nt, nullptr, 0, c->clu, c->st);
         e = hipGetLastError();
     }

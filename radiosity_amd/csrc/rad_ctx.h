@@ -45,6 +45,7 @@ struct rad_ctx {
     float *tri = nullptr;          // 9 planes of ntri
     uint32_t *tri_patch = nullptr; // ntri
     float4 *tsph = nullptr;        // ntri bounding spheres (centre, radius)
+    float4 *tback = nullptr;       // ntri drawn sides (k_tri_sphere)
     float4 *clu = nullptr;         // bounds of the runs of 64 and 16 triangles
     float *frames = nullptr;       // npatch*9
     float *refl = nullptr;         // npatch*3

@@ -88,6 +88,13 @@ constexpr uint32_t kSplitBins = 8192;
 // hemicube 128: 16,384 triangles 155 us at 8 slots a workgroup (512
 // workgroups), 122 us at 2 (2,048); 200,000 triangles (50,000 pairs) keep 8.
 constexpr uint32_t kSetupGroups = 1200;
+// Blocks of 256 triangles x slots (of at most 4) from which a setup workgroup
+// takes all five faces instead of one: with the faces apart it reads the
+// triangles five times and its exact phase has a fifth of the lanes busy, but
+// five times the workgroups.  Five workgroups against one, time of a pass at
+// hemicube 256: 97 blocks, 1 slot 48.6 against 50.6 us, 4 slots 63.0, 63.3; 195
+// blocks, 2 slots 67.6, 67.3; 782 blocks, 1 slot 75.4, 67.7, 4 slots 100.7, 91.0.
+constexpr uint32_t kFaceBlocks = 384;
 
 // Control block of a context (u32 words on the device), written by the
 // shoot kernels and read by the pass gate in k_prepare_clear:
@@ -188,11 +195,11 @@ void launch_clear(uint32_t K, uint32_t *bin_count, uint32_t ntiles, float *ff, u
 // writes the item buffer, ff or ffq != null reduces into F rows and hits).  h selects the counter block,
 // spill region and clip queue (0, or 1 for the second half of a split pass).
 void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h,
-                         const float *tri, const float4 *tsph, const uint32_t *tri_patch,
-                         uint32_t ntri, const float *mvp, const uint32_t *nshoot,
+                         const float *tri, const float4 *tsph, const float4 *tback,
+                         const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const uint32_t *nshoot,
                          const BinBuffers &bb, uint32_t *counters, const uint32_t *slot_tbeg,
                          const uint32_t *slot_tcnt, const uint32_t *slot_w, hipStream_t st);
-void launch_tri_sphere(const float *tri, uint32_t ntri, float4 *sph, hipStream_t st);
+void launch_tri_sphere(const float *tri, uint32_t ntri, float4 *sph, float4 *back, hipStream_t st);
 void launch_bin(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const float *tri,
                 const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const BinBuffers &bb,
                 uint32_t *counters, const uint32_t *slot_w, hipStream_t st);

@@ -481,14 +481,19 @@ __device__ static inline void setup_face(const float *mm, float4 scis, const flo
     emit_tri(a, b, c, id, fv, s, face, bc);
 }
 
-__device__ static uint32_t cull_faces(const float *__restrict__ sm, const float (&vx)[3][3],
-                                      float4 sph, int f0, int f1);
+__device__ static uint32_t cull_faces(const float *__restrict__ sm, const float (&lv)[9][256],
+                                      float4 sph, float4 back, float halfW, int f0, int f1);
 
 // Bounding sphere of every triangle, once per scene: the centroid as stored
 // and the largest vertex distance from it, inflated by 1e-5 relative so it
-// bounds the vertices whatever the rounding of the distances.
+// bounds the vertices whatever the rounding of the distances.  And its drawn
+// side: the camera mirrors (right = up x dir), so a triangle is
+// counter-clockwise seen from the side of (v2 - v0) x (v1 - v0); that over the
+// longest edge, which leaves the triangle's smallest height as its length,
+// and the longest edge.
 __global__ __launch_bounds__(256) void k_tri_sphere(const float *__restrict__ tri, uint32_t ntri,
-                                                    float4 *__restrict__ sph)
+                                                    float4 *__restrict__ sph,
+                                                    float4 *__restrict__ back)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ntri)
@@ -506,12 +511,26 @@ __global__ __launch_bounds__(256) void k_tri_sphere(const float *__restrict__ tr
         r2 = fmaxf(r2, dx * dx + dy * dy + dz * dz);
     }
     sph[t] = make_float4(cx, cy, cz, sqrtf(r2) * 1.00001f);
+    float e1[3], e2[3], l1 = 0.0f, l2 = 0.0f, l3 = 0.0f;
+    for (int c = 0; c < 3; ++c) {
+        e1[c] = v[1][c] - v[0][c];
+        e2[c] = v[2][c] - v[0][c];
+        const float e3 = v[2][c] - v[1][c];
+        l1 += e1[c] * e1[c];
+        l2 += e2[c] * e2[c];
+        l3 += e3 * e3;
+    }
+    const float edge = sqrtf(fmaxf(l1, fmaxf(l2, l3)));
+    const float inv = edge > 0.0f ? 1.0f / edge : 0.0f;
+    back[t] = make_float4((e2[1] * e1[2] - e2[2] * e1[1]) * inv,
+                          (e2[2] * e1[0] - e2[0] * e1[2]) * inv,
+                          (e2[0] * e1[1] - e2[1] * e1[0]) * inv, edge);
 }
 
-void launch_tri_sphere(const float *tri, uint32_t ntri, float4 *sph, hipStream_t st)
+void launch_tri_sphere(const float *tri, uint32_t ntri, float4 *sph, float4 *back, hipStream_t st)
 {
     if (ntri)
-        k_tri_sphere<<<(ntri + 255) / 256, 256, 0, st>>>(tri, ntri, sph);
+        k_tri_sphere<<<(ntri + 255) / 256, 256, 0, st>>>(tri, ntri, sph, back);
 }
 
 // Tile columns [g0, g1] and rows [h0, h1] of a record's texel bbox.
@@ -540,6 +559,7 @@ __device__ static inline void unpack_bbox(uint64_t v, uint32_t tshift, uint32_t 
 // [slot_tbeg[s], slot_tbeg[s] + slot_tcnt[s]); blockIdx.x walks that range.
 __global__ __launch_bounds__(256) void k_raster_setup(uint32_t W, const float *__restrict__ tri,
                                                       const float4 *__restrict__ tsph,
+                                                      const float4 *__restrict__ tback,
                                                       const uint32_t *__restrict__ tri_patch,
                                                       uint32_t ntri, const float *__restrict__ mvp,
                                                       const uint32_t *__restrict__ nshoot,
@@ -576,8 +596,7 @@ __global__ __launch_bounds__(256) void k_raster_setup(uint32_t W, const float *_
     // and the per-slot set-up by the slot count; each keeps its own record region, tile counts and
     // record count.
     uint32_t ltb = 0xFFFFFFFFu, ltc = 0;
-    float vx[3][3];
-    float4 sph = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 sph = make_float4(0.0f, 0.0f, 0.0f, 0.0f), back = sph;
     for (uint32_t g = 0; g < group;) {
         const uint32_t s = (slot0 + blockIdx.y * group) + g;
         if (s >= ns)
@@ -613,12 +632,11 @@ __global__ __launch_bounds__(256) void k_raster_setup(uint32_t W, const float *_
 #pragma unroll
                 for (int k = 0; k < 3; ++k)
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        vx[k][c] = tri[(size_t)(3 * k + c) * ntri + t];
-                        lv[3 * k + c][threadIdx.x] = vx[k][c];
-                    }
+                    for (int c = 0; c < 3; ++c)
+                        lv[3 * k + c][threadIdx.x] = tri[(size_t)(3 * k + c) * ntri + t];
                 lid[threadIdx.x] = tri_patch[t] + 1u;
                 sph = tsph[t];
+                back = tback[t];
             }
         }
         for (uint32_t i = threadIdx.x; i < nsh * bc.ntiles; i += blockDim.x)
@@ -634,7 +652,8 @@ __global__ __launch_bounds__(256) void k_raster_setup(uint32_t W, const float *_
         // an LDS queue
         if (tl0 + threadIdx.x < tc) {
             for (uint32_t sh = 0; sh < nsh; ++sh) {
-                uint32_t fm = cull_faces(mvp + (size_t)(s + sh) * kShooterStride, vx, sph, f0, f1);
+                uint32_t fm = cull_faces(mvp + (size_t)(s + sh) * kShooterStride, lv, sph, back,
+                                         0.5f * (float)Ws, f0, f1);
                 while (fm) {
                     int f = __ffs(fm) - 1;
                     fm &= fm - 1;
@@ -667,22 +686,52 @@ __global__ __launch_bounds__(256) void k_raster_setup(uint32_t W, const float *_
         // the records into their tiles' lists: one returning global atomic per
         // touched tile reserves the entries, whose first place takes the
         // count's place in LDS ...
+        const uint32_t e1 = lnrec2[0], e2 = e1 + lnrec2[1], e3 = e2 + lnrec2[2],
+                       e4 = e3 + lnrec2[3];
+        auto rec_of = [&](uint32_t f, uint32_t &sh) {
+            sh = (f >= e1 ? 1u : 0u) + (f >= e2 ? 1u : 0u) + (f >= e3 ? 1u : 0u);
+            const uint32_t q = f - (sh == 0 ? 0u : sh == 1 ? e1 : sh == 2 ? e2 : e3);
+            return rbof(s + sh) * kRecsPerBlock + q;
+        };
+        // (a thread's first bbox comes back during the atomics)
+        uint32_t sh0 = 0, r0 = 0;
+        uint64_t v0 = 0;
+        if (threadIdx.x < e4) {
+            r0 = rec_of(threadIdx.x, sh0);
+            v0 = bc.bbox[r0];
+        }
         uint32_t *const cnt = bc.bin_count + (size_t)s * bc.ntiles;
-        for (uint32_t i = threadIdx.x; i < nsh * bc.ntiles; i += blockDim.x)
-            if (lcnt[i])
-                lcnt[i] = atomicAdd(&cnt[i], lcnt[i]);
+        const uint32_t nl = nsh * bc.ntiles;
+        for (uint32_t i0 = threadIdx.x; i0 < nl; i0 += 4u * blockDim.x) {
+            uint32_t c[4];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t i = i0 + j * blockDim.x;
+                c[j] = i < nl ? lcnt[i] : 0u;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                if (c[j])
+                    c[j] = atomicAdd(&cnt[i0 + j * blockDim.x], c[j]);
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t i = i0 + j * blockDim.x;
+                if (i < nl)
+                    lcnt[i] = c[j];
+            }
+        }
         if (threadIdx.x < nsh)
             blk_nrec[rbof(s + threadIdx.x)] = lnrec2[threadIdx.x];
         __syncthreads();
         // ... and every record counts on from it
-        const uint32_t e1 = lnrec2[0], e2 = e1 + lnrec2[1], e3 = e2 + lnrec2[2],
-                       e4 = e3 + lnrec2[3];
         for (uint32_t f = threadIdx.x; f < e4; f += blockDim.x) {
-            const uint32_t sh = (f >= e1 ? 1u : 0u) + (f >= e2 ? 1u : 0u) + (f >= e3 ? 1u : 0u);
-            const uint32_t q = f - (sh == 0 ? 0u : sh == 1 ? e1 : sh == 2 ? e2 : e3);
-            const uint32_t r = rbof(s + sh) * kRecsPerBlock + q;
+            uint32_t sh = sh0, r = r0;
+            if (f != threadIdx.x) {
+                r = rec_of(f, sh);
+                v0 = bc.bbox[r];
+            }
             uint32_t g0, g1, h0, h1;
-            unpack_bbox(bc.bbox[r], bc.tshift, g0, g1, h0, h1);
+            unpack_bbox(v0, bc.tshift, g0, g1, h0, h1);
             for (uint32_t gy = h0; gy <= h1; ++gy)
                 for (uint32_t gx = g0; gx <= g1; ++gx) {
                     const uint32_t b = gy * bc.ntx + gx;
@@ -710,9 +759,20 @@ __global__ __launch_bounds__(256) void k_raster_setup(uint32_t W, const float *_
 //    in the front face it is nearer than the near plane.  This removes the
 //    shooter's own plane (floor under a floor patch) before any per-face work;
 //  - a face whose frustum (90 degree pyramid around its axis, near 0.01)
-//    misses the sphere by more than a margin.
-__device__ static uint32_t cull_faces(const float *__restrict__ sm, const float (&vx)[3][3],
-                                      float4 sph, int f0, int f1)
+//    misses the sphere by more than a margin;
+//  - a triangle (of one face only, by the last test) of area A whose plane the eye lies at least D > 0 behind:
+//    with depths in [wmin, wmax] it projects to a clockwise area of at least
+//    (W/2)^2 2 A D / wmax^3 square pixels.  Snapping and rounding move a
+//    vertex by at most delta pixels per axis, which changes the area by at
+//    most 5.7 delta L + 8 delta^2 for a longest projected edge
+//    L <= sqrt2 (W/2) edge (1 + kappa) / wmin, kappa the largest |x / w|; the
+//    two tests ask twice that, multiplied out, so the snapped triangle is
+//    clockwise too and would be dropped.  back: k_tri_sphere's, whose product
+//    with the centre's offset is 2 A D / edge.  (Two in five triangles that
+//    pass the other culls in rooms with boxes; each costs the exact pipeline
+//    three projections.)
+__device__ static uint32_t cull_faces(const float *__restrict__ sm, const float (&lv)[9][256],
+                                      float4 sph, float4 back, float halfW, int f0, int f1)
 {
     if (sm[92] != 0.0f)
         return ((1u << f1) - 1u) & ~((1u << f0) - 1u);
@@ -721,17 +781,18 @@ __device__ static uint32_t cull_faces(const float *__restrict__ sm, const float 
     const float ux = sm[86], uy = sm[87], uz = sm[88];
     const float wx = sm[89], wy = sm[90], wz = sm[91];
     const float cx = sph.x - ex, cy = sph.y - ey, cz = sph.z - ez, rho = sph.w;
-    const float pa = cx * nx + cy * ny + cz * nz;
-    const float pb = cx * ux + cy * uy + cz * uz;
-    const float pc = cx * wx + cy * wy + cz * wz;
-    const float mq = 1e-4f * (fabsf(pa) + fabsf(pb) + fabsf(pc) + rho) + 1e-6f;
+    const float pa = fmaf(cz, nz, fmaf(cy, ny, cx * nx));
+    const float pb = fmaf(cz, uz, fmaf(cy, uy, cx * ux));
+    const float pc = fmaf(cz, wz, fmaf(cy, wy, cx * wx));
+    const float mq = fmaf(1e-4f, fabsf(pa) + fabsf(pb) + fabsf(pc) + rho, 1e-6f);
     if (pa + rho + mq < 0.0f)
         return 0u;
     if (pa - rho - mq <= 0.0099f) {
         bool below = true;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            float dx = vx[k][0] - ex, dy = vx[k][1] - ey, dz = vx[k][2] - ez;
+            float dx = lv[3 * k][threadIdx.x] - ex, dy = lv[3 * k + 1][threadIdx.x] - ey,
+                  dz = lv[3 * k + 2][threadIdx.x] - ez;
             float h = dx * nx + dy * ny + dz * nz;
             float tol = fminf(1e-6f * (fabsf(dx) + fabsf(dy) + fabsf(dz)), 0.0099f);
             below = below && (h < tol);
@@ -739,20 +800,43 @@ __device__ static uint32_t cull_faces(const float *__restrict__ sm, const float 
         if (below)
             return 0u;
     }
-    const float m = rho * 1.4143f + mq;
-    uint32_t mask = 0u;
-    for (int face = f0; face < f1; ++face) {
-        float q, s1, s2;
-        switch (face) {
-        case 0: q = pb; s1 = pa; s2 = pc; break;   // UP    (axis  u)
-        case 1: q = -pb; s1 = pa; s2 = pc; break;  // DOWN  (axis -u)
-        case 2: q = pc; s1 = pa; s2 = pb; break;   // LEFT  (axis n x u)
-        case 3: q = -pc; s1 = pa; s2 = pb; break;  // RIGHT (axis -(n x u))
-        default: q = pa; s1 = pb; s2 = pc; break;  // FRONT (axis n)
+    const float m = fmaf(rho, 1.4143f, mq);
+    const float far = fmaxf(fabsf(pa), fmaxf(fabsf(pb), fabsf(pc))), T = far - m;
+    const uint32_t faces = ((1u << f1) - 1u) & ~((1u << f0) - 1u);
+    if (!(T > 0.0f)) {
+        // near the eye: face by face
+        uint32_t mask = 0u;
+        for (int face = f0; face < f1; ++face) {
+            float q, s1, s2;
+            switch (face) {
+            case 0: q = pb; s1 = pa; s2 = pc; break;   // UP    (axis  u)
+            case 1: q = -pb; s1 = pa; s2 = pc; break;  // DOWN  (axis -u)
+            case 2: q = pc; s1 = pa; s2 = pb; break;   // LEFT  (axis n x u)
+            case 3: q = -pc; s1 = pa; s2 = pb; break;  // RIGHT (axis -(n x u))
+            default: q = pa; s1 = pb; s2 = pc; break;  // FRONT (axis n)
+            }
+            if (q + m < fabsf(s1) || q + m < fabsf(s2) || q + rho + m < 0.0099f)
+                continue;
+            mask |= 1u << face;
         }
-        if (q + m < fabsf(s1) || q + m < fabsf(s2) || q + rho + m < 0.0099f)
-            continue;
-        mask |= 1u << face;
+        return mask;
+    }
+    // farther than its margin: the face of the largest coordinate and those
+    // whose coordinate comes within the margin of it
+    uint32_t mask = (fabsf(pb) >= T ? (pb > 0.0f ? 1u : 2u) : 0u) |
+                    (fabsf(pc) >= T ? (pc > 0.0f ? 4u : 8u) : 0u) | (pa >= T ? 16u : 0u);
+    mask &= faces;
+    const float l1 = fabsf(cx) + fabsf(cy) + fabsf(cz);
+    const float db = fmaf(-4e-6f * l1, back.w, fmaf(cz, back.z, fmaf(cy, back.y, cx * back.x)));
+    if (db > 0.0f && (mask & (mask - 1u)) == 0u) {
+        const float wmin = far - rho - mq, wmax = far + rho + mq;
+        const float S = __builtin_amdgcn_fmed3f(fabsf(pa), fabsf(pb), fabsf(pc)) + rho;
+        const float em = 2e-6f * (fabsf(ex) + fabsf(ey) + fabsf(ez));
+        const float dw = fmaf(fmaf(1.6e-5f, halfW, 0.0025f), wmin, halfW * fmaf(1e-6f, l1, em));
+        const float a = 0.5f * halfW * db * wmin * wmin, w3 = 16.0f * dw * wmax * wmax * wmax;
+        if (wmin > 0.02f && S <= 8.0f * wmin && a * wmin > w3 * (wmin + S) &&
+            a * halfW * back.w > w3 * dw)
+            mask = 0u;
     }
     return mask;
 }
@@ -1255,8 +1339,8 @@ static BinCtx bin_ctx(const BinBuffers &bb, uint32_t h, uint32_t *counters)
 }
 
 void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h,
-                         const float *tri, const float4 *tsph, const uint32_t *tri_patch,
-                         uint32_t ntri, const float *mvp, const uint32_t *nshoot,
+                         const float *tri, const float4 *tsph, const float4 *tback,
+                         const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const uint32_t *nshoot,
                          const BinBuffers &bb, uint32_t *counters, const uint32_t *slot_tbeg,
                          const uint32_t *slot_tcnt, const uint32_t *slot_w, hipStream_t st)
 {
@@ -1266,7 +1350,7 @@ void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h
         group = n;
     dim3 grid(bb.nblk, (n + group - 1) / group, bb.nz);
     k_raster_setup<<<grid, 256, 4 * bb.ntiles * sizeof(uint32_t), st>>>(
-        g.W, tri, tsph, tri_patch, ntri, mvp, nshoot, bin_ctx(bb, h, counters), bb.blk_nrec,
+        g.W, tri, tsph, tback, tri_patch, ntri, mvp, nshoot, bin_ctx(bb, h, counters), bb.blk_nrec,
         slot_tbeg, slot_tcnt, slot_w, group, s0, s1);
 }
 

@@ -181,20 +181,26 @@ enum TriClass { kTriOut, kTriClip, kTriIn };
 // margin included): outside, in need of clipping, or inside.
 __device__ static inline TriClass classify_tri(const CV4 *poly, float4 scis)
 {
-    uint32_t all_out = 0x1f, any_out = 0;
+    // every clip_dist >= 0 (a difference has the sign of its comparison; NaN
+    // is outside) for nearly all triangles
+    bool in = true;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        uint32_t o = 0;
-#pragma unroll
-        for (int p = 0; p < 5; ++p)
-            o |= (clip_dist(poly[k], p) >= 0.0f ? 0u : 1u) << p;
-        all_out &= o;
-        any_out |= o;
+        const float w = poly[k].c[3], gw = kGuard * w;
+        in = in && poly[k].c[2] >= -w && fabsf(poly[k].c[0]) <= gw && fabsf(poly[k].c[1]) <= gw;
     }
-    if (all_out)
-        return kTriOut;
-    if (any_out)
-        return kTriClip;
+    if (!in) {
+        uint32_t all_out = 0x1f;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            uint32_t o = 0;
+#pragma unroll
+            for (int p = 0; p < 5; ++p)
+                o |= (clip_dist(poly[k], p) >= 0.0f ? 0u : 1u) << p;
+            all_out &= o;
+        }
+        return all_out ? kTriOut : kTriClip;
+    }
     // All vertices in front of the near plane (w > 0): reject against the
     // scissor rectangle in clip space with a one-pixel margin.
     const float lo_x = scis.x, hi_x = scis.y, lo_y = scis.z, hi_y = scis.w;

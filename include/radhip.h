@@ -56,7 +56,7 @@ typedef struct rad_config {
     uint32_t ocl_workitems_x; /* Config::oclWorkitemsX: spans per row for the run form (4) */
     uint32_t mode;            /* RAD_MODE_* */
     uint32_t select;          /* RAD_SELECT_* */
-    uint32_t small_tri_px;    /* raster tuning: triangle pixels in a tile drawn by one lane (0: 64) */
+    uint32_t small_tri_px;    /* raster tuning: triangle pixels in a tile drawn by one lane (0: 40 to 64, by the pass) */
     uint32_t tile_px;         /* raster tuning: screen tile side 8, 16 or 32 of the binned
                                  rasterizer (0: auto; small passes are then drawn without bins) */
     uint32_t graph_passes;    /* rad_step replays this many passes as one captured

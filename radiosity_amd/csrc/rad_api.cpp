@@ -124,6 +124,27 @@ static bool use_direct(const rad_ctx *c, uint32_t k, uint32_t *T)
     return c->auto_tile && direct_wins(k, c->g.W, ntri, T);
 }
 
+// The in-lane triangle limit of a pass over k slots where none was chosen.
+// Passes of up to 3 shooters (tiles of 16, or drawn directly) last as long as
+// a tile's slowest chunks, and a lower limit hands more of them to whole
+// wavefronts; at hemicube 128 and below, with more tiles than the GPU holds
+// at once, less divergence pays too.  Time of a pass at 40, 48 and 64 pixels:
+// 200,000 triangles at hemicube 256, 1 shooter 58.9, 61.3, 65.7 us, 2 73.8,
+// 76.2, 79.7, 4 94.8, 92.3, 92.2, 64 323, 318, 318; 60,000 at hemicube 128,
+// 64 shooters (3,072 tiles) 187.1, 187.5, 189.8; 20,000, 32 (1,536 tiles)
+// 95.6, 93.7, 91.5; the dense build over 16,384 patches (3,072 tiles) 27.2,
+// 27.1, 27.8 ms.  Drawn directly: 20,000 triangles at hemicube 256, 1 shooter
+// 28.9, 29.0, 29.5, 6,000 at hemicube 64, 16 shooters 55.2, 54.7, 54.6.
+static uint32_t lane_limit(const rad_ctx *c, uint32_t k)
+{
+    if (!c->auto_small)
+        return c->small_px;
+    if (c->last_direct || c->bb.tshift == 4)
+        return k < 4 ? 40u : c->small_px;
+    const bool many = c->bb.tshift == 5 && c->g.W <= 128 && k * c->bb.ntiles > 2048u;
+    return many ? 48u : c->small_px;
+}
+
 // A pass of kSplitMin or more slots and kSplitBins or more bins renders as
 // two halves side by side, except a timed one (stage events bracket whole
 // stages).
@@ -164,16 +185,19 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
     const bool fq = !ids && c->det;
     // stage j (0 setup, 1 bins, 2 tiles) of slots [s0, s1) with counter
     // block h on stream st
+    uint32_t T;
+    c->last_direct = use_direct(c, k, &T);
+    const uint32_t small_px = lane_limit(c, k);
     auto stage = [&](int j, uint32_t s0, uint32_t s1, uint32_t h, hipStream_t st) {
         if (j == 0)
-            launch_raster_setup(c->g, s0, s1, h, c->tri, c->tsph, c->tback, c->tri_patch, c->ntri, c->mvp,
-                                c->nshoot, c->bb, c->counters, c->pk.slot_tbeg,
-                                c->pk.slot_tcnt, c->pk.slot_w, st);
+            launch_raster_setup(c->g, s0, s1, h, c->tri, c->tsph, c->tback, c->tri_patch,
+                                c->ntri, c->mvp, c->nshoot, c->bb, c->counters,
+                                c->pk.slot_tbeg, c->pk.slot_tcnt, c->pk.slot_w, st);
         else if (j == 1)
             launch_bin(c->g, s0, s1, h, c->tri, c->tri_patch, c->ntri, c->mvp, c->bb, c->counters,
                        c->pk.slot_w, st);
         else
-            launch_tile(c->g, s0, s1, h, c->nshoot, c->bb, c->small_px, ids, depth,
+            launch_tile(c->g, s0, s1, h, c->nshoot, c->bb, small_px, ids, depth,
                         c->pk.slot_w ? c->pk.dffs : c->dff, c->rowlen, c->pk.slot_pbeg,
                         ids || fq ? nullptr : c->ff, fq ? c->ffq : nullptr, hits, c->counters,
                         c->pk.slot_w, c->pk.slot_dffo, c->fblk, c->K, st);
@@ -185,8 +209,6 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
     // With shoot_half, the first half's F rows are shot on the context
     // stream as soon as its tiles are done, while the second half still
     // renders; the caller shoots the second half.
-    uint32_t T;
-    c->last_direct = use_direct(c, k, &T);
     c->last_k = k;
     if (c->last_direct) {
         for (int j = 0; j < 2; ++j)
@@ -197,7 +219,7 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
         d.nslot = k;
         d.ntri = c->ntri;
         d.rowlen = c->rowlen;
-        d.small_px = c->small_px;
+        d.small_px = small_px;
         d.fstride = c->K;
         d.nshoot = c->nshoot;
         d.tri = c->tri;
@@ -499,6 +521,7 @@ int rad_create(const rad_config *cfg, rad_ctx **out)
         ncu = prop.multiProcessorCount;
     c->sel_blocks = ncu * 2;
     c->auto_tile = cfg->tile_px == 0;
+    c->auto_small = cfg->small_tri_px == 0;
     // screen tiles: 32x32 when enough hemicubes fill the GPU, else 16x16
     // (32x32 also when a hemicube would have more tiles than the bins hold)
     uint32_t T = cfg->tile_px ? cfg->tile_px : (c->K >= 4 ? 32u : 16u);
@@ -1419,8 +1442,9 @@ int rad_autotune(rad_ctx *c, uint32_t passes, rad_tune_result *out)
     }
     bool timing = c->timing;
     c->timing = false;
-    const bool was_auto = c->auto_tile;
+    const bool was_auto = c->auto_tile, was_auto_small = c->auto_small;
     c->auto_tile = false; // the candidates are the binned rasterizer's
+    c->auto_small = false;
     // K shooters spread evenly over the patch list: early in a solve the
     // selection holds only the few emitters, which is no sample of the work
     std::vector<uint32_t> spread(c->K);

@@ -139,18 +139,22 @@ static uint32_t lane_limit(const rad_ctx *c, uint32_t k)
 {
     if (!c->auto_small)
         return c->small_px;
-    if (c->last_direct || c->bb.tshift == 4)
+    if (c->last_direct)
         return k < 4 ? 40u : c->small_px;
+    if (c->bb.tshift == 4)
+        return 40u;
     const bool many = c->bb.tshift == 5 && c->g.W <= 128 && k * c->bb.ntiles > 2048u;
     return many ? 48u : c->small_px;
 }
 
 // A pass of kSplitMin or more slots and kSplitBins or more bins renders as
 // two halves side by side, except a timed one (stage events bracket whole
-// stages).
+// stages) and a pack's of scenes up to kSplitPack triangles.
 static bool split_render(const rad_ctx *c, uint32_t k)
 {
     uint32_t T;
+    if (c->pk.nscene && c->bb.nblk * 256u <= kSplitPack)
+        return false;
     return k >= kSplitMin && k * c->bb.ntiles >= kSplitBins && !c->timing &&
            !use_direct(c, k, &T);
 }
@@ -403,6 +407,32 @@ int bin_lists(rad_ctx *c)
     return dalloc(c, &c->bb.list, (size_t)c->bb.nbins * cap);
 }
 
+// The tile side of a context without a chosen one, for a scene of ntri
+// triangles (0: none yet; in a pack the largest's). Tiles of 32 read a record
+// that touches several tiles less often and cost fewer workgroups; tiles of
+// 16 spread few hemicubes, or dense ones, over four times as many. Time of a
+// pass, 16 against 32: hemicube 128 (48 tiles of 32), 12 shooters, 3,000
+// triangles 61.5 and 60.4 us, 16,000 64.6, 70.8; 16 (768 tiles) 66.3, 63.5
+// and 69.6, 74.4; 32 (1,536), 3,000 86.1, 76.5, 16,000 92.5, 95.2, and 32
+// deterministic ones over 20,000 107, 110; 64 (3,072) over 33,000 141, 134,
+// though from lights alone 60,000 took 167, 183. Hemicube 256 (192 tiles), 4
+// shooters, 3,000 triangles 65.7, 56.4, 60,000 71.4, 78.6; 8, 60,000 85.1,
+// 81.7: there a setup workgroup clears and reserves 768 tile counts for each
+// of its shooters.
+static uint32_t tile_side(const rad_ctx *c, uint32_t ntri)
+{
+    const uint32_t t16 = ((c->g.TW + 15) / 16) * ((c->g.TH + 15) / 16);
+    const uint32_t t32 = ((c->g.TW + 31) / 32) * ((c->g.TH + 31) / 32);
+    if (t16 > kMaxTilesPerSlab)
+        return 32u;
+    const uint32_t n32 = c->K * t32;
+    if (c->K < 4 || n32 < 640u)
+        return 16u;
+    const bool dense = n32 <= 768u ? ntri >= 100u * t32
+                                   : c->g.W <= 128 && n32 <= 1536u && ntri >= 300u * t32;
+    return dense ? 16u : 32u;
+}
+
 // Screen tile side T (8, 16, 32) and the in-lane triangle limit; (re)sizes
 // the per-(shooter, tile) bin arrays.
 int set_tiles(rad_ctx *c, uint32_t T, uint32_t small_px)
@@ -522,11 +552,8 @@ int rad_create(const rad_config *cfg, rad_ctx **out)
     c->sel_blocks = ncu * 2;
     c->auto_tile = cfg->tile_px == 0;
     c->auto_small = cfg->small_tri_px == 0;
-    // screen tiles: 32x32 when enough hemicubes fill the GPU, else 16x16
-    // (32x32 also when a hemicube would have more tiles than the bins hold)
-    uint32_t T = cfg->tile_px ? cfg->tile_px : (c->K >= 4 ? 32u : 16u);
-    if (!cfg->tile_px && ((c->g.TW + T - 1) / T) * ((c->g.TH + T - 1) / T) > kMaxTilesPerSlab)
-        T = 32;
+    c->auto_side = c->auto_tile;
+    const uint32_t T = cfg->tile_px ? cfg->tile_px : tile_side(c, 0);
     if ((rc = set_tiles(c, T, cfg->small_tri_px ? cfg->small_tri_px : 64u))) {
         rad_destroy(c);
         return rc;
@@ -655,6 +682,9 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     c->hash_valid = false;
     int rc;
     size_t K = c->K;
+    const uint32_t side = c->auto_side ? tile_side(c, nblk * 256u) : c->cfg.tile_px;
+    if (side != c->cfg.tile_px && (rc = set_tiles(c, side, c->small_px)))
+        return rc;
     if ((rc = dalloc(c, &c->tri, (size_t)ntri * 9)) || (rc = dalloc(c, &c->tri_patch, ntri)) ||
         (rc = dalloc(c, &c->tsph, ntri)) || (rc = dalloc(c, &c->tback, ntri)) ||
         (rc = dalloc(c, &c->clu, cluster_words(ntri, 0))) ||
@@ -1445,6 +1475,8 @@ int rad_autotune(rad_ctx *c, uint32_t passes, rad_tune_result *out)
     const bool was_auto = c->auto_tile, was_auto_small = c->auto_small;
     c->auto_tile = false; // the candidates are the binned rasterizer's
     c->auto_small = false;
+    const bool was_auto_side = c->auto_side;
+    c->auto_side = false;
     // K shooters spread evenly over the patch list: early in a solve the
     // selection holds only the few emitters, which is no sample of the work
     std::vector<uint32_t> spread(c->K);
@@ -1516,8 +1548,11 @@ int rad_autotune(rad_ctx *c, uint32_t passes, rad_tune_result *out)
     if (rc == RAD_OK && r.tile_px == 0)
         rc = fail(c, RAD_E_LIMIT, "autotune: every candidate overflowed the bins");
     int rc2 = set_tiles(c, rc == RAD_OK ? r.tile_px : T0, rc == RAD_OK ? r.small_tri_px : S0);
-    if (rc)
+    if (rc) {
         c->auto_tile = was_auto;
+        c->auto_small = was_auto_small;
+        c->auto_side = was_auto_side;
+    }
     if (rc)
         return rc;
     if (rc2)

@@ -94,6 +94,7 @@ struct rad_ctx {
     uint32_t small_px = 16;        // in-lane rasterization limit (pixels of a tile)
     int sel_blocks = 1024;
     bool auto_tile = true;         // no tile side chosen: small passes are drawn directly
+    bool auto_side = true;         // ... nor by the tuner: tile_side
     bool auto_small = true;        // no in-lane triangle limit chosen: lane_limit
     bool last_direct = false;      // the last pass was, over last_k slots
     uint32_t last_k = 0;

@@ -630,18 +630,25 @@ __global__ __launch_bounds__(kDirThreads) void k_direct(DirectArgs a)
 }
 
 // Whether k slots of hemicube side W over scenes of at most ntri triangles
-// are drawn directly, and the tile side: 32, or 16 where 32 gives fewer than
-// 128 workgroups.  The line, direct against binned (8 passes in a graph, box
-// rooms, us per 24 passes): 8,000 triangles, hemicube 128: 1 slot (48
-// workgroups of 32) 945 / 1332, 8 slots (384) 1556 / 1821, 16 slots (768)
-// 2205 / 2026; hemicube 256: 2 slots (384) 1446 / 1833, 4 slots (768) 1910 /
-// 1850.  40,000 triangles, hemicube 64: 24 slots (288) 2722 / 3280; hemicube
-// 128, 8 slots 2348 / 2446; 80,000 triangles: 4824 / 4241 and 3333 / 3371.
+// are drawn directly, and the tile side.  A workgroup has a CU to itself: tiles
+// of 16 while those fit at once, else of 32.  It looks at every cluster of the
+// scene and draws its tile's share alone, so it wins for few triangles a
+// tile.  Direct against binned, us per pass (8 in a graph, box rooms): tiles of
+// 16, hemicube 32 (12 tiles), 8 slots, 8,000 triangles 40.3 / 46.7, 14,000 49.7 /
+// 47.6; 64 (48 tiles), 4 slots, 20,000 43.9 / 46.7, 40,000 57.4 / 52.3; 128 (192
+// tiles), 1 slot, 40,000 36.7 / 38.2.  Tiles of 32, hemicube 64 (12 tiles), 16
+// slots, 8,000 51.2 / 55.9, 20,000 68.5 / 59.5; 128 (48 tiles), 4 slots, 20,000
+// 49.2 / 51.4, 40,000 61.1 / 53.7; 256 (192 tiles), 1 slot, 28,000 37.6 / 40.5,
+// 40,000 45.5 / 43.3.  More than fit at once: 128, 8 slots, 4,000 53.4 / 54.9,
+// 14,000 59.3 / 56.1; 256, 2 slots, 8,000 50.0 / 52.6; 64, 32 slots, 4,000 72.2 /
+// 64.9.
 bool direct_wins(uint32_t k, uint32_t W, uint32_t ntri, uint32_t *T)
 {
     const uint32_t wg = k * direct_tiles(W, 32);
-    *T = wg < 128 ? 16u : 32u;
-    return wg <= 512 && ntri <= 64 * kDirChunk;
+    *T = wg <= 64 ? 16u : 32u;
+    if (wg > 256)
+        return wg <= 384 && W >= 128 && ntri <= 8192;
+    return ntri <= 600u * direct_tiles(W, *T) && ntri <= (wg <= 64 ? 64 * kDirChunk : 34816u);
 }
 
 void launch_direct(const DirectArgs &args, uint32_t T, hipStream_t st)

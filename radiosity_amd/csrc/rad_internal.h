@@ -81,6 +81,11 @@ constexpr uint32_t kSplitMin = 16; // smallest pass rendered as two halves
 // 32 shooters at hemicube 256 (6,144) 277 -> 279; 20 at hemicube 128 247 -> 263;
 // 16 at hemicube 64 82 -> 93.
 constexpr uint32_t kSplitBins = 8192;
+// ... and in a pack the largest scene's triangles above which: its passes
+// shoot and select only when both halves are done.  32 scenes, 64 shooters at
+// hemicube 256, whole against halves: up to 2,000 triangles 85 and 93 us, up to
+// 20,000 197, 203, 20,000 to 40,000 355, 356, 60,000 to 80,000 637, 624.
+constexpr uint32_t kSplitPack = 32768;
 // Workgroups the setup should have before each walks more
 // than one shooter slot (then up to 8, which reads the vertices once per 8
 // shooters).  About five per CU are resident; walking 8 slots whatever the

@@ -1908,13 +1908,16 @@ __global__ __launch_bounds__(NT) void k_shoot(uint32_t mode, const uint32_t *__r
                 ff[(size_t)(g0 + (uint32_t)__ffsll((long long)m) - 1) * npatch + j] = 0.0f;
         }
     }
-    if (live) {
-        if (last) {
-            // Main.cpp:1287-1295
-            if (n && sid[n - 1] == j)
-                stop_test(ctl, u0, u1, u2);
-            for (uint32_t s = 0; s < n; ++s) {
-                if (sid[s] == j) {
+    if (last) {
+        // Main.cpp:1287-1295
+        if (live && n && sid[n - 1] == j)
+            stop_test(ctl, u0, u1, u2);
+        // the pass's shooters among the wavefront's receivers, in order
+        for (uint32_t s0 = 0; s0 < n; s0 += 64) {
+            const bool here = s0 + lane < n && (sid[s0 + lane] >> 6) == blk;
+            for (uint64_t m = __ballot(here); m; m &= m - 1) {
+                const uint32_t s = s0 + (uint32_t)__ffsll((long long)m) - 1u;
+                if (live && sid[s] == j) {
                     float d0 = snap[3 * s + 0], d1 = snap[3 * s + 1], d2 = snap[3 * s + 2];
                     shot[3 * (size_t)j + 0] += d0;
                     shot[3 * (size_t)j + 1] += d1;
@@ -1925,6 +1928,8 @@ __global__ __launch_bounds__(NT) void k_shoot(uint32_t mode, const uint32_t *__r
                 }
             }
         }
+    }
+    if (live) {
         unshot[3 * (size_t)j + 0] = u0;
         unshot[3 * (size_t)j + 1] = u1;
         unshot[3 * (size_t)j + 2] = u2;

@@ -1774,8 +1774,8 @@ int sum_parts(rad_ctx *c, GatherBufs &g, double *out)
 extern "C" {
 
 // The shooting-layout build as replays of a captured graph of
-// kDenseGraphPasses passes: each pass takes the next K rows from a device
-// counter (k_iota_next), renders them and stores them transposed; passes
+// kDenseGraphPasses passes, whose first row a device counter holds: each pass
+// renders its K rows, stores them transposed and prepares the next; passes
 // beyond the last patch select nobody and store nothing.  The F rows are
 // zero at the start of every captured pass (the transposed store zeroes
 // what it reads).
@@ -1786,19 +1786,24 @@ static int dense_build_graph(rad_ctx *c, uint32_t npass)
                      c->counters, c->bb.ent_cap, c->st);
         c->ff_dirty = 0;
     }
-    const uint32_t start = 0u - c->K; // the first pass advances it to row 0
+    const uint32_t rows = kDenseGraphPasses * c->K;
+    const uint32_t start = 0u - rows; // the first replay advances it to row 0
     HIPCHK(c, hipMemcpyAsync(c->ctl + kCtlDenseBase, &start, 4, hipMemcpyHostToDevice, c->st));
+    const NextPass np{c->K,   c->shooters,  c->nshoot, c->frames, c->snap,
+                      c->mvp, c->bb.count, (size_t)c->K * c->bb.ntiles, c->counters,
+                      c->bb.ent_cap};
+    launch_dense_prepare(np, c->unshot, c->ctl, c->npatch, c->st);
     HIPCHK(c, hipStreamSynchronize(c->st));
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     HIPCHK(c, hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
     int rc = RAD_OK;
+    launch_dense_advance(rows, c->ctl, c->st);
     for (uint32_t p = 0; p < kDenseGraphPasses && rc == RAD_OK; ++p) {
-        launch_iota_next(c->K, c->npatch, c->ctl, c->shooters, c->nshoot, c->st);
-        if ((rc = render_pass(c, c->K, 0, nullptr, nullptr, nullptr)))
+        if ((rc = render_pass(c, c->K, 0, nullptr, nullptr, nullptr, nullptr, nullptr, false, true)))
             break;
-        launch_dense_store_t_dev(c->ff, c->K, c->ctl, c->nshoot, c->npatch, c->npad, c->area,
-                                 c->fhi, c->flo, c->st);
+        launch_dense_store_t_dev(c->ff, p * c->K, c->ctl, c->npatch, c->npad, c->area, c->fhi,
+                                 c->flo, np, c->unshot, c->st);
         c->ff_dirty = 0;
         rc = check_launch(c, "dense store");
     }

@@ -15,6 +15,7 @@
 //   vectors (E, B, r) rp x npad f32, same column-major order
 //   YP     S x rp x npad f32: split-K partial products F X
 #include "rad_internal.h"
+#include "rad_prepare.h"
 
 namespace rad {
 
@@ -59,22 +60,53 @@ __global__ void k_iota_shooters(uint32_t row0, uint32_t k, uint32_t *shooters, u
         *nshoot = k;
 }
 
-// The next pass of a captured dense build: ctl[kCtlDenseBase] advances by K
-// (one workgroup of at least K threads) and its rows become the shooters.
-__global__ void k_iota_next(uint32_t K, uint32_t npatch, uint32_t *__restrict__ ctl,
-                            uint32_t *__restrict__ shooters, uint32_t *__restrict__ nshoot)
+// The first row of a captured dense build's next group of passes.
+__global__ void k_dense_advance(uint32_t rows, uint32_t *__restrict__ ctl)
 {
-    __shared__ uint32_t base;
+    if (threadIdx.x == 0)
+        ctl[kCtlDenseBase] += rows;
+}
+
+// The rows a pass of a captured dense build takes: K from row0 on or the rest
+// of the patches (none beyond the last, or once the stop flag is set).
+__device__ static inline uint32_t dense_rows(const uint32_t *__restrict__ ctl, uint32_t K,
+                                             uint32_t row0, uint32_t npatch)
+{
+    return row0 < npatch && !ctl[kCtlStop] ? min(K, npatch - row0) : 0u;
+}
+
+// The preparation of the pass that takes K rows from row0 on, by nwg
+// workgroups of 256 threads: the first one's shooters, MVPs and snapshots, the
+// others' cleared bins and counters.
+__device__ static void dense_prepare(const NextPass &np, const float *__restrict__ unshot,
+                                     const uint32_t *__restrict__ ctl, uint32_t row0,
+                                     uint32_t npatch, uint32_t wg, uint32_t nwg)
+{
+    __shared__ uint32_t ssel[RAD_MAX_K], sn;
+    if (wg) {
+        clear_range((size_t)(wg - 1u) * blockDim.x + threadIdx.x, (size_t)(nwg - 1u) * blockDim.x,
+                    np.bin_count, np.nbins, nullptr, nullptr, 0, np.counters, np.ent_cap);
+        return;
+    }
+    const uint32_t k = dense_rows(ctl, np.K, row0, npatch);
+    for (uint32_t s = threadIdx.x; s < k; s += blockDim.x) {
+        ssel[s] = row0 + s;
+        np.shooters[s] = row0 + s;
+    }
     if (threadIdx.x == 0) {
-        base = ctl[kCtlDenseBase] + K;
-        ctl[kCtlDenseBase] = base;
+        sn = k;
+        *np.nshoot = k;
     }
     __syncthreads();
-    const uint32_t k = base < npatch ? min(K, npatch - base) : 0u;
-    if (threadIdx.x < k)
-        shooters[threadIdx.x] = base + threadIdx.x;
-    if (threadIdx.x == 0)
-        *nshoot = k;
+    for (uint32_t i = threadIdx.x; i < np.K * 5u; i += blockDim.x)
+        prepare_item(i, np.K, ssel, &sn, np.frames, unshot, np.snap, np.mvp, nullptr);
+}
+
+__global__ __launch_bounds__(256) void k_dense_prepare(NextPass np, const float *__restrict__ unshot,
+                                                       const uint32_t *__restrict__ ctl,
+                                                       uint32_t npatch)
+{
+    dense_prepare(np, unshot, ctl, 0u, npatch, blockIdx.x, gridDim.x);
 }
 
 // Rows row0 .. row0+k-1 of F from the F rows of one pass (k x npatch f32).
@@ -124,8 +156,11 @@ __global__ void k_dense_store(const float *__restrict__ ff, uint32_t k, uint32_t
 // and of lo).  Only the k columns of this pass are written.  Each thread
 // issues its 16 loads of a chunk at once, and sets every nonzero F entry it
 // read back to zero, so the pass's F rows are left zero for the next one.
-// With dctl != null (a captured build), row0 is dctl[kCtlDenseBase] and k
-// is *dk.
+// With dctl != null (a captured build), the rows are the np.K from
+// dctl[kCtlDenseBase] + row0 on, and the workgroups from nstore on prepare the
+// next pass, which takes the np.K after those: a launch of its own for its
+// shooters and one for the rest took 9 us of a pass's 96 (64 shooters, 16,384
+// patches, hemicube 128).
 __global__ __launch_bounds__(256) void k_dense_store_t(float *__restrict__ ff, uint32_t k,
                                                        uint32_t row0, uint32_t npatch,
                                                        uint32_t npad,
@@ -133,11 +168,17 @@ __global__ __launch_bounds__(256) void k_dense_store_t(float *__restrict__ ff, u
                                                        uint16_t *__restrict__ fhi,
                                                        uint16_t *__restrict__ flo,
                                                        const uint32_t *__restrict__ dctl,
-                                                       const uint32_t *__restrict__ dk)
+                                                       uint32_t nstore, NextPass np,
+                                                       const float *__restrict__ unshot)
 {
     if (dctl) {
-        row0 = dctl[kCtlDenseBase];
-        k = *dk;
+        row0 += dctl[kCtlDenseBase];
+        if (blockIdx.x >= nstore) {
+            dense_prepare(np, unshot, dctl, row0 + np.K, npatch, blockIdx.x - nstore,
+                          gridDim.x - nstore);
+            return;
+        }
+        k = dense_rows(dctl, np.K, row0, npatch);
     }
     __shared__ uint32_t tile[64][65]; // hi | lo << 16 per (receiver, shooter)
     const uint32_t t = threadIdx.x, jl = t & 63;
@@ -788,21 +829,30 @@ void launch_dense_store_t(float *ff, uint32_t k, uint32_t row0, uint32_t npatch,
                           hipStream_t st)
 {
     k_dense_store_t<<<(npatch + 63) / 64, 256, 0, st>>>(ff, k, row0, npatch, npad, area, fhi,
-                                                        flo, nullptr, nullptr);
+                                                        flo, nullptr, 0u, NextPass{}, nullptr);
 }
 
-void launch_iota_next(uint32_t K, uint32_t npatch, uint32_t *ctl, uint32_t *shooters,
-                      uint32_t *nshoot, hipStream_t st)
+// Workgroups of dense_prepare: 1,024 bins each for those that clear.
+static uint32_t prepare_wgs(const NextPass &np) { return 1u + (uint32_t)((np.nbins + 1023) / 1024); }
+
+void launch_dense_advance(uint32_t rows, uint32_t *ctl, hipStream_t st)
 {
-    k_iota_next<<<1, (K + 63) / 64 * 64, 0, st>>>(K, npatch, ctl, shooters, nshoot);
+    k_dense_advance<<<1, 64, 0, st>>>(rows, ctl);
 }
 
-void launch_dense_store_t_dev(float *ff, uint32_t K, const uint32_t *ctl, const uint32_t *nshoot,
-                              uint32_t npatch, uint32_t npad, const float *area, uint16_t *fhi,
-                              uint16_t *flo, hipStream_t st)
+void launch_dense_prepare(const NextPass &np, const float *unshot, const uint32_t *ctl,
+                          uint32_t npatch, hipStream_t st)
 {
-    k_dense_store_t<<<(npatch + 63) / 64, 256, 0, st>>>(ff, K, 0u, npatch, npad, area, fhi, flo,
-                                                        ctl, nshoot);
+    k_dense_prepare<<<prepare_wgs(np), 256, 0, st>>>(np, unshot, ctl, npatch);
+}
+
+void launch_dense_store_t_dev(float *ff, uint32_t row0, const uint32_t *ctl, uint32_t npatch,
+                              uint32_t npad, const float *area, uint16_t *fhi, uint16_t *flo,
+                              const NextPass &np, const float *unshot, hipStream_t st)
+{
+    const uint32_t nstore = (npatch + 63) / 64;
+    k_dense_store_t<<<nstore + prepare_wgs(np), 256, 0, st>>>(
+        ff, 0u, row0, npatch, npad, area, fhi, flo, ctl, nstore, np, unshot);
 }
 
 void launch_dense_from_f32(const float *src, uint32_t rows, uint32_t row0, uint32_t npatch,

@@ -332,15 +332,16 @@ void launch_dense_store(const float *ff, uint32_t k, uint32_t row0, uint32_t npa
 void launch_dense_store_t(float *ff, uint32_t k, uint32_t row0, uint32_t npatch,
                           uint32_t npad, const float *area, uint16_t *fhi, uint16_t *flo,
                           hipStream_t st);
-// A captured dense build: the next pass's rows (ctl[kCtlDenseBase] advanced
-// by K, from 0 - K before the first; K rows or the rest of the patches) as
-// its shooters, and the transposed store of the pass's rows taken from the
-// device (ctl[kCtlDenseBase], nshoot).
-void launch_iota_next(uint32_t K, uint32_t npatch, uint32_t *ctl, uint32_t *shooters,
-                      uint32_t *nshoot, hipStream_t st);
-void launch_dense_store_t_dev(float *ff, uint32_t K, const uint32_t *ctl, const uint32_t *nshoot,
-                              uint32_t npatch, uint32_t npad, const float *area, uint16_t *fhi,
-                              uint16_t *flo, hipStream_t st);
+// A captured dense build: the first row of its next group of passes
+// (ctl[kCtlDenseBase] advanced by rows); the preparation of its first pass
+// (rows 0 on); the transposed store of the rows from ctl[kCtlDenseBase] + row0
+// on, which also prepares the pass that takes the rows after those.
+void launch_dense_advance(uint32_t rows, uint32_t *ctl, hipStream_t st);
+void launch_dense_prepare(const NextPass &np, const float *unshot, const uint32_t *ctl,
+                          uint32_t npatch, hipStream_t st);
+void launch_dense_store_t_dev(float *ff, uint32_t row0, const uint32_t *ctl, uint32_t npatch,
+                              uint32_t npad, const float *area, uint16_t *fhi, uint16_t *flo,
+                              const NextPass &np, const float *unshot, hipStream_t st);
 void launch_dense_from_f32(const float *src, uint32_t rows, uint32_t row0, uint32_t npatch,
                            uint32_t npad, uint16_t *fhi, uint16_t *flo, hipStream_t st);
 void launch_dense_to_f32(const uint16_t *fhi, const uint16_t *flo, uint32_t rows, uint32_t row0,

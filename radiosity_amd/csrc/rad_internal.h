@@ -34,9 +34,13 @@ struct alignas(16) RasterRec {
     int32_t x[3], y[3];   // snapped face-local window coordinates (1/256 px)
     float dzdx, dzdy, z0; // depth plane anchored at vertex 0
     uint32_t id;          // patch + 1
-    uint32_t sf;          // shooter slot * 8 + face
-    uint32_t pad;
+    uint32_t sf;          // shooter slot << 2 | kSpan bits
+    uint32_t vp;          // the face's viewport origin in the slab, x | y << 16
 };
+// The snapped vertices' span allows 32-bit edge functions in draw_lane32, in
+// draw_wave32 (kLane32Span, kWave32Span): found once by the setup, where the
+// tile kernel found it again, and the face's origin, for each tile of a record.
+constexpr uint32_t kSpanLane = 1u, kSpanWave = 2u;
 static_assert(sizeof(RasterRec) == 48, "RasterRec layout");
 
 // Counters used by one pass (reset by the clear kernel).

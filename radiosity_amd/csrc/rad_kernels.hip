@@ -252,8 +252,9 @@ __device__ static inline int place_tri(const SV &a, const SV &b, const SV &c, ui
     }
     RasterRec rr;
     make_record(a, b, c, area2, id, rr);
-    rr.sf = s * 8u + (uint32_t)face;
-    rr.pad = 0u;
+    rr.sf = s << 2 | (span_within(rr, kLane32Span) ? kSpanLane : 0u) |
+            (span_within(rr, kWave32Span) ? kSpanWave : 0u);
+    rr.vp = (uint32_t)(fv.vpx & 0xFFFF) | (uint32_t)fv.vpy << 16;
     // bbox in texel coordinates of the hemicube slab
     int32_t tx0 = fv.vpx + ix0, tx1 = fv.vpx + ix1, ty0 = fv.vpy + iy0, ty1 = fv.vpy + iy1;
     bc.recs[p.r] = rr;
@@ -888,7 +889,7 @@ __device__ static const uint32_t *whole_list(ConstFacts f,
     }
     const uint32_t nsp = min((uint32_t)f->nspill, (uint32_t)f->spill_cap);
     for (uint32_t q = me; q < nsp; q += kTileThreads)
-        if ((recs[f->spill_base + q].sf >> 3) == s)
+        if ((recs[f->spill_base + q].sf >> 2) == s)
             take(f->spill_base + q);
     __syncthreads();
     if (me == 0)
@@ -974,7 +975,6 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
         oy += (int32_t)((quad >> 1) << tshift);
     }
     const uint32_t T = 1u << tshift, TT = T * T;
-    const int32_t Wi = (int32_t)W;
     const uint32_t me = threadIdx.x;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(me >> 6);
     constexpr uint32_t kNoRec = ~0u;
@@ -1025,8 +1025,8 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
                 // touches other quadrants only
             } else if (area <= small_px) {
                 const RasterRec r = recs[ri];
-                FaceView fv = face_view(Wi, (int)(r.sf & 7u));
-                draw_lane(r, fv.vpx, fv.vpy, ax0, ax1, ay0, ay1, ox, oy, tshift, tk, ph, nph);
+                draw_lane(r, r.sf & kSpanLane, (int32_t)(int16_t)r.vp, (int32_t)(r.vp >> 16), ax0,
+                          ax1, ay0, ay1, ox, oy, tshift, tk, ph, nph);
             } else if (ph == 0) {
                 const uint32_t q = atomicAdd(&nbig, 1u);
                 perm[q] = ri;
@@ -1044,15 +1044,13 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
             const int32_t ax1 = min((int32_t)((bb >> 32) & 0xFFFFu), ox + (int32_t)T - 1);
             const int32_t ay0 = max((int32_t)((bb >> 16) & 0xFFFFu), oy);
             const int32_t ay1 = min((int32_t)(bb >> 48), oy + (int32_t)T - 1);
-            FaceView fv = face_view(Wi, (int)(rb.sf & 7u));
-            const int32_t xspan = max(rb.x[0], max(rb.x[1], rb.x[2])) - min(rb.x[0], min(rb.x[1], rb.x[2]));
-            const int32_t yspan = max(rb.y[0], max(rb.y[1], rb.y[2])) - min(rb.y[0], min(rb.y[1], rb.y[2]));
-            if (xspan <= kWave32Span && yspan <= kWave32Span) {
-                draw_wave32(rb, fv.vpx, fv.vpy, ax0, ax1, ay0, ay1, ox, oy, tshift, tk);
+            const int32_t vpx = (int32_t)(int16_t)rb.vp, vpy = (int32_t)(rb.vp >> 16);
+            if (__builtin_amdgcn_readfirstlane(rb.sf) & kSpanWave) {
+                draw_wave32(rb, vpx, vpy, ax0, ax1, ay0, ay1, ox, oy, tshift, tk);
             } else {
                 Edges e;
                 make_edges(rb.x, rb.y, e);
-                draw_wave(rb, e, fv.vpx, fv.vpy, ax0, ax1, ay0, ay1, ox, oy, tshift, tk);
+                draw_wave(rb, e, vpx, vpy, ax0, ax1, ay0, ay1, ox, oy, tshift, tk);
             }
         }
         ri = rnext;

@@ -581,6 +581,13 @@ __device__ static inline void draw_wave(const RasterRec &r, const Edges &e, int3
     }
 }
 
+// 1 for an edge that owns its pixels (A > 0, or A == 0 and B < 0), else 0:
+// the sign of B - 2^16 A, for |A| and |B| below 2^15.
+__device__ static inline int32_t edge_bias(int32_t A, int32_t B)
+{
+    return (int32_t)((uint32_t)(B - (int32_t)((uint32_t)A << 16)) >> 31);
+}
+
 // draw_wave for a record whose snapped vertices span at most 96 pixels in x
 // and in y (kWave32Span subpixels): every pixel a lane visits, the 8 x 8
 // blocks' overshoot past the bbox included, lies within 16 pixels of the
@@ -600,8 +607,7 @@ __device__ static inline void draw_wave32(const RasterRec &r, int32_t vpx, int32
     for (int k = 0; k < 3; ++k) {
         const int q = k == 2 ? 0 : k + 1;
         const int32_t A = r.y[k] - r.y[q], B = r.x[q] - r.x[k];
-        const int32_t bias = (A > 0 || (A == 0 && B < 0)) ? 1 : 0;
-        er[k] = __mul24(A, px0 - r.x[k]) + __mul24(B, py0 - r.y[k]) + bias - 1;
+        er[k] = __mul24(A, px0 - r.x[k]) + __mul24(B, py0 - r.y[k]) + edge_bias(A, B) - 1;
         sx[k] = A * (8 * kSub);
         sy[k] = B * (8 * kSub);
     }
@@ -667,10 +673,9 @@ __device__ static inline void draw_lane32(const RasterRec &r, int32_t vpx, int32
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         int q = k == 2 ? 0 : k + 1;
-        int32_t A = r.y[k] - r.y[q], B = r.x[q] - r.x[k];
-        int32_t bias = (A > 0 || (A == 0 && B < 0)) ? 1 : 0;
+        const int32_t A = r.y[k] - r.y[q], B = r.x[q] - r.x[k];
         // E(p) = A (p.x - x_k) + B (p.y - y_k); inside iff E + bias - 1 >= 0
-        v[k] = __mul24(A, px0 - r.x[k]) + __mul24(B, py0 - r.y[k]) + bias - 1;
+        v[k] = __mul24(A, px0 - r.x[k]) + __mul24(B, py0 - r.y[k]) + edge_bias(A, B) - 1;
         dA[k] = A * kSub;
         dB[k] = B * kSub * (int32_t)nph;
     }
@@ -700,12 +705,12 @@ __device__ static inline void draw_lane32(const RasterRec &r, int32_t vpx, int32
     }
 }
 
-__device__ static inline void draw_lane(const RasterRec &r, int32_t vpx, int32_t vpy,
+__device__ static inline void draw_lane(const RasterRec &r, bool narrow, int32_t vpx, int32_t vpy,
                                         int32_t ax0, int32_t ax1, int32_t ay0, int32_t ay1,
                                         int32_t ox, int32_t oy, uint32_t tshift, uint64_t *tk,
                                         uint32_t ph, uint32_t nph)
 {
-    if (!span_within(r, kLane32Span)) {
+    if (!narrow) {
         if (ph != 0)
             return; // phase 0 draws these (rare) records whole
         Edges e;

@@ -125,22 +125,24 @@ static bool use_direct(const rad_ctx *c, uint32_t k, uint32_t *T)
 }
 
 // The in-lane triangle limit of a pass over k slots where none was chosen.
-// Passes of up to 3 shooters (tiles of 16, or drawn directly) last as long as
-// a tile's slowest chunks, and a lower limit hands more of them to whole
-// wavefronts; at hemicube 128 and below, with more tiles than the GPU holds
-// at once, less divergence pays too.  Time of a pass at 40, 48 and 64 pixels:
-// 200,000 triangles at hemicube 256, 1 shooter 58.9, 61.3, 65.7 us, 2 73.8,
-// 76.2, 79.7, 4 94.8, 92.3, 92.2, 64 323, 318, 318; 60,000 at hemicube 128,
-// 64 shooters (3,072 tiles) 187.1, 187.5, 189.8; 20,000, 32 (1,536 tiles)
-// 95.6, 93.7, 91.5; the dense build over 16,384 patches (3,072 tiles) 27.2,
-// 27.1, 27.8 ms.  Drawn directly: 20,000 triangles at hemicube 256, 1 shooter
-// 28.9, 29.0, 29.5, 6,000 at hemicube 64, 16 shooters 55.2, 54.7, 54.6.
+// Tiles of 16 hold fewer triangles and last as long as their slowest chunks,
+// and a lower limit hands more of those to whole wavefronts; with tiles of 32
+// at hemicube 128 and below, and more of them than the GPU holds at once,
+// less divergence pays too. Time of a pass at 40, 48 and 64 pixels: tiles of
+// 16, 200,000 triangles at hemicube 256, 1 shooter 58.9, 61.3, 65.7 us, 2
+// 73.8, 76.2, 79.7, 8,000 at 128, 8 shooters 54.8 and 63.0 (40, 64); tiles of
+// 32, 200,000, 4 shooters 94.8, 92.3, 92.2, 64 323, 318, 318; 60,000 at
+// hemicube 128, 64 shooters (3,072 tiles) 187.1, 187.5, 189.8; 20,000, 32
+// (1,536 tiles) 95.6, 93.7, 91.5; the dense build over 16,384 patches (3,072
+// tiles) 27.2, 27.1, 27.8 ms. Drawn directly, where lanes without a triangle
+// share the rows of the others, the limit counts a lane's own pixels: 6,000
+// triangles at hemicube 64, 16 shooters 54.0 at 40, 53.3 at 64.
 static uint32_t lane_limit(const rad_ctx *c, uint32_t k)
 {
     if (!c->auto_small)
         return c->small_px;
     if (c->last_direct)
-        return k < 4 ? 40u : c->small_px;
+        return c->small_px;
     if (c->bb.tshift == 4)
         return 40u;
     const bool many = c->bb.tshift == 5 && c->g.W <= 128 && k * c->bb.ntiles > 2048u;

@@ -889,28 +889,35 @@ uint32_t gemm_tiles(uint32_t R)
 #ifndef RAD_GEMM_WVS
 #define RAD_GEMM_WVS 12
 #endif
-// Rows of one workgroup of a product.
-static uint32_t gemm_wg_rows(uint32_t rt, bool split)
+// Rows of one workgroup of a product.  The widest single-half sweep takes 12
+// waves (384 rows), unless 8 give a single round of workgroups: there the
+// CUs are filled by more k slices instead, and the fewer rows a workgroup has
+// the fewer slices, whose planes the update reads.  A solve of 192 columns to
+// 1e-4, 12 and 8 waves: 4,096 patches 1,174 and 1,077 us, 6,144 1,523, 1,399,
+// 8,192 1,862, 1,793, 10,240 (1.25 rounds) 2,351, 2,663, 12,288 2,858, 3,195,
+// 16,384 (two rounds) 4,753, 4,649, 24,576 8,314, 8,894.
+static uint32_t gemm_wg_rows(uint32_t rt, bool split, uint32_t npad, uint32_t S, uint32_t ncu)
 {
     const uint32_t wv = rt >= 4 ? 8u : 4u;
-    return (rt >= 12 && !split ? (uint32_t)RAD_GEMM_WVS : wv) * 32u;
+    const bool wide = rt >= 12 && !split && (npad + 255u) / 256u * S > ncu;
+    return (wide ? (uint32_t)RAD_GEMM_WVS : wv) * 32u;
 }
 
 GemmSplit gemm_split(uint32_t rt, bool split, uint32_t npad, uint32_t S, uint32_t ncu)
 {
-    const uint32_t rows = gemm_wg_rows(rt, split);
+    const uint32_t rows = gemm_wg_rows(rt, split, npad, S, ncu);
     const uint32_t tiles = (npad + rows - 1) / rows, nch = npad >> 6;
     // row tiles whose tiles x S workgroups make whole rounds over the CUs
     // keep S slices; the rest, fewer than ncu / S tiles, get S2 slices
     const uint32_t full = tiles * S / ncu * ncu / S;
     if (full >= tiles || ncu % S != 0)
-        return GemmSplit{S, S, tiles * rows};
+        return GemmSplit{S, S, tiles * rows, rows};
     uint32_t S2 = ncu / (tiles - full);
     if (S2 > nch)
         S2 = nch;
     if (S2 < S)
         S2 = S;
-    return GemmSplit{S, S2, full * rows};
+    return GemmSplit{S, S2, full * rows, rows};
 }
 
 template <int RT>
@@ -924,13 +931,15 @@ static void gemm_rt(bool split, const uint16_t *fhi, const uint16_t *flo, const 
     // two chunks of A in flight for the single-half sweep; the split product
     // already holds both halves of A and X (PF = 2 would cost occupancy)
     constexpr int PFS = RT >= 4 ? RAD_GEMM_PF : 1;
-    const uint32_t rows = gemm_wg_rows(RT, split);
+    const uint32_t rows = ks.rows;
     const uint32_t tiles = (npad + rows - 1) / rows, head = ks.rsplit / rows;
     const uint32_t nwg = head * ks.S + (tiles - head) * ks.S2;
     if (split)
         k_gemm<RT, true, WV, 1><<<nwg, WV * 64, 0, st>>>(fhi, flo, xhi, xlo, npad, ks, yp);
-    else
+    else if (WVS == WV || rows == WVS * 32u)
         k_gemm<RT, false, WVS, PFS><<<nwg, WVS * 64, 0, st>>>(fhi, flo, xhi, xlo, npad, ks, yp);
+    else
+        k_gemm<RT, false, WV, PFS><<<nwg, WV * 64, 0, st>>>(fhi, flo, xhi, xlo, npad, ks, yp);
 }
 
 void launch_gemm(uint32_t rt, bool split, const uint16_t *fhi, const uint16_t *flo,

@@ -355,9 +355,9 @@ uint32_t gemm_tiles(uint32_t R);
 // of npad / S columns, the rows from rsplit on (the row tiles of the last,
 // partial round of workgroups) over S2 slices of about npad / S2 columns,
 // so that round also fills the CUs.  The partial products hold max(S, S2)
-// planes.
+// planes.  rows: of a workgroup.
 struct GemmSplit {
-    uint32_t S, S2, rsplit;
+    uint32_t S, S2, rsplit, rows;
 };
 GemmSplit gemm_split(uint32_t rt, bool split, uint32_t npad, uint32_t S, uint32_t ncu);
 void launch_gemm(uint32_t rt, bool split, const uint16_t *fhi, const uint16_t *flo,

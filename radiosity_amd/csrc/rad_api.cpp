@@ -706,8 +706,9 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     c->bb.nblk = nblk ? nblk : 1;
     c->bb.nz = K <= 4 && (uint64_t)c->bb.nblk * K < kFaceBlocks ? 5u : 1u;
     c->bb.setup_group = 8;
+    const uint32_t groups = nblk < (ntri + 255u) / 256u ? kSetupGroupsPack : kSetupGroups;
     while (c->bb.setup_group > 1 &&
-           (uint64_t)c->bb.nblk * c->bb.nz * K < (uint64_t)kSetupGroups * c->bb.setup_group)
+           (uint64_t)c->bb.nblk * c->bb.nz * K < (uint64_t)groups * c->bb.setup_group)
         c->bb.setup_group /= 2;
     uint64_t regions = (uint64_t)c->bb.nblk * K * c->bb.nz * kRecsPerBlock;
     uint64_t spill = regions / 8 + 65536;

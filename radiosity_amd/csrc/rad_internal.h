@@ -97,6 +97,12 @@ constexpr uint32_t kSplitPack = 32768;
 // hemicube 128: 16,384 triangles 155 us at 8 slots a workgroup (512
 // workgroups), 122 us at 2 (2,048); 200,000 triangles (50,000 pairs) keep 8.
 constexpr uint32_t kSetupGroups = 1200;
+// In a pack neighbouring slots mostly belong to different scenes, so a
+// workgroup reads other triangles for almost every slot, and those beyond a
+// smaller scene's triangles have nothing to do.  32 scenes, 64 slots at
+// hemicube 256, 1,200 against 4,500: 500 to 20,000 triangles 194 and 186 us a
+// pass, 20,000 to 40,000 353, 333; 64 scenes to 60,000, 128 slots 388, 378.
+constexpr uint32_t kSetupGroupsPack = 4500;
 // Blocks of 256 triangles x slots (of at most 4) from which a setup workgroup
 // takes all five faces instead of one: with the faces apart it reads the
 // triangles five times and its exact phase has a fifth of the lanes busy, but

@@ -127,16 +127,19 @@ static bool use_direct(const rad_ctx *c, uint32_t k, uint32_t *T)
 // The in-lane triangle limit of a pass over k slots where none was chosen.
 // Tiles of 16 hold fewer triangles and last as long as their slowest chunks,
 // and a lower limit hands more of those to whole wavefronts; with tiles of 32
-// at hemicube 128 and below, and more of them than the GPU holds at once,
+// at hemicube 128 and below, and in packs (whose scenes mostly have smaller
+// hemicubes than the largest), and more of them than the GPU holds at once,
 // less divergence pays too. Time of a pass at 40, 48 and 64 pixels: tiles of
 // 16, 200,000 triangles at hemicube 256, 1 shooter 58.9, 61.3, 65.7 us, 2
 // 73.8, 76.2, 79.7, 8,000 at 128, 8 shooters 54.8 and 63.0 (40, 64); tiles of
 // 32, 200,000, 4 shooters 94.8, 92.3, 92.2, 64 323, 318, 318; 60,000 at
 // hemicube 128, 64 shooters (3,072 tiles) 187.1, 187.5, 189.8; 20,000, 32
 // (1,536 tiles) 95.6, 93.7, 91.5; the dense build over 16,384 patches (3,072
-// tiles) 27.2, 27.1, 27.8 ms. Drawn directly, where lanes without a triangle
-// share the rows of the others, the limit counts a lane's own pixels: 6,000
-// triangles at hemicube 64, 16 shooters 54.0 at 40, 53.3 at 64.
+// tiles) 27.2, 27.1, 27.8 ms; packs of 32 scenes of 500 to 20,000 177, 177,
+// 184 us, of 20,000 to 40,000 329, 329, 332. Drawn directly, where lanes
+// without a triangle share the rows of the others, the limit counts a lane's
+// own pixels: 6,000 triangles at hemicube 64, 16 shooters 54.0 at 40, 53.3 at
+// 64.
 static uint32_t lane_limit(const rad_ctx *c, uint32_t k)
 {
     if (!c->auto_small)
@@ -145,7 +148,8 @@ static uint32_t lane_limit(const rad_ctx *c, uint32_t k)
         return c->small_px;
     if (c->bb.tshift == 4)
         return 40u;
-    const bool many = c->bb.tshift == 5 && c->g.W <= 128 && k * c->bb.ntiles > 2048u;
+    const bool many = c->bb.tshift == 5 && (c->g.W <= 128 || c->pk.nscene) &&
+                      k * c->bb.ntiles > 2048u;
     return many ? 48u : c->small_px;
 }
 

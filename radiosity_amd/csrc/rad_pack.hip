@@ -22,7 +22,8 @@ namespace rad {
 // packed keys (power bits << 32 | ~index): each wavefront keeps a sorted
 // list, one key per lane, that takes the keys above its k-th, then the lists
 // merge pairwise.  32 rooms of 500-20,000 patches wanting up to 10 shooters:
-// 23 us, where a block maximum per shooter, each over the whole scene
+// 17 us (23 without the bound from the first maxima, whose first batches were
+// sorted whole), where a block maximum per shooter, each over the whole scene
 // again, took 158.  Shooters past the 64th (a scene may ask for up to 256)
 // are still found by rounds of block maxima below the previous key.
 constexpr uint32_t kPackSelThreads = 1024;
@@ -49,7 +50,9 @@ __global__ __launch_bounds__(kPackSelThreads) void k_pack_select(
     const int kl = (int)(k < 64u ? k : 64u);
     uint64_t top = 0, thr = 0; // thr: the list's kl-th key
     constexpr int kLoads = 4; // batches of a wavefront loaded at once
-    for (uint32_t b = pb + (uint32_t)w * 64u; b < pe; b += kLoads * kPackSelThreads) {
+    constexpr uint32_t kStep = kLoads * kPackSelThreads;
+    uint64_t key[kLoads];
+    auto load = [&](uint32_t b) {
         float u0[kLoads], u1[kLoads], u2[kLoads], ar[kLoads];
 #pragma unroll
         for (int q = 0; q < kLoads; ++q) {
@@ -65,10 +68,47 @@ __global__ __launch_bounds__(kPackSelThreads) void k_pack_select(
         for (int q = 0; q < kLoads; ++q) {
             const uint32_t j = b + (uint32_t)q * kPackSelThreads + (uint32_t)lane;
             num += (double)ar[q] * ((double)u0[q] + (double)u1[q] + (double)u2[q]);
-            const uint64_t key = key_of(ar[q] * (u0[q] + u1[q] + u2[q]), j);
-            if (__ballot(key > thr))
-                wave_take_desc(top, thr, key, kl);
+            key[q] = key_of(ar[q] * (u0[q] + u1[q] + u2[q]), j);
         }
+    };
+    uint32_t b = pb + (uint32_t)w * 64u;
+    load(b);
+    // The k-th largest of the wavefronts' first maxima bounds the k-th largest
+    // key from below, so even the first batches bring few keys to insert.
+    uint64_t low = 0;
+    if (kl > 0 && kl <= (int)NW) {
+        uint64_t m = key[0];
+#pragma unroll
+        for (int q = 1; q < kLoads; ++q)
+            m = key[q] > m ? key[q] : m;
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint64_t v = __shfl_xor(m, o, 64);
+            m = v > m ? v : m;
+        }
+        if (lane == 0)
+            wl[0][w] = m;
+        __syncthreads();
+        const uint64_t mine = lane < (int)NW ? wl[0][lane] : 0ull;
+        int above = 0;
+#pragma unroll
+        for (int q = 0; q < (int)NW; ++q)
+            above += lane_read_u64(mine, q) > mine ? 1 : 0;
+        // (keys differ; zeros, if any, are below every bound)
+        const uint64_t at = __ballot(lane < (int)NW && mine != 0ull && above == kl - 1);
+        if (at)
+            low = lane_read_u64(mine, __ffsll((long long)at) - 1) - 1ull;
+        thr = low;
+    }
+    for (; b < pe;) {
+#pragma unroll
+        for (int q = 0; q < kLoads; ++q)
+            if (__ballot(key[q] > thr)) {
+                wave_take_desc(top, thr, key[q], kl);
+                thr = thr > low ? thr : low;
+            }
+        b += kStep;
+        if (b < pe)
+            load(b);
     }
     for (int o = 32; o > 0; o >>= 1)
         num += __shfl_down(num, o, 64);

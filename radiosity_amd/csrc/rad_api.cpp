@@ -399,8 +399,8 @@ int one_pass(rad_ctx *c, bool do_select, size_t evbase, bool chain_in = false,
 }
 
 // The bins' lists: room for 16 times the records per bin of a scene spread
-// evenly over the tiles, within 4 GiB in all.  A fuller bin is drawn from its
-// slot's records without a list (k_tile_raster), so the size is no limit.
+// evenly over the tiles, within 4 GiB in all.  A fuller bin's workgroup makes
+// its list in the pool (whole_list), so the size is no limit.
 int bin_lists(rad_ctx *c)
 {
     const uint64_t ntri = (uint64_t)c->bb.nblk * 256;
@@ -706,7 +706,7 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
         HIPCHK(c, hipMemset(c->ffq, 0, K * rowlen * 8));
     }
     // records: one region of kRecsPerBlock per (setup block, shooter) plus a
-    // spill region; bin entries: three per record slot
+    // spill region; bin entries in all: two per record slot
     c->bb.nblk = nblk ? nblk : 1;
     c->bb.nz = K <= 4 && (uint64_t)c->bb.nblk * K < kFaceBlocks ? 5u : 1u;
     c->bb.setup_group = 8;

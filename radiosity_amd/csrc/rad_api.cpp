@@ -205,7 +205,7 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
                                 c->pk.slot_tbeg, c->pk.slot_tcnt, c->pk.slot_w, st);
         else if (j == 1)
             launch_bin(c->g, s0, s1, h, c->tri, c->tri_patch, c->ntri, c->mvp, c->bb, c->counters,
-                       c->pk.slot_w, st);
+                       c->pk.slot_w, fq, st);
         else
             launch_tile(c->g, s0, s1, h, c->nshoot, c->bb, small_px, ids, depth,
                         c->pk.slot_w ? c->pk.dffs : c->dff, c->rowlen, c->pk.slot_pbeg,
@@ -1643,7 +1643,7 @@ int rad_debug_bins(rad_ctx *c, uint32_t *out, uint32_t *ntiles, uint32_t *tile_p
                             c->nshoot, c->bb, cnt, c->pk.slot_tbeg, c->pk.slot_tcnt, c->pk.slot_w,
                             c->st);
         launch_bin(c->g, 0, c->last_k, 0, c->tri, c->tri_patch, c->ntri, c->mvp, c->bb, cnt,
-                   c->pk.slot_w, c->st);
+                   c->pk.slot_w, false, c->st);
         const hipError_t e = hipStreamSynchronize(c->st);
         dfree(cnt);
         HIPCHK(c, e);

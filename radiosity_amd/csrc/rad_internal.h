@@ -209,6 +209,7 @@ void launch_clear(uint32_t K, uint32_t *bin_count, uint32_t ntiles, float *ff, u
 // of the bins, clipped triangles), tile (LDS depth test; out_ids != null
 // writes the item buffer, ff or ffq != null reduces into F rows and hits).  h selects the counter block,
 // spill region and clip queue (0, or 1 for the second half of a split pass).
+// fixed: the tiles that follow go to the fixed-point rows ffq.
 void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h,
                          const float *tri, const float4 *tsph, const float4 *tback,
                          const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const uint32_t *nshoot,
@@ -217,7 +218,7 @@ void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h
 void launch_tri_sphere(const float *tri, uint32_t ntri, float4 *sph, float4 *back, hipStream_t st);
 void launch_bin(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const float *tri,
                 const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const BinBuffers &bb,
-                uint32_t *counters, const uint32_t *slot_w, hipStream_t st);
+                uint32_t *counters, const uint32_t *slot_w, bool fixed, hipStream_t st);
 void launch_tile(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const uint32_t *nshoot,
                  const BinBuffers &bb, uint32_t small_px, uint32_t *out_ids, float *out_depth,
                  const float *dff, uint32_t rowlen, const uint32_t *slot_pbeg, float *ff,

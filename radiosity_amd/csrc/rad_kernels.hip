@@ -1193,26 +1193,29 @@ void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h
 // How many of a launch's nb bins may be drawn as quadrants, those of
 // kSplitRecs records or more: a launch whose bins are all resident at once, or
 // nearly, lasts as long as its fullest bin.  A pass of 64 shooters over 33,000
-// triangles at hemicube 128 (3,072 bins) takes 85.1 us instead of 88.4 and one
-// of 32 over 20,000, deterministic (1,536 bins), 109 instead of 114.  With
+// triangles at hemicube 128 (3,072 bins) takes 85.1 us instead of 88.4.  With
 // several times more bins (12,288: 64 shooters at hemicube 256) the largest,
 // started first, end before the others do, and with one hemicube (192) the
 // quadrants' reading of the whole list cost 1 %.  From 1,024 records on, or
 // for more than 1 bin in 16, a pass of 25 shooters over 16,000 triangles lost
 // up to 1 %.
-static uint32_t split_cap(const BinBuffers &bb, uint32_t nb)
+// None with the fixed-point rows: which of the fullest bins become quadrants
+// depends on the order of atomics (and on clipped triangles binned meanwhile),
+// and a quadrant sums the runs of 16 texels in float where a whole tile sums
+// those of 32, so the rows' bits would change from run to run.
+static uint32_t split_cap(const BinBuffers &bb, uint32_t nb, bool fixed)
 {
-    return bb.tshift == 5 && nb > 512u && nb <= 4096u ? nb / 16u : 0u;
+    return !fixed && bb.tshift == 5 && nb > 512u && nb <= 4096u ? nb / 16u : 0u;
 }
 
 void launch_bin(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const float *tri,
                 const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const BinBuffers &bb,
-                uint32_t *counters, const uint32_t *slot_w, hipStream_t st)
+                uint32_t *counters, const uint32_t *slot_w, bool fixed, hipStream_t st)
 {
     const uint32_t b0 = s0 * bb.ntiles, nb = (s1 - s0) * bb.ntiles;
     const uint32_t norder = (nb + 256u * kOrderPer - 1) / (256u * kOrderPer);
     k_order_clip<<<norder + bb.clip_blocks, 256, 0, st>>>(
-        norder, nb, b0, split_cap(bb, nb), bb.order + b0, bb.nbins, g.W, tri, tri_patch, ntri, mvp,
+        norder, nb, b0, split_cap(bb, nb, fixed), bb.order + b0, bb.nbins, g.W, tri, tri_patch, ntri, mvp,
         bin_ctx(bb, h, counters), bb.blk_nrec, bb.nblk * bb.nz,
         bb.pool + (size_t)h * bb.ent_cap, bb.ent_cap, slot_w);
 }
@@ -1226,7 +1229,7 @@ void launch_tile(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const 
 {
     const uint32_t nb = (s1 - s0) * bb.ntiles;
     const uint32_t *order = bb.order + (size_t)s0 * bb.ntiles;
-    const uint32_t nwg = nb + 3u * split_cap(bb, nb);
+    const uint32_t nwg = nb + 3u * split_cap(bb, nb, ffq != nullptr);
     uint32_t *ctr = counters + h * kCntN;
     const BinFacts *facts = reinterpret_cast<const BinFacts *>(ctr + kCntFacts);
     if (ffq)

@@ -589,7 +589,7 @@ void rad_destroy(rad_ctx *c)
                     c->trip_e,
                     c->mvp,  c->snap,     c->shooters, c->nshoot, c->counters, c->ctl, c->sel,
                     c->resid, c->bb.recs, c->bb.count,
-                    c->bb.list, c->bb.blk_nrec, c->bb.bbox, c->bb.clipq, c->cand, c->parts, c->bb.order,
+                    c->bb.list, c->bb.pool, c->bb.blk_nrec, c->bb.bbox, c->bb.clipq, c->cand, c->parts, c->bb.order,
                     c->fhi,  c->flo,      c->pk.sc_tbeg, c->pk.sc_pbeg, c->pk.sc_slots,
                     c->pk.sc_slot_beg, c->pk.sc_nsel, c->pk.sc_done, c->pk.sc_den, c->pk.sc_res,
                     c->pk.sc_shot,

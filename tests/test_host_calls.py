@@ -1,0 +1,59 @@
+"""What the host code allocates and launches, on the CPU: it runs against a
+stand-in for the HIP runtime (device_double.cpp) that counts allocations and
+names launches."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="session")
+def on_double(tmp_path_factory):
+    """Runs a program against the stand-in, in a process of its own: D is the
+    stand-in, R the package, np numpy."""
+    so = str(tmp_path_factory.mktemp("double") / "device_double.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I",
+                    "/opt/rocm/include", os.path.join(ROOT, "tests", "device_double.cpp"), "-o", so],
+                   check=True)
+
+    def run(code):
+        head = f"""
+            import ctypes as C, numpy as np
+            D = C.CDLL({so!r}, mode=C.RTLD_GLOBAL)
+            D.double_live.restype = D.double_live_bytes.restype = C.c_size_t
+            D.double_limit.argtypes = [C.c_size_t]
+            import radiosity_amd as R
+            """
+        p = subprocess.run([sys.executable, "-c", textwrap.dedent(head) + textwrap.dedent(code)],
+                           cwd=ROOT, capture_output=True, text=True, timeout=300)
+        assert p.returncode == 0, p.stdout + p.stderr
+
+    return run
+
+
+def test_close_returns_every_allocation(on_double):
+    """Plain scenes, a replaced scene, a pack, the deterministic rows, a dense
+    matrix with its solve, a graph."""
+    on_double("""
+        def boxes(n, seed=3):
+            return R.Scene.boxes(nboxes=4, room=(5.0, 3.0, 5.0), target_tris=n, nlights=2, seed=seed)
+        for kw in (dict(hemicube=16, hemicubes=1), dict(hemicube=64, hemicubes=16, graph_passes=4)):
+            s = R.Solver(**kw)
+            s.set_deterministic(True)
+            s.upload(boxes(600))
+            s.upload(boxes(3000))
+            s.prepare()
+            s.step(9)
+            s.autotune(1)
+            s.dense_upload(np.zeros((s.npatch, s.npatch), np.float32))
+            s.dense_apply(np.zeros((3, s.npatch), np.float32))
+            s.pack_upload([boxes(300 + 200 * i, i + 1) for i in range(3)], [1, 1, 1])
+            s.step(2)
+            assert D.double_live() > 30
+            s.close()
+            assert D.double_live() == 0, (kw, D.double_live(), D.double_live_bytes())
+        """)

@@ -599,8 +599,10 @@ __global__ __launch_bounds__(256) void k_raster_setup(uint32_t W, const float *_
 //    shooter's own plane (floor under a floor patch) before any per-face work;
 //  - a face whose frustum (90 degree pyramid around its axis, near 0.01)
 //    misses the sphere by more than a margin;
-//  - a triangle (of one face only, by the last test) of area A whose plane the eye lies at least D > 0 behind:
-//    with depths in [wmin, wmax] it projects to a clockwise area of at least
+//  - a triangle (of one face only, by the last test over all five faces, also
+//    where the workgroup looks at one: on a second face it would be nearer and
+//    wider than the bounds below) of area A whose plane the eye lies at least
+//    D > 0 behind: with depths in [wmin, wmax] it projects to a clockwise area of at least
 //    (W/2)^2 2 A D / wmax^3 square pixels.  Snapping and rounding move a
 //    vertex by at most delta pixels per axis, which changes the area by at
 //    most 5.7 delta L + 8 delta^2 for a longest projected edge
@@ -664,10 +666,12 @@ __device__ static uint32_t cull_faces(const float *__restrict__ sm, const float 
     // whose coordinate comes within the margin of it
     uint32_t mask = (fabsf(pb) >= T ? (pb > 0.0f ? 1u : 2u) : 0u) |
                     (fabsf(pc) >= T ? (pc > 0.0f ? 4u : 8u) : 0u) | (pa >= T ? 16u : 0u);
+    // (of one face whichever faces this workgroup looks at)
+    const bool one = (mask & (mask - 1u)) == 0u;
     mask &= faces;
     const float l1 = fabsf(cx) + fabsf(cy) + fabsf(cz);
     const float db = fmaf(-4e-6f * l1, back.w, fmaf(cz, back.z, fmaf(cy, back.y, cx * back.x)));
-    if (db > 0.0f && (mask & (mask - 1u)) == 0u) {
+    if (db > 0.0f && one) {
         const float wmin = far - rho - mq, wmax = far + rho + mq;
         const float S = __builtin_amdgcn_fmed3f(fabsf(pa), fabsf(pb), fabsf(pc)) + rho;
         const float em = 2e-6f * (fabsf(ex) + fabsf(ey) + fabsf(ez));

@@ -32,10 +32,16 @@ namespace rad {
 //     when the triangles do not share N within 0.5 %), and the smallest
 //     area / longest edge of a triangle
 //  2  unit normal N on the side the triangles are drawn from, and the
-//     smallest area of a triangle
+//     smallest area of a triangle (0 when their normals are not within kTilt
+//     of N)
 // In a pack the clusters of scene s start at tbeg / 64 + s, which leaves
 // room for a partly filled last cluster in every scene.
 constexpr uint32_t kCluWords = 15; // 16-byte words per cluster
+// Sine of the largest angle between N and the normals of a run taken for flat:
+// well above the rounding of a plane's vertices (about 1e-7 of their
+// coordinates over a triangle's height), and too small to cost the back-face
+// test of a run anything (it asks for more than a milliradian).
+constexpr float kTilt = 2.5e-4f;
 
 template <int N, typename Op> __device__ static inline float lanes_red(float x, Op op)
 {
@@ -64,6 +70,9 @@ __device__ static inline void run_bounds(const float (&v)[3][3], const float (&n
     for (int c = 0; c < 3; ++c)
         nn[c] = __shfl(n[c], (int)((threadIdx.x & 63u) & ~(uint32_t)(N - 1)), 64);
     const float same = lanes_red<N>(n[0] * nn[0] + n[1] * nn[1] + n[2] * nn[2], mn);
+    const float kx = n[1] * nn[2] - n[2] * nn[1], ky = n[2] * nn[0] - n[0] * nn[2],
+                kz = n[0] * nn[1] - n[1] * nn[0];
+    const float tilt = lanes_red<N>(kx * kx + ky * ky + kz * kz, mx);
     float eps = 0.0f;
 #pragma unroll
     for (int k = 0; k < 3; ++k)
@@ -75,7 +84,7 @@ __device__ static inline void run_bounds(const float (&v)[3][3], const float (&n
     if (write) {
         out[0] = make_float4(ctr[0], ctr[1], ctr[2], half[0]);
         out[1] = make_float4(half[1], half[2], same >= 0.995f ? eps : -1.0f, q);
-        out[2] = make_float4(nn[0], nn[1], nn[2], area);
+        out[2] = make_float4(nn[0], nn[1], nn[2], tilt <= kTilt * kTilt ? area : 0.0f);
     }
 }
 
@@ -217,13 +226,15 @@ __device__ static inline float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x)
 //    1e-5 W / 2 << 0.5 pixel of the horizon, where the nearest kept pixel
 //    centre is half a pixel away (in the front face: nearer than the near
 //    plane).  This drops the shooter's own wall.
-//  - the eye lies at least D > 0 behind the run's plane: a triangle of
-//    area A with depths in [wmin, wmax] projects to a clockwise area of at
-//    least (W/2)^2 2 A D / wmax^3 square pixels.  Snapping and rounding move
-//    a vertex by at most delta pixels per axis, which changes the area by at
-//    most 5.7 delta L + 8 delta^2 for a longest projected edge
-//    L <= sqrt2 (W/2) edge (1 + kappa) / wmin, kappa the largest |x / w|; the
-//    two tests ask twice that, so the snapped triangle is clockwise too.
+//  - the eye lies at least D > 0 behind the plane of every triangle of a flat
+//    run (behind the run's plane, less what normals kTilt off N make of the
+//    distance to a vertex): a triangle of area A with depths in [wmin, wmax]
+//    projects to a clockwise area of at least (W/2)^2 2 A D / wmax^3 square
+//    pixels.  Snapping and rounding move a vertex by at most delta pixels per
+//    axis, which changes the area by at most 5.7 delta L + 8 delta^2 for a
+//    longest projected edge L <= sqrt2 (W/2) edge (1 + kappa) / wmin, kappa
+//    the largest |x / w|; the two tests ask twice that, so the snapped triangle
+//    is clockwise too.
 __device__ static inline bool run_in_tile(const TileView &v, const float4 *__restrict__ b,
                                           float halfW)
 {
@@ -248,7 +259,7 @@ __device__ static inline bool run_in_tile(const TileView &v, const float4 *__res
     const float hmax = pa + cn * eps + fsqrt(kx * kx + ky * ky + kz * kz) * rho;
     if (rho < 4.0f * dmin && hmax < fminf(2e-6f * dmin, 0.0098f))
         return false;
-    const float D = dx * b2.x + dy * b2.y + dz * b2.z - eps - 1e-6f * l1;
+    const float D = dx * b2.x + dy * b2.y + dz * b2.z - eps - 1e-6f * l1 - kTilt * (dl + rho);
     const float Z = dx * w[0] + dy * w[1] + dz * w[2];
     const float hw = b0.w * fabsf(w[0]) + b1.x * fabsf(w[1]) + b1.y * fabsf(w[2]);
     const float wmin = Z - hw - m, wmax = Z + hw + m;

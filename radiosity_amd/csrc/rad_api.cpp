@@ -706,7 +706,7 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
         HIPCHK(c, hipMemset(c->ffq, 0, K * rowlen * 8));
     }
     // records: one region of kRecsPerBlock per (setup block, shooter) plus a
-    // spill region; bin entries in all: two per record slot
+    // spill region
     c->bb.nblk = nblk ? nblk : 1;
     c->bb.nz = K <= 4 && (uint64_t)c->bb.nblk * K < kFaceBlocks ? 5u : 1u;
     c->bb.setup_group = 8;
@@ -714,18 +714,24 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     while (c->bb.setup_group > 1 &&
            (uint64_t)c->bb.nblk * c->bb.nz * K < (uint64_t)groups * c->bb.setup_group)
         c->bb.setup_group /= 2;
-    uint64_t regions = (uint64_t)c->bb.nblk * K * c->bb.nz * kRecsPerBlock;
-    uint64_t spill = regions / 8 + 65536;
-    if (regions + kCntBlocks * spill > (1ull << 31))
+    const uint64_t regions = (uint64_t)c->bb.nblk * K * c->bb.nz * kRecsPerBlock;
+    // What a pass may hold is the same whatever the launch shapes: it counts a
+    // region per face for up to four shooters.
+    const uint64_t slots = (uint64_t)c->bb.nblk * K * (K <= 4 ? 5u : 1u) * kRecsPerBlock;
+    const uint64_t spill = slots / 8 + 65536;
+    if (slots + kCntBlocks * spill > (1ull << 31))
         return fail(c, RAD_E_LIMIT, "scene too large for the rasterizer record regions");
     c->bb.spill_base = (uint32_t)regions;
-    c->bb.spill_cap = (uint32_t)spill;
+    // a region all five faces share takes 768 of the up to 1,280 records of
+    // its triangles, which five regions have room for
+    const uint64_t shared = K <= 4 && c->bb.nz == 1 ? (uint64_t)c->bb.nblk * K * 512 : 0;
+    c->bb.spill_cap = (uint32_t)(spill + shared);
     c->bb.clip_cap = (uint32_t)(spill / 2);
     c->bb.clip_blocks = 128;
-    uint64_t went = 2 * (regions + spill);
+    const uint64_t went = 2 * (slots + spill);
     c->bb.ent_cap = (uint32_t)(went > 0xF0000000ull ? 0xF0000000ull : went);
     // each half of a split pass has its own spill region and clipping queue
-    const uint64_t nrec = regions + kCntBlocks * spill;
+    const uint64_t nrec = regions + (uint64_t)kCntBlocks * c->bb.spill_cap;
     if ((rc = dalloc(c, &c->bb.recs, nrec)) || (rc = dalloc(c, &c->bb.bbox, nrec)) ||
         (rc = bin_lists(c)) || (rc = dalloc(c, &c->bb.pool, (size_t)kCntBlocks * c->bb.ent_cap)) ||
         (rc = dalloc(c, &c->bb.blk_nrec, (size_t)c->bb.nblk * K * c->bb.nz)) ||

@@ -1,0 +1,34 @@
+"""Scenes near the rasterizer's capacities: the launch shapes and tile sides
+that the library takes by itself refuse none that others take."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(rad, tri, eyes):
+    n = len(eyes)
+    frame = np.concatenate([eyes, np.tile([[0.0, 0, 1, 0, 1, 0]], (n, 1))], 1)
+    one = np.ones((n, 3), np.float32)
+    return rad.Scene(tri.astype(np.float32), np.sort(np.arange(len(tri)) % n), frame, 0.5 * one,
+                     np.ones(n), one, 0 * one)
+
+
+def test_many_triangles_to_clip(rad):
+    """One shooter, 100,000 triangles (a workgroup takes all five faces of
+    them), 70,000 of which cross the near plane."""
+    rng = np.random.default_rng(2)
+    c = np.concatenate([rng.uniform(-0.002, 0.002, (70000, 1, 2)), np.full((70000, 1, 1), 0.01)], 2)
+    d = rng.uniform(-8e-4, 8e-4, (70000, 3, 3))
+    d[:, 0, 2], d[:, 1, 2] = -6e-4, 6e-4
+    far = rng.uniform(-4, 4, (30000, 1, 3)) + rng.uniform(-0.05, 0.05, (30000, 3, 3))
+    sc = _scene(rad, np.concatenate([c + d, far]), np.zeros((1, 3)))
+    print("triangles to clip", flush=True)
+    s = rad.Solver(hemicube=64, hemicubes=1)
+    s.upload(sc)
+    ids = s.render([0])
+    assert s.debug_counters()["clip"] >= 70000
+    assert np.array_equal(ids, O.render_hemicube(64, sc.tri, sc.tri_patch, sc.frame[0]))
+

@@ -716,7 +716,9 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
         c->bb.setup_group /= 2;
     const uint64_t regions = (uint64_t)c->bb.nblk * K * c->bb.nz * kRecsPerBlock;
     // What a pass may hold is the same whatever the launch shapes: it counts a
-    // region per face for up to four shooters.
+    // region per face for up to four shooters, and a tile side of 16 taken
+    // where a context of K shooters has tiles of 32 makes up to four times the
+    // entries.
     const uint64_t slots = (uint64_t)c->bb.nblk * K * (K <= 4 ? 5u : 1u) * kRecsPerBlock;
     const uint64_t spill = slots / 8 + 65536;
     if (slots + kCntBlocks * spill > (1ull << 31))
@@ -728,7 +730,7 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     c->bb.spill_cap = (uint32_t)(spill + shared);
     c->bb.clip_cap = (uint32_t)(spill / 2);
     c->bb.clip_blocks = 128;
-    const uint64_t went = 2 * (slots + spill);
+    const uint64_t went = (c->auto_side && K >= 4 && side == 16 ? 8 : 2) * (slots + spill);
     c->bb.ent_cap = (uint32_t)(went > 0xF0000000ull ? 0xF0000000ull : went);
     // each half of a split pass has its own spill region and clipping queue
     const uint64_t nrec = regions + (uint64_t)kCntBlocks * c->bb.spill_cap;

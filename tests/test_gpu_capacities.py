@@ -32,3 +32,28 @@ def test_many_triangles_to_clip(rad):
     assert s.debug_counters()["clip"] >= 70000
     assert np.array_equal(ids, O.render_hemicube(64, sc.tri, sc.tri_patch, sc.frame[0]))
 
+
+def test_entries_of_small_tiles(rad):
+    """Twelve shooters amid 3,000 large triangles: in tiles of 32, the entries
+    fit; in tiles of 16, which the library takes, they are more than that
+    limit."""
+    rng = np.random.default_rng(3)
+    c = rng.normal(size=(3000, 1, 3))
+    c[:, :, 2] = np.abs(c[:, :, 2])
+    c *= rng.uniform(3, 5, (3000, 1, 1)) / np.linalg.norm(c, axis=2, keepdims=True)
+    tri = c + 2.0 * rng.uniform(-1, 1, (3000, 3, 3))
+    n = np.cross(tri[:, 2] - tri[:, 0], tri[:, 1] - tri[:, 0])
+    back = (n * tri.mean(1)).sum(1) > 0  # all of them seen from the middle
+    tri[back] = tri[back][:, [0, 2, 1]]
+    sc = _scene(rad, tri, rng.uniform(-0.1, 0.1, (12, 3)))
+    sh = np.arange(12)
+    out = []
+    for tile in (32, 0):
+        print(f"entries, tile {tile}", flush=True)
+        s = rad.Solver(hemicube=128, hemicubes=12, tile_px=tile)
+        s.upload(sc)
+        ids = s.render(sh)
+        out.append((ids, s.debug_counters(), s.debug_bins()[1]))
+        s.close()
+    assert out[1][2] == 16 and out[1][1]["entries"] > out[0][1]["entry_cap"]
+    assert np.array_equal(out[0][0], out[1][0])

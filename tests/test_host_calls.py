@@ -62,26 +62,32 @@ def test_close_returns_every_allocation(on_double):
 def test_capacities_of_every_launch_shape(on_double):
     """What a pass may hold (records beyond their regions, entries, triangles to
     clip) counts a region of 768 records for each 256 triangles, shooter and,
-    up to four shooters, face."""
+    up to four shooters, face; four times the entries where a side of 16 was
+    taken for four shooters or more."""
     on_double("""
         def caps(W, K, ntri, tile):
             s = R.Solver(hemicube=W, hemicubes=K, tile_px=tile)
             s.upload(R.Scene(np.zeros((ntri, 9)), np.zeros(ntri), np.eye(3).reshape(1, 9),
                              np.ones((1, 3)), np.ones(1), np.ones((1, 3)), np.ones((1, 3))))
-            c = s.debug_counters()
+            c, (_, side) = s.debug_counters(), s.debug_bins()
             s.close()
-            return c
+            return c, side
+        seen = set()
         for W in (16, 64, 128, 256):
             for K in (1, 3, 4, 5, 12, 32, 64):
                 for ntri in (1, 700, 3000, 24000, 60000, 120000):
                     for tile in (0, 32):
                         if K * ntri > 1000000:
                             continue
-                        c = caps(W, K, ntri, tile)
+                        c, side = caps(W, K, ntri, tile)
                         slots = -(-ntri // 256) * K * (5 if K <= 4 else 1) * 768
                         spill = slots // 8 + 65536
                         entries = 2 * (slots + spill)
+                        if not tile and K >= 4 and side == 16:
+                            entries *= 4
+                        seen.add((tile, K >= 4, side))
                         assert c["clip_cap"] == spill // 2, (W, K, ntri, tile)
                         assert c["spill_cap"] >= spill, (W, K, ntri, tile)
-                        assert c["entry_cap"] >= entries, (W, K, ntri, tile)
+                        assert c["entry_cap"] == entries, (W, K, ntri, tile)
+        assert (0, True, 16) in seen and (0, True, 32) in seen
         """)

@@ -251,7 +251,8 @@ int rad_debug_bins(rad_ctx *ctx, uint32_t *out_or_null, uint32_t *ntiles, uint32
  * earlier pass overflowed.  Capacities: out_caps (optional, 3 entries) gets
  * the spill capacity, the bin-entry capacity and the clip-queue capacity.
  * A large pass renders as two halves, each with these
- * capacities: [3], [5] and [6] are then the fuller half's, [4] the sum. */
+ * capacities: [3], [5] and [6] are then the fuller half's, [4] the sum.  A pass
+ * drawn whole has those of both halves where hemicubes is 16 or more. */
 int rad_debug_counters(rad_ctx *ctx, uint32_t *out8, uint32_t *out_caps_or_null);
 
 /* Diagnostics (no counterpart in the reference): the candidate pool of the

@@ -189,7 +189,7 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
         launch_prepare_clear(k, shooters ? shooters : c->shooters, c->nshoot,
                              frames ? frames : c->frames, c->unshot, c->snap, c->mvp, c->bb.count,
                              c->bb.ntiles, c->ff_dirty ? c->ff : nullptr, hits, rows, c->rowlen,
-                             c->counters, c->bb.ent_cap, c->ctl, c->st);
+                             c->counters, c->ctl, c->st);
     c->ff_dirty = 0;
     record(c, evbase + 2);
     const bool fq = !ids && c->det;
@@ -198,14 +198,15 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
     uint32_t T;
     c->last_direct = use_direct(c, k, &T);
     const uint32_t small_px = lane_limit(c, k);
+    const bool halved = split_render(c, k);
     auto stage = [&](int j, uint32_t s0, uint32_t s1, uint32_t h, hipStream_t st) {
         if (j == 0)
             launch_raster_setup(c->g, s0, s1, h, c->tri, c->tsph, c->tback, c->tri_patch,
                                 c->ntri, c->mvp, c->nshoot, c->bb, c->counters,
-                                c->pk.slot_tbeg, c->pk.slot_tcnt, c->pk.slot_w, st);
+                                c->pk.slot_tbeg, c->pk.slot_tcnt, c->pk.slot_w, !halved, st);
         else if (j == 1)
             launch_bin(c->g, s0, s1, h, c->tri, c->tri_patch, c->ntri, c->mvp, c->bb, c->counters,
-                       c->pk.slot_w, fq, st);
+                       c->pk.slot_w, !halved, fq, st);
         else
             launch_tile(c->g, s0, s1, h, c->nshoot, c->bb, small_px, ids, depth,
                         c->pk.slot_w ? c->pk.dffs : c->dff, c->rowlen, c->pk.slot_pbeg,
@@ -252,7 +253,7 @@ int render_pass(rad_ctx *c, uint32_t k, size_t evbase, uint32_t *ids, float *dep
         d.counters = c->counters;
         d.fblk = d.ff ? c->fblk : nullptr;
         launch_direct(d, T, c->st);
-    } else if (split_render(c, k)) {
+    } else if (halved) {
         HIPCHK(c, hipEventRecord(c->ev_fork, c->st));
         HIPCHK(c, hipStreamWaitEvent(c->st2, c->ev_fork, 0));
         for (int j = 0; j < 3; ++j) {
@@ -291,14 +292,16 @@ int check_overflow(rad_ctx *c)
         return fail(c, RAD_E_HIP, std::string("counters: ") + hipGetErrorString(e));
     for (int h = 0; h < kCntBlocks; ++h) {
         const uint32_t *b = cnt + h * kCntN;
-        if (b[kCntOverflow] || b[kCntEntries] > c->bb.ent_cap || cnt[kCntSticky]) {
+        BinFacts f;
+        memcpy(&f, b + kCntFacts, sizeof(f));
+        if (b[kCntOverflow] || b[kCntEntries] > f.pool_cap || cnt[kCntSticky]) {
             uint32_t zero = 0;
             (void)hipMemcpy(c->counters + kCntSticky, &zero, 4, hipMemcpyHostToDevice);
             return fail(c, RAD_E_LIMIT, "rasterizer bins overflowed (records " +
                                             std::to_string(b[kCntSpill]) + " spilled of " +
-                                            std::to_string(c->bb.spill_cap) + ", entries " +
+                                            std::to_string(f.spill_cap) + ", entries " +
                                             std::to_string(b[kCntEntries]) + " of " +
-                                            std::to_string(c->bb.ent_cap) + ")");
+                                            std::to_string(f.pool_cap) + ")");
         }
     }
     return RAD_OK;
@@ -348,7 +351,7 @@ int one_pass(rad_ctx *c, bool do_select, size_t evbase, bool chain_in = false,
     int rc;
     const NextPass np{c->K,    c->shooters, c->nshoot,   c->frames,
                       c->snap, c->mvp,      c->bb.count, (size_t)c->K * c->bb.ntiles,
-                      c->counters, c->bb.ent_cap};
+                      c->counters};
     bool prepared = chain_in;
     record(c, evbase + 0);
     if (c->pk.nscene) {
@@ -730,8 +733,9 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     c->bb.spill_cap = (uint32_t)(spill + shared);
     c->bb.clip_cap = (uint32_t)(spill / 2);
     c->bb.clip_blocks = 128;
+    c->bb.halves = K >= kSplitMin ? (uint32_t)kCntBlocks : 1u;
     const uint64_t went = (c->auto_side && K >= 4 && side == 16 ? 8 : 2) * (slots + spill);
-    c->bb.ent_cap = (uint32_t)(went > 0xF0000000ull ? 0xF0000000ull : went);
+    c->bb.ent_cap = (uint32_t)(went > kMaxEntries ? kMaxEntries : went);
     // each half of a split pass has its own spill region and clipping queue
     const uint64_t nrec = regions + (uint64_t)kCntBlocks * c->bb.spill_cap;
     if ((rc = dalloc(c, &c->bb.recs, nrec)) || (rc = dalloc(c, &c->bb.bbox, nrec)) ||
@@ -1181,7 +1185,7 @@ static int step_impl(rad_ctx *c, uint32_t passes)
         // them zero again
         if (c->ff_dirty) {
             launch_clear(c->K, c->bb.count, c->bb.ntiles, c->ff, nullptr, c->ff_dirty, c->rowlen,
-                         c->counters, c->bb.ent_cap, c->st);
+                         c->counters, c->st);
             if ((rc = check_launch(c, "clear")))
                 return rc;
             c->ff_dirty = 0;
@@ -1645,13 +1649,12 @@ int rad_debug_bins(rad_ctx *c, uint32_t *out, uint32_t *ntiles, uint32_t *tile_p
         int rc;
         if ((rc = dalloc(c, &cnt, kCntN * kCntBlocks)))
             return rc;
-        launch_clear(c->K, c->bb.count, c->bb.ntiles, nullptr, nullptr, 0, 0, cnt, c->bb.ent_cap,
-                     c->st);
+        launch_clear(c->K, c->bb.count, c->bb.ntiles, nullptr, nullptr, 0, 0, cnt, c->st);
         launch_raster_setup(c->g, 0, c->last_k, 0, c->tri, c->tsph, c->tback, c->tri_patch, c->ntri, c->mvp,
                             c->nshoot, c->bb, cnt, c->pk.slot_tbeg, c->pk.slot_tcnt, c->pk.slot_w,
-                            c->st);
+                            true, c->st);
         launch_bin(c->g, 0, c->last_k, 0, c->tri, c->tri_patch, c->ntri, c->mvp, c->bb, cnt,
-                   c->pk.slot_w, false, c->st);
+                   c->pk.slot_w, true, false, c->st);
         const hipError_t e = hipStreamSynchronize(c->st);
         dfree(cnt);
         HIPCHK(c, e);
@@ -1798,15 +1801,14 @@ static int dense_build_graph(rad_ctx *c, uint32_t npass)
 {
     if (c->ff_dirty) {
         launch_clear(c->K, c->bb.count, c->bb.ntiles, c->ff, nullptr, c->ff_dirty, c->rowlen,
-                     c->counters, c->bb.ent_cap, c->st);
+                     c->counters, c->st);
         c->ff_dirty = 0;
     }
     const uint32_t rows = kDenseGraphPasses * c->K;
     const uint32_t start = 0u - rows; // the first replay advances it to row 0
     HIPCHK(c, hipMemcpyAsync(c->ctl + kCtlDenseBase, &start, 4, hipMemcpyHostToDevice, c->st));
     const NextPass np{c->K,   c->shooters,  c->nshoot, c->frames, c->snap,
-                      c->mvp, c->bb.count, (size_t)c->K * c->bb.ntiles, c->counters,
-                      c->bb.ent_cap};
+                      c->mvp, c->bb.count, (size_t)c->K * c->bb.ntiles, c->counters};
     launch_dense_prepare(np, c->unshot, c->ctl, c->npatch, c->st);
     HIPCHK(c, hipStreamSynchronize(c->st));
     hipGraph_t graph = nullptr;

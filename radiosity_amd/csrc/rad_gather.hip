@@ -85,7 +85,7 @@ __device__ static void dense_prepare(const NextPass &np, const float *__restrict
     __shared__ uint32_t ssel[RAD_MAX_K], sn;
     if (wg) {
         clear_range((size_t)(wg - 1u) * blockDim.x + threadIdx.x, (size_t)(nwg - 1u) * blockDim.x,
-                    np.bin_count, np.nbins, nullptr, nullptr, 0, np.counters, np.ent_cap);
+                    np.bin_count, np.nbins, nullptr, nullptr, 0, np.counters);
         return;
     }
     const uint32_t k = dense_rows(ctl, np.K, row0, npatch);

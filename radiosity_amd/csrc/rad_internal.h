@@ -59,6 +59,7 @@ enum {
 };
 constexpr uint32_t kBinClasses = 8;     // size classes of the launch order
 constexpr uint32_t kBinSeen = 0x80000000u; // in a bin's count: summed into kCntEntries
+constexpr uint64_t kMaxEntries = 0xF0000000ull;
 constexpr uint32_t kSplitRecs = 1536;   // records from which a bin is drawn as quadrants
 // What the tile kernel reads beside its arguments: counters of the pass, and
 // what only a bin fuller than its list needs.
@@ -67,7 +68,8 @@ struct BinFacts {
     uint32_t cls[kBinClasses];
     const uint32_t *blk_nrec;
     uint32_t *pool, *pool_used;
-    uint32_t nreg, spill_base, spill_cap, pool_cap, split_cap, pad;
+    uint32_t nreg, spill_base, spill_cap, split_cap;
+    uint32_t pool_cap, pad; // pool_cap: also the most entries the pass may have
 };
 static_assert((kCntFacts + 4) == kCntClass && kCntFacts * 4 + sizeof(BinFacts) <= kCntPool * 4 &&
                   kCntFacts % 2 == 0 && kCntN % 2 == 0,
@@ -136,7 +138,8 @@ struct BinBuffers {
     uint32_t nbins, bin_cap;
     uint32_t nblk;         // setup blocks per shooter and face group (256 triangles each)
     uint32_t nz;           // face groups: 5 (one face per block, small K) or 1
-    uint32_t spill_base, spill_cap, ent_cap;
+    uint32_t halves;       // 2 where a pass may be split, else 1
+    uint32_t spill_base, spill_cap, ent_cap; // of each half
     uint2 *clipq;          // kCntBlocks queues of clip_cap clipping jobs
     uint32_t clip_cap;
     int clip_blocks;
@@ -199,26 +202,28 @@ void launch_prepare(const Geometry &g, uint32_t K, const uint32_t *shooters,
 void launch_prepare_clear(uint32_t K, const uint32_t *shooters, uint32_t *nshoot,
                           const float *frames, const float *unshot, float *snap, float *mvp,
                           uint32_t *bin_count, uint32_t ntiles, float *ff, uint32_t *hits,
-                          uint32_t ff_rows, uint32_t rowlen, uint32_t *counters, uint32_t ent_cap,
+                          uint32_t ff_rows, uint32_t rowlen, uint32_t *counters,
                           const uint32_t *ctl, hipStream_t st);
 void launch_clear(uint32_t K, uint32_t *bin_count, uint32_t ntiles, float *ff, uint32_t *hits,
-                  uint32_t ff_rows, uint32_t rowlen, uint32_t *counters, uint32_t ent_cap,
+                  uint32_t ff_rows, uint32_t rowlen, uint32_t *counters,
                   hipStream_t st);
 // Binned render of the shooter slots [s0, s1) (of which those below nshoot
 // are drawn) in three launches: setup (records and bins), bin (launch order
 // of the bins, clipped triangles), tile (LDS depth test; out_ids != null
 // writes the item buffer, ff or ffq != null reduces into F rows and hits).  h selects the counter block,
 // spill region and clip queue (0, or 1 for the second half of a split pass).
-// fixed: the tiles that follow go to the fixed-point rows ffq.
+// whole: not as halves.  fixed: the tiles that follow go to the fixed-point rows ffq.
 void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h,
                          const float *tri, const float4 *tsph, const float4 *tback,
                          const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const uint32_t *nshoot,
                          const BinBuffers &bb, uint32_t *counters, const uint32_t *slot_tbeg,
-                         const uint32_t *slot_tcnt, const uint32_t *slot_w, hipStream_t st);
+                         const uint32_t *slot_tcnt, const uint32_t *slot_w, bool whole, hipStream_t st);
 void launch_tri_sphere(const float *tri, uint32_t ntri, float4 *sph, float4 *back, hipStream_t st);
 void launch_bin(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const float *tri,
                 const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const BinBuffers &bb,
-                uint32_t *counters, const uint32_t *slot_w, bool fixed, hipStream_t st);
+                uint32_t *counters, const uint32_t *slot_w, bool whole, bool fixed, hipStream_t st);
+// Entries such a pass may have.
+uint32_t entry_cap(const BinBuffers &bb, bool whole);
 void launch_tile(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const uint32_t *nshoot,
                  const BinBuffers &bb, uint32_t small_px, uint32_t *out_ids, float *out_depth,
                  const float *dff, uint32_t rowlen, const uint32_t *slot_pbeg, float *ff,
@@ -249,7 +254,6 @@ struct NextPass {
     uint32_t *bin_count;
     size_t nbins;
     uint32_t *counters;
-    uint32_t ent_cap;
 };
 // With np (its frames, snapshots, MVPs, bins and counters) the selection
 // also prepares the pass.

@@ -114,11 +114,10 @@ void launch_prepare(const Geometry &g, uint32_t K, const uint32_t *shooters,
 
 // --------------------------------------------------------------------- clear
 __global__ void k_clear(uint32_t *__restrict__ bin_count, size_t nbins, float *__restrict__ ff,
-                        uint32_t *__restrict__ hits, size_t nff, uint32_t *__restrict__ counters,
-                        uint32_t ent_cap)
+                        uint32_t *__restrict__ hits, size_t nff, uint32_t *__restrict__ counters)
 {
     clear_range((size_t)blockIdx.x * blockDim.x + threadIdx.x, (size_t)gridDim.x * blockDim.x,
-                bin_count, nbins, ff, hits, nff, counters, ent_cap);
+                bin_count, nbins, ff, hits, nff, counters);
 }
 
 // k_prepare and k_clear of a pass in one launch (the first np workgroups
@@ -134,7 +133,7 @@ __global__ __launch_bounds__(256) void k_prepare_clear(
     uint32_t *__restrict__ nshoot, const float *__restrict__ frames,
     const float *__restrict__ unshot, float *__restrict__ snap, float *__restrict__ mvp,
     uint32_t *__restrict__ bin_count, size_t nbins, float *__restrict__ ff,
-    uint32_t *__restrict__ hits, size_t nff, uint32_t *__restrict__ counters, uint32_t ent_cap,
+    uint32_t *__restrict__ hits, size_t nff, uint32_t *__restrict__ counters,
     const uint32_t *__restrict__ ctl)
 {
     if (blockIdx.x < np) {
@@ -145,14 +144,13 @@ __global__ __launch_bounds__(256) void k_prepare_clear(
     if (ctl && blockIdx.x == np && threadIdx.x == 0 && ctl[kCtlStop])
         *nshoot = 0u;
     clear_range((size_t)(blockIdx.x - np) * blockDim.x + threadIdx.x,
-                (size_t)(gridDim.x - np) * blockDim.x, bin_count, nbins, ff, hits, nff, counters,
-                ent_cap);
+                (size_t)(gridDim.x - np) * blockDim.x, bin_count, nbins, ff, hits, nff, counters);
 }
 
 void launch_prepare_clear(uint32_t K, const uint32_t *shooters, uint32_t *nshoot,
                           const float *frames, const float *unshot, float *snap, float *mvp,
                           uint32_t *bin_count, uint32_t ntiles, float *ff, uint32_t *hits,
-                          uint32_t ff_rows, uint32_t rowlen, uint32_t *counters, uint32_t ent_cap,
+                          uint32_t ff_rows, uint32_t rowlen, uint32_t *counters,
                           const uint32_t *ctl, hipStream_t st)
 {
     const uint32_t np = (K * 5 + 255) / 256;
@@ -165,11 +163,11 @@ void launch_prepare_clear(uint32_t K, const uint32_t *shooters, uint32_t *nshoot
         blocks = 1;
     k_prepare_clear<<<(unsigned)(np + blocks), 256, 0, st>>>(np, K, shooters, nshoot, frames,
                                                             unshot, snap, mvp, bin_count, nbins,
-                                                            ff, hits, nff, counters, ent_cap, ctl);
+                                                            ff, hits, nff, counters, ctl);
 }
 
 void launch_clear(uint32_t K, uint32_t *bin_count, uint32_t ntiles, float *ff, uint32_t *hits,
-                  uint32_t ff_rows, uint32_t rowlen, uint32_t *counters, uint32_t ent_cap,
+                  uint32_t ff_rows, uint32_t rowlen, uint32_t *counters,
                   hipStream_t st)
 {
     // ff null: the F rows are known to be zero (the last shoot cleared them)
@@ -180,7 +178,7 @@ void launch_clear(uint32_t K, uint32_t *bin_count, uint32_t ntiles, float *ff, u
         blocks = 8192;
     if (blocks == 0)
         blocks = 1;
-    k_clear<<<(unsigned)blocks, 256, 0, st>>>(bin_count, nbins, ff, hits, nff, counters, ent_cap);
+    k_clear<<<(unsigned)blocks, 256, 0, st>>>(bin_count, nbins, ff, hits, nff, counters);
 }
 
 // ---------------------------------------------------------------- rasterizer
@@ -1156,8 +1154,12 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
     }
 }
 
-static BinCtx bin_ctx(const BinBuffers &bb, uint32_t h, uint32_t *counters)
+// Counter block h's part of the buffers: its half's, or both halves' for a pass
+// drawn whole by a context whose larger passes are split (bb.halves), so that
+// what a pass may hold does not depend on whether it is.
+static BinCtx bin_ctx(const BinBuffers &bb, uint32_t h, bool whole, uint32_t *counters)
 {
+    const uint32_t parts = whole ? bb.halves : 1u;
     BinCtx bc;
     bc.recs = bb.recs;
     bc.bbox = bb.bbox;
@@ -1167,9 +1169,9 @@ static BinCtx bin_ctx(const BinBuffers &bb, uint32_t h, uint32_t *counters)
     bc.lcnt = nullptr;
     bc.region = 0;
     bc.spill_base = bb.spill_base + h * bb.spill_cap;
-    bc.spill_cap = bb.spill_cap;
+    bc.spill_cap = parts * bb.spill_cap;
     bc.clipq = bb.clipq + (size_t)h * bb.clip_cap;
-    bc.clip_cap = bb.clip_cap;
+    bc.clip_cap = parts * bb.clip_cap;
     bc.ntx = bb.ntx;
     bc.ntiles = bb.ntiles;
     bc.tshift = bb.tshift;
@@ -1178,11 +1180,18 @@ static BinCtx bin_ctx(const BinBuffers &bb, uint32_t h, uint32_t *counters)
     return bc;
 }
 
+uint32_t entry_cap(const BinBuffers &bb, bool whole)
+{
+    const uint64_t n = (uint64_t)bb.ent_cap * (whole ? bb.halves : 1u);
+    return (uint32_t)(n > kMaxEntries ? kMaxEntries : n);
+}
+
 void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h,
                          const float *tri, const float4 *tsph, const float4 *tback,
                          const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const uint32_t *nshoot,
                          const BinBuffers &bb, uint32_t *counters, const uint32_t *slot_tbeg,
-                         const uint32_t *slot_tcnt, const uint32_t *slot_w, hipStream_t st)
+                         const uint32_t *slot_tcnt, const uint32_t *slot_w, bool whole,
+                         hipStream_t st)
 {
     const uint32_t n = s1 - s0;
     uint32_t group = bb.setup_group ? bb.setup_group : 1u;
@@ -1190,7 +1199,7 @@ void launch_raster_setup(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h
         group = n;
     dim3 grid(bb.nblk, (n + group - 1) / group, bb.nz);
     k_raster_setup<<<grid, 256, 4 * bb.ntiles * sizeof(uint32_t), st>>>(
-        g.W, tri, tsph, tback, tri_patch, ntri, mvp, nshoot, bin_ctx(bb, h, counters), bb.blk_nrec,
+        g.W, tri, tsph, tback, tri_patch, ntri, mvp, nshoot, bin_ctx(bb, h, whole, counters), bb.blk_nrec,
         slot_tbeg, slot_tcnt, slot_w, group, s0, s1);
 }
 
@@ -1214,14 +1223,14 @@ static uint32_t split_cap(const BinBuffers &bb, uint32_t nb, bool fixed)
 
 void launch_bin(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const float *tri,
                 const uint32_t *tri_patch, uint32_t ntri, const float *mvp, const BinBuffers &bb,
-                uint32_t *counters, const uint32_t *slot_w, bool fixed, hipStream_t st)
+                uint32_t *counters, const uint32_t *slot_w, bool whole, bool fixed, hipStream_t st)
 {
     const uint32_t b0 = s0 * bb.ntiles, nb = (s1 - s0) * bb.ntiles;
     const uint32_t norder = (nb + 256u * kOrderPer - 1) / (256u * kOrderPer);
     k_order_clip<<<norder + bb.clip_blocks, 256, 0, st>>>(
         norder, nb, b0, split_cap(bb, nb, fixed), bb.order + b0, bb.nbins, g.W, tri, tri_patch, ntri, mvp,
-        bin_ctx(bb, h, counters), bb.blk_nrec, bb.nblk * bb.nz,
-        bb.pool + (size_t)h * bb.ent_cap, bb.ent_cap, slot_w);
+        bin_ctx(bb, h, whole, counters), bb.blk_nrec, bb.nblk * bb.nz,
+        bb.pool + (size_t)h * bb.ent_cap, entry_cap(bb, whole), slot_w);
 }
 
 void launch_tile(const Geometry &g, uint32_t s0, uint32_t s1, uint32_t h, const uint32_t *nshoot,
@@ -2058,8 +2067,7 @@ __global__ __launch_bounds__(1024) void k_next_pass(const uint64_t *__restrict__
         pool->count = 0u;
     for (uint32_t i = t; i < np.K * 5; i += blockDim.x)
         prepare_item(i, np.K, ssel, &sn, np.frames, unshot, np.snap, np.mvp, nullptr);
-    clear_range(t, blockDim.x, np.bin_count, np.nbins, nullptr, nullptr, 0, np.counters,
-                np.ent_cap);
+    clear_range(t, blockDim.x, np.bin_count, np.nbins, nullptr, nullptr, 0, np.counters);
 }
 
 void launch_next_pass(const uint64_t *lists, uint32_t nlists, const NextPass &np,
@@ -2132,8 +2140,7 @@ __global__ __launch_bounds__(1024) void k_next_top1(uint32_t rule, const uint64_
     __syncthreads();
     if (t < 5)
         prepare_item(t, 1u, &ssel, &sn, np.frames, unshot, np.snap, np.mvp, nullptr);
-    clear_range(t, blockDim.x, np.bin_count, np.nbins, nullptr, nullptr, 0, np.counters,
-                np.ent_cap);
+    clear_range(t, blockDim.x, np.bin_count, np.nbins, nullptr, nullptr, 0, np.counters);
 }
 
 void launch_next_top1(uint32_t rule, const uint64_t *keys, uint32_t nkeys, const NextPass &np,
@@ -2619,7 +2626,7 @@ __global__ __launch_bounds__(kRefThreads) void k_select_reference(
         for (uint32_t i = threadIdx.x; i < np.K * 5; i += kRefThreads)
             prepare_item(i, np.K, li, &sn, np.frames, unshot, np.snap, np.mvp, nullptr);
         clear_range(threadIdx.x, kRefThreads, np.bin_count, np.nbins, nullptr, nullptr, 0,
-                    np.counters, np.ent_cap);
+                    np.counters);
     }
     if (threadIdx.x == 0)
         *nshoot = sn;

@@ -147,15 +147,17 @@ __device__ static void prepare_item(uint32_t t, uint32_t K, const uint32_t *__re
 __device__ static void clear_range(size_t i, size_t stride, uint32_t *__restrict__ bin_count,
                                    size_t nbins, float *__restrict__ ff,
                                    uint32_t *__restrict__ hits, size_t nff,
-                                   uint32_t *__restrict__ counters, uint32_t ent_cap)
+                                   uint32_t *__restrict__ counters)
 {
     if (i == 0) {
         // every block of pass counters (one per half-pass), the sticky flag
         // in the first
         bool bad = false;
-        for (int h = 0; h < kCntBlocks; ++h)
-            bad = bad || counters[h * kCntN + kCntOverflow] != 0 ||
-                  counters[h * kCntN + kCntEntries] > ent_cap;
+        for (int h = 0; h < kCntBlocks; ++h) {
+            const uint32_t *const cnt = counters + h * kCntN;
+            const BinFacts *const f = reinterpret_cast<const BinFacts *>(cnt + kCntFacts);
+            bad = bad || cnt[kCntOverflow] != 0 || cnt[kCntEntries] > f->pool_cap;
+        }
         for (int h = 0; h < kCntBlocks; ++h)
             for (int k = 0; k < kCntN; ++k)
                 if (h || k != kCntSticky)

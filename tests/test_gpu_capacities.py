@@ -33,19 +33,22 @@ def test_many_triangles_to_clip(rad):
     assert np.array_equal(ids, O.render_hemicube(64, sc.tri, sc.tri_patch, sc.frame[0]))
 
 
-def test_entries_of_small_tiles(rad):
-    """Twelve shooters amid 3,000 large triangles: in tiles of 32, the entries
-    fit; in tiles of 16, which the library takes, they are more than that
-    limit."""
+def _large(rad, n):
+    """n shooters amid 3,000 large triangles, all of them seen from the middle."""
     rng = np.random.default_rng(3)
     c = rng.normal(size=(3000, 1, 3))
     c[:, :, 2] = np.abs(c[:, :, 2])
     c *= rng.uniform(3, 5, (3000, 1, 1)) / np.linalg.norm(c, axis=2, keepdims=True)
     tri = c + 2.0 * rng.uniform(-1, 1, (3000, 3, 3))
-    n = np.cross(tri[:, 2] - tri[:, 0], tri[:, 1] - tri[:, 0])
-    back = (n * tri.mean(1)).sum(1) > 0  # all of them seen from the middle
+    back = (np.cross(tri[:, 2] - tri[:, 0], tri[:, 1] - tri[:, 0]) * tri.mean(1)).sum(1) > 0
     tri[back] = tri[back][:, [0, 2, 1]]
-    sc = _scene(rad, tri, rng.uniform(-0.1, 0.1, (12, 3)))
+    return _scene(rad, tri, rng.uniform(-0.1, 0.1, (n, 3)))
+
+
+def test_entries_of_small_tiles(rad):
+    """Twelve shooters: in tiles of 32, the entries fit; in tiles of 16, which
+    the library takes, they are more than that limit."""
+    sc = _large(rad, 12)
     sh = np.arange(12)
     out = []
     for tile in (32, 0):
@@ -57,3 +60,19 @@ def test_entries_of_small_tiles(rad):
         s.close()
     assert out[1][2] == 16 and out[1][1]["entries"] > out[0][1]["entry_cap"]
     assert np.array_equal(out[0][0], out[1][0])
+
+
+def test_entries_of_a_whole_pass(rad):
+    """24 shooters in 4,608 tiles of 16, drawn whole: more entries than each
+    half of a split pass may have, and fewer than both."""
+    sc = _large(rad, 24)
+    print("entries of a whole pass", flush=True)
+    s = rad.Solver(hemicube=128, hemicubes=24, tile_px=16)
+    s.upload(sc)
+    ids = s.render(np.arange(24))
+    c = s.debug_counters()
+    assert c["entry_cap"] < c["entries"] < 2 * c["entry_cap"]
+    res = s.tex_res
+    for k in (0, 23):
+        assert np.array_equal(ids[k * res:(k + 1) * res],
+                              O.render_hemicube(128, sc.tri, sc.tri_patch, sc.frame[k]))

@@ -76,6 +76,7 @@ template <typename T> int dalloc(rad_ctx *c, T **p, size_t n)
     hipError_t e = hipMalloc((void **)p, n * sizeof(T));
     if (e != hipSuccess) {
         *p = nullptr;
+        (void)hipGetLastError(); // not the next launch's error
         return fail(c, RAD_E_NOMEM, "hipMalloc of " + std::to_string(n * sizeof(T)) +
                                         " bytes: " + hipGetErrorString(e));
     }
@@ -402,8 +403,11 @@ int one_pass(rad_ctx *c, bool do_select, size_t evbase, bool chain_in = false,
 }
 
 // The bins' lists: room for 16 times the records per bin of a scene spread
-// evenly over the tiles, within 4 GiB in all.  A fuller bin's workgroup makes
-// its list in the pool (whole_list), so the size is no limit.
+// evenly over the tiles, within 4 GiB in all, or for half of it and so on where
+// the device has no memory for that (1.6 GB for 64 shooters of 200,000
+// triangles at hemicube 256).  A fuller bin's workgroup makes its list in the
+// pool (whole_list), so the size is no limit.  Allocated after the buffers that
+// a scene cannot do without.
 int bin_lists(rad_ctx *c)
 {
     const uint64_t ntri = (uint64_t)c->bb.nblk * 256;
@@ -412,8 +416,13 @@ int bin_lists(rad_ctx *c)
         cap *= 2;
     while (cap > 256 && (uint64_t)c->bb.nbins * cap > (1ull << 30))
         cap /= 2;
+    int rc;
+    while ((rc = dalloc(c, &c->bb.list, (size_t)c->bb.nbins * cap)) && cap > 16) {
+        c->err.clear();
+        cap /= 2;
+    }
     c->bb.bin_cap = cap;
-    return dalloc(c, &c->bb.list, (size_t)c->bb.nbins * cap);
+    return rc;
 }
 
 // The tile side of a context without a chosen one, for a scene of ntri
@@ -442,6 +451,14 @@ static uint32_t tile_side(const rad_ctx *c, uint32_t ntri)
     return dense ? 16u : 32u;
 }
 
+// A scene whose buffers were allocated but not filled is no scene.
+int drop_scene(rad_ctx *c, int rc)
+{
+    c->ntri = c->npatch = c->nquad = 0;
+    c->hash_valid = false;
+    return rc;
+}
+
 // Screen tile side T (8, 16, 32) and the in-lane triangle limit; (re)sizes
 // the per-(shooter, tile) bin arrays.
 int set_tiles(rad_ctx *c, uint32_t T, uint32_t small_px)
@@ -455,6 +472,19 @@ int set_tiles(rad_ctx *c, uint32_t T, uint32_t small_px)
         return fail(c, RAD_E_ARG, "too many screen tiles per hemicube (use a larger tile_px)");
     if (c->st)
         (void)hipStreamSynchronize(c->st);
+    // without memory for the new bins the old ones stay
+    const size_t nbins = (size_t)c->K * ntx * nty;
+    uint32_t *count = nullptr, *order = nullptr;
+    int rc;
+    if ((rc = dalloc(c, &count, nbins)) || (rc = dalloc(c, &order, nbins * kBinClasses))) {
+        dfree(count);
+        return rc;
+    }
+    dfree(c->bb.count);
+    dfree(c->bb.order);
+    c->bb.count = count;
+    c->bb.order = order;
+    c->bb.nbins = (uint32_t)nbins;
     c->bb.tshift = T == 8 ? 3 : (T == 16 ? 4 : 5);
     c->bb.ntx = ntx;
     c->bb.nty = nty;
@@ -463,13 +493,9 @@ int set_tiles(rad_ctx *c, uint32_t T, uint32_t small_px)
     c->cfg.tile_px = T;
     c->cfg.small_tri_px = small_px;
     drop_graph(c);
-    size_t nbins = (size_t)c->K * c->bb.ntiles;
-    int rc;
-    c->bb.nbins = (uint32_t)nbins;
-    if ((rc = dalloc(c, &c->bb.count, nbins)) ||
-        (rc = dalloc(c, &c->bb.order, nbins * kBinClasses)))
-        return rc;
-    return c->npatch ? bin_lists(c) : RAD_OK;
+    if (c->npatch && (rc = bin_lists(c)))
+        return drop_scene(c, rc); // no pass without lists
+    return RAD_OK;
 }
 
 int need_scene(rad_ctx *c)
@@ -737,12 +763,12 @@ int scene_alloc(rad_ctx *c, uint32_t ntri, uint32_t npatch, uint32_t nblk, uint3
     const uint64_t went = (c->auto_side && K >= 4 && side == 16 ? 8 : 2) * (slots + spill);
     c->bb.ent_cap = (uint32_t)(went > kMaxEntries ? kMaxEntries : went);
     // each half of a split pass has its own spill region and clipping queue
-    const uint64_t nrec = regions + (uint64_t)kCntBlocks * c->bb.spill_cap;
+    const uint64_t nrec = regions + (uint64_t)c->bb.halves * c->bb.spill_cap;
     if ((rc = dalloc(c, &c->bb.recs, nrec)) || (rc = dalloc(c, &c->bb.bbox, nrec)) ||
-        (rc = bin_lists(c)) || (rc = dalloc(c, &c->bb.pool, (size_t)kCntBlocks * c->bb.ent_cap)) ||
+        (rc = dalloc(c, &c->bb.pool, (size_t)c->bb.halves * c->bb.ent_cap)) ||
         (rc = dalloc(c, &c->bb.blk_nrec, (size_t)c->bb.nblk * K * c->bb.nz)) ||
-        (rc = dalloc(c, &c->bb.clipq, (size_t)kCntBlocks * c->bb.clip_cap)) ||
-        (rc = dalloc(c, &c->cand, 2 * topk_cand_half(npatch, c->K))))
+        (rc = dalloc(c, &c->bb.clipq, (size_t)c->bb.halves * c->bb.clip_cap)) ||
+        (rc = dalloc(c, &c->cand, 2 * topk_cand_half(npatch, c->K))) || (rc = bin_lists(c)))
         return rc;
     HIPCHK(c, hipMemset(c->ff, 0, K * rowlen * 4));
     HIPCHK(c, hipMemset(c->fblk, 0, (size_t)(rowlen + 63) / 64 * K * 4));
@@ -795,14 +821,6 @@ int upload_copy(rad_ctx *c, const float *tri_xyz, const uint32_t *tri_patch, uin
     c->geom_hash = scene_hash(ntri, npatch, tri_xyz, tri_patch, frames, refl, area);
     c->hash_valid = true;
     return RAD_OK;
-}
-
-// A scene whose buffers were allocated but not filled is no scene.
-int drop_scene(rad_ctx *c, int rc)
-{
-    c->ntri = c->npatch = c->nquad = 0;
-    c->hash_valid = false;
-    return rc;
 }
 
 int upload_impl(rad_ctx *c, const float *tri_xyz, const uint32_t *tri_patch, uint32_t ntri,

@@ -128,19 +128,19 @@ enum {
 
 // Bins of the sort-middle rasterizer: one per (shooter slot, tile).
 struct BinBuffers {
-    RasterRec *recs;       // nblk*K regions of kRecsPerBlock, then kCntBlocks spill regions of spill_cap
+    RasterRec *recs;       // nblk*K regions of kRecsPerBlock, then `halves` spill regions of spill_cap
     uint64_t *bbox;        // texel bbox per record slot, of which the lists are made
     uint32_t *blk_nrec;    // records per (shooter, setup block)
     uint32_t *count;       // records per bin
     uint32_t *list;        // bin_cap record slots per bin
-    uint32_t *pool;        // kCntBlocks areas of ent_cap entries: lists of fuller bins
+    uint32_t *pool;        // `halves` areas of ent_cap entries: lists of fuller bins
     uint32_t *order;       // kBinClasses queues of nbins bins (tile launch order)
     uint32_t nbins, bin_cap;
     uint32_t nblk;         // setup blocks per shooter and face group (256 triangles each)
     uint32_t nz;           // face groups: 5 (one face per block, small K) or 1
     uint32_t halves;       // 2 where a pass may be split, else 1
     uint32_t spill_base, spill_cap, ent_cap; // of each half
-    uint2 *clipq;          // kCntBlocks queues of clip_cap clipping jobs
+    uint2 *clipq;          // `halves` queues of clip_cap clipping jobs
     uint32_t clip_cap;
     int clip_blocks;
     uint32_t ntx, nty, ntiles, tshift;

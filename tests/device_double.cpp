@@ -12,7 +12,8 @@
 namespace {
 
 std::map<void *, size_t> live;          // allocations not freed yet
-size_t live_bytes, limit = SIZE_MAX;    // hipMalloc refuses what would exceed limit
+size_t live_bytes, limit = SIZE_MAX;    // hipMalloc refuses what would exceed limit,
+size_t largest = SIZE_MAX;              // and any single one beyond largest
 std::map<const void *, std::string> kernels;
 void (*launched)(const char *name, void **args);
 float elapsed; // each hipEventElapsedTime reads 1 ms more than the last
@@ -24,11 +25,12 @@ extern "C" {
 size_t double_live(void) { return live.size(); }
 size_t double_live_bytes(void) { return live_bytes; }
 void double_limit(size_t bytes) { limit = bytes; }
+void double_largest(size_t bytes) { largest = bytes; }
 void double_on_launch(void (*f)(const char *, void **)) { launched = f; }
 
 hipError_t hipMalloc(void **p, size_t n)
 {
-    if (n > limit || live_bytes > limit - n)
+    if (n > largest || n > limit || live_bytes > limit - n)
         return hipErrorOutOfMemory;
     *p = calloc(n, 1);
     live[*p] = n;

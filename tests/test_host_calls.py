@@ -25,7 +25,7 @@ def on_double(tmp_path_factory):
             import ctypes as C, numpy as np
             D = C.CDLL({so!r}, mode=C.RTLD_GLOBAL)
             D.double_live.restype = D.double_live_bytes.restype = C.c_size_t
-            D.double_limit.argtypes = [C.c_size_t]
+            D.double_limit.argtypes = D.double_largest.argtypes = [C.c_size_t]
             import radiosity_amd as R
             """
         p = subprocess.run([sys.executable, "-c", textwrap.dedent(head) + textwrap.dedent(code)],
@@ -90,4 +90,56 @@ def test_capacities_of_every_launch_shape(on_double):
                         assert c["spill_cap"] >= spill, (W, K, ntri, tile)
                         assert c["entry_cap"] == entries, (W, K, ntri, tile)
         assert (0, True, 16) in seen and (0, True, 32) in seen
+        """)
+
+
+def test_lists_in_the_memory_there_is(on_double):
+    """An upload, and another tile side later, without memory for the tiles'
+    lists at their full size take smaller ones; without any, the context has no
+    scene.  No launch gets a missing list."""
+    on_double("""
+        sc = R.Scene.boxes(nboxes=8, room=(6.0, 3.0, 6.0), target_tris=6000, nlights=2, seed=3)
+        tiles = []
+        def note(name, args):
+            if b"k_tile_raster" in name:
+                tiles.append([C.cast(args[i], C.POINTER(C.c_void_p))[0] for i in (7, 8)])
+        CB = C.CFUNCTYPE(None, C.c_char_p, C.POINTER(C.c_void_p))
+        D.double_on_launch(cb := CB(note))
+
+        def solver(limit):
+            D.double_limit(limit)
+            s = R.Solver(hemicube=64, hemicubes=40, tile_px=32)
+            s.upload(sc)
+            return s
+
+        s = solver(1 << 62)
+        full = D.double_live_bytes()
+        s.close()
+        lists = 4 * 40 * 12 * 8192  # 40 x 12 tiles, 16 x 6,000 / 12 entries and up
+        assert full > lists
+        # the upload, with a quarter of the lists' memory
+        s = solver(full - lists * 3 // 4)
+        assert D.double_live_bytes() < full - lists // 2
+        s.step(3)
+        s.close()
+        # other tiles later, with a quarter; and with none
+        s = solver(1 << 62)
+        D.double_largest(lists // 4)
+        s.autotune(1)
+        s.step(3)
+        s.close()
+        D.double_largest(1 << 62)
+        s = solver(1 << 62)
+        D.double_largest(70000)
+        for call, word in ((lambda: s.autotune(1), "out of memory"), (lambda: s.step(1), "no scene")):
+            try:
+                call()
+                raise SystemExit("done without lists")
+            except R.RadError as e:
+                assert word in str(e), e
+        D.double_largest(1 << 62)
+        s.upload(sc)
+        s.step(3)
+        s.close()
+        assert len(tiles) > 20 and all(p for t in tiles for p in t)
         """)

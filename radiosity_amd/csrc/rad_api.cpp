@@ -1562,6 +1562,7 @@ int rad_autotune(rad_ctx *c, uint32_t passes, rad_tune_result *out)
     // still than the best candidate
     uint32_t Td;
     c->auto_tile = was_auto;
+    c->small_px = r.tile_px ? r.small_tri_px : S0; // as they will run
     if (rc == RAD_OK && use_direct(c, c->K, &Td)) {
         rc = render_pass(c, c->K, 0, nullptr, nullptr, nullptr); // warm
         (void)hipEventRecord(e0, c->st);

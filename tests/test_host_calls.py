@@ -143,3 +143,22 @@ def test_lists_in_the_memory_there_is(on_double):
         s.close()
         assert len(tiles) > 20 and all(p for t in tiles for p in t)
         """)
+
+
+def test_autotune_times_direct_passes_with_the_limit_it_chose(on_double):
+    """The stand-in's times grow with every call, so the first candidate's
+    limit of 16 pixels is chosen."""
+    on_double("""
+        limits = []
+        def note(name, args):
+            if b"k_direct" in name:
+                limits.append(C.cast(args[0], C.POINTER(C.c_uint32))[5])  # DirectArgs::small_px
+        CB = C.CFUNCTYPE(None, C.c_char_p, C.POINTER(C.c_void_p))
+        D.double_on_launch(cb := CB(note))
+        s = R.Solver(hemicube=64, hemicubes=8)
+        s.upload(R.Scene.boxes(nboxes=4, room=(5.0, 3.0, 5.0), target_tris=2000, nlights=2, seed=3))
+        s.step(1)
+        assert limits == [64]
+        assert s.autotune(2)[1] == 16
+        assert limits == [64] + 3 * [16], limits
+        """)

@@ -252,7 +252,9 @@ int rad_debug_bins(rad_ctx *ctx, uint32_t *out_or_null, uint32_t *ntiles, uint32
  * the spill capacity, the bin-entry capacity and the clip-queue capacity.
  * A large pass renders as two halves, each with these
  * capacities: [3], [5] and [6] are then the fuller half's, [4] the sum.  A pass
- * drawn whole has those of both halves where hemicubes is 16 or more. */
+ * drawn whole has those of both halves where hemicubes is 16 or more.  A pass
+ * drawn without bins has no entries, records or queued faces: [3], [5] and [6]
+ * are 0 (rad_debug_bins makes its counts when asked). */
 int rad_debug_counters(rad_ctx *ctx, uint32_t *out8, uint32_t *out_caps_or_null);
 
 /* Diagnostics (no counterpart in the reference): the candidate pool of the

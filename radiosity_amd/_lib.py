@@ -497,8 +497,9 @@ class Solver:
         return out.reshape(self.K, nt.value), tp.value
 
     def debug_counters(self):
-        """The rasterizer's pass counters of the last pass (dict) and the
-        spill, bin-entry and clip-queue capacities."""
+        """The rasterizer's pass counters of the last pass (dict; entries, spill
+        and clip are 0 after one drawn without bins) and the spill, bin-entry
+        and clip-queue capacities."""
         out = np.zeros(8, np.uint32)
         caps = np.zeros(3, np.uint32)
         self._chk(lib().rad_debug_counters(self._ctx, uptr(out), uptr(caps)), "rad_debug_counters")

@@ -14,7 +14,8 @@
 // (34 us for one shooter of the 1,534-triangle Cornell box at hemicube 128;
 // this one 17).  A triangle is set up once per tile it touches and a
 // workgroup holds a whole CU, so beyond two rounds of workgroups over the
-// CUs, or some 50,000 triangles, the bins win (direct_wins).
+// CUs, or 8,192 to 49,152 triangles by the number of workgroups, the bins win
+// (direct_wins).
 #include "rad_internal.h"
 #include "rad_raster.h"
 
@@ -285,7 +286,7 @@ __host__ __device__ static inline uint32_t direct_tiles(uint32_t W, uint32_t T)
 }
 
 constexpr uint32_t kDirThreads = 1024;
-constexpr uint32_t kDirChunk = 768;   // clusters a workgroup looks at before drawing
+constexpr uint32_t kDirMax = 768;     // clusters of the largest scene (direct_wins)
 constexpr uint32_t kDirTri = 2048;    // triangles it queues before drawing
 constexpr uint32_t kDirClip = 128;    // clip jobs a wavefront queues
 constexpr uint32_t kDirTwoLevel = 48; // clusters from which they are tested before their groups
@@ -310,12 +311,12 @@ __global__ __launch_bounds__(kDirThreads) void k_direct(DirectArgs a)
 {
     constexpr uint32_t NT = kDirThreads, NW = NT / 64;
     extern __shared__ uint64_t tk[]; // T x T depth keys
-    // indices relative to the chunk: a cluster, a group (4 per cluster), a
-    // triangle (64 per cluster)
-    __shared__ uint16_t clist[kDirChunk], glist[4 * kDirChunk], tq[kDirTri];
+    // indices within the scene: a cluster, a group (4 per cluster), a triangle
+    // (64 per cluster)
+    __shared__ uint16_t clist[kDirMax], glist[4 * kDirMax], tq[kDirTri];
     __shared__ uint16_t clipq[NW][kDirClip];
     __shared__ CV4 lp[NW][kClipMax];
-    static_assert(64 * kDirChunk <= 65536, "16-bit triangle indices");
+    static_assert(64 * kDirMax <= 65536, "16-bit triangle indices");
     __shared__ uint32_t nc_, ng_, nt_;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -416,177 +417,166 @@ __global__ __launch_bounds__(kDirThreads) void k_direct(DirectArgs a)
     };
     __syncthreads();
     const bool cull = v.cull != 0u;
-    for (uint32_t c0 = 0; c0 < nclu; c0 += kDirChunk) {
-        const uint32_t nc = min(kDirChunk, nclu - c0);
-        const float4 *const cl = clu + kCluWords * (size_t)c0;
-        const uint32_t t0 = tb + 64u * c0, ntc = min(te - t0, 64u * nc);
-        const bool two = cull && nclu > kDirTwoLevel;
-        if (c0) {
-            if (threadIdx.x == 0) {
-                nc_ = 0u;
-                ng_ = 0u;
-            }
-            __syncthreads();
-        }
-        // the clusters, then the groups of 16, that may touch the tile
-        if (two) {
-            for (uint32_t c = threadIdx.x; (c & ~63u) < nc; c += NT)
-                append(c < nc && run_in_tile(reload(v), cl + kCluWords * c, halfW), c, clist, &nc_);
-            __syncthreads();
-        }
-        const uint32_t nq = 4u * (two ? nc_ : nc);
-        for (uint32_t i = threadIdx.x; (i & ~63u) < nq; i += NT) {
-            bool vis = i < nq;
-            uint32_t g = i;
-            if (vis) {
-                if (two)
-                    g = 4u * clist[i >> 2] + (i & 3u);
-                vis = g * 16u < ntc;
-                if (vis && cull)
-                    vis = run_in_tile(reload(v), cl + kCluWords * (g >> 2) + 3u * (1u + (g & 3u)), halfW);
-            }
-            append(vis, g, glist, &ng_);
-        }
+    const uint32_t ntc = te - tb;
+    const bool two = cull && nclu > kDirTwoLevel;
+    // the clusters, then the groups of 16, that may touch the tile
+    if (two) {
+        for (uint32_t c = threadIdx.x; (c & ~63u) < nclu; c += NT)
+            append(c < nclu && run_in_tile(reload(v), clu + kCluWords * c, halfW), c, clist, &nc_);
         __syncthreads();
-        const uint32_t ng = ng_;
-        for (uint32_t g0 = 0; g0 < ng; g0 += kDirTri / 16u) {
-            const uint32_t g1 = min(ng, g0 + kDirTri / 16u);
-            // the triangles whose spheres may touch the tile, so that the
-            // exact pipeline runs with full wavefronts (and clips none that
-            // merely reaches behind the eye)
-            if (cull) {
-                if (c0 || g0) {
-                    if (threadIdx.x == 0)
-                        nt_ = 0u;
-                    __syncthreads();
-                }
-                for (uint32_t i = 16u * g0 + threadIdx.x; (i & ~63u) < 16u * g1; i += NT) {
-                    bool vis = i < 16u * g1;
-                    uint32_t t = 0;
-                    if (vis) {
-                        t = 16u * glist[i >> 4] + (i & 15u);
-                        vis = t < ntc && sphere_in_tile(reload(v), a.tsph[t0 + t]);
-                    }
-                    append(vis, t, tq, &nt_);
-                }
+    }
+    const uint32_t nq = 4u * (two ? nc_ : nclu);
+    for (uint32_t i = threadIdx.x; (i & ~63u) < nq; i += NT) {
+        bool vis = i < nq;
+        uint32_t g = i;
+        if (vis) {
+            if (two)
+                g = 4u * clist[i >> 2] + (i & 3u);
+            vis = g * 16u < ntc;
+            if (vis && cull)
+                vis = run_in_tile(reload(v), clu + kCluWords * (g >> 2) + 3u * (1u + (g & 3u)), halfW);
+        }
+        append(vis, g, glist, &ng_);
+    }
+    __syncthreads();
+    const uint32_t ng = ng_;
+    for (uint32_t g0 = 0; g0 < ng; g0 += kDirTri / 16u) {
+        const uint32_t g1 = min(ng, g0 + kDirTri / 16u);
+        // the triangles whose spheres may touch the tile, so that the
+        // exact pipeline runs with full wavefronts (and clips none that
+        // merely reaches behind the eye)
+        if (cull) {
+            if (g0) {
+                if (threadIdx.x == 0)
+                    nt_ = 0u;
                 __syncthreads();
             }
-            // The exact pipeline and the drawing, every wavefront on its own:
-            // up to 64 triangles per step, fewer (a power of two) when there
-            // are not enough for every wavefront; then lanes share one, each
-            // doing its pipeline and drawing every nph-th of its rows (1
-            // shooter over 20,000 triangles at hemicube 256: 28.7 us with a
-            // lane per triangle, 27.2).
-            // Triangles to clip are queued by their wavefront and taken one
-            // per step.
-            const uint32_t nt = cull ? nt_ : 16u * (g1 - g0);
-            uint32_t lb = 0; // log2 of the triangles per step
-            while (lb < 6u && (NW << lb) < nt)
-                ++lb;
-            const uint32_t bs = 1u << lb;
-            uint32_t qi = wv * bs, cn = 0;
-            uint16_t *const cq = clipq[wv];
-            while (true) {
-                const bool batch = qi < nt && cn <= kDirClip - 64u;
-                if (!batch && cn == 0)
-                    break;
-                wave_lds_sync();
-                const TileView &vw = reload(v);
-                SV A, B, C;
-                uint32_t id = 0;
-                bool have = false;
-                // row phase of the lane's triangle, log2 of the phases
-                uint32_t ph = 0, lph = 0;
-                if (batch) {
-                    bool clip = false;
-                    uint32_t tr = ntc;
-                    const uint32_t i = qi + (lane & (bs - 1u));
-                    ph = lane >> lb;
-                    lph = 6u - lb;
-                    if (i < nt) {
-                        tr = cull ? tq[i] : 16u * glist[g0 + (i >> 4)] + (i & 15u);
-                    }
-                    if (tr < ntc) {
-                        const uint32_t t = t0 + tr;
-                        float vx[3][3];
+            for (uint32_t i = 16u * g0 + threadIdx.x; (i & ~63u) < 16u * g1; i += NT) {
+                bool vis = i < 16u * g1;
+                uint32_t t = 0;
+                if (vis) {
+                    t = 16u * glist[i >> 4] + (i & 15u);
+                    vis = t < ntc && sphere_in_tile(reload(v), a.tsph[tb + t]);
+                }
+                append(vis, t, tq, &nt_);
+            }
+            __syncthreads();
+        }
+        // The exact pipeline and the drawing, every wavefront on its own:
+        // up to 64 triangles per step, fewer (a power of two) when there
+        // are not enough for every wavefront; then lanes share one, each
+        // doing its pipeline and drawing every nph-th of its rows (1
+        // shooter over 20,000 triangles at hemicube 256: 28.7 us with a
+        // lane per triangle, 27.2).
+        // Triangles to clip are queued by their wavefront and taken one
+        // per step.
+        const uint32_t nt = cull ? nt_ : 16u * (g1 - g0);
+        uint32_t lb = 0; // log2 of the triangles per step
+        while (lb < 6u && (NW << lb) < nt)
+            ++lb;
+        const uint32_t bs = 1u << lb;
+        uint32_t qi = wv * bs, cn = 0;
+        uint16_t *const cq = clipq[wv];
+        while (true) {
+            const bool batch = qi < nt && cn <= kDirClip - 64u;
+            if (!batch && cn == 0)
+                break;
+            wave_lds_sync();
+            const TileView &vw = reload(v);
+            SV A, B, C;
+            uint32_t id = 0;
+            bool have = false;
+            // row phase of the lane's triangle, log2 of the phases
+            uint32_t ph = 0, lph = 0;
+            if (batch) {
+                bool clip = false;
+                uint32_t tr = ntc;
+                const uint32_t i = qi + (lane & (bs - 1u));
+                ph = lane >> lb;
+                lph = 6u - lb;
+                if (i < nt) {
+                    tr = cull ? tq[i] : 16u * glist[g0 + (i >> 4)] + (i & 15u);
+                }
+                if (tr < ntc) {
+                    const uint32_t t = tb + tr;
+                    float vx[3][3];
 #pragma unroll
-                        for (int k = 0; k < 3; ++k)
+                    for (int k = 0; k < 3; ++k)
 #pragma unroll
-                            for (int c = 0; c < 3; ++c)
-                                vx[k][c] = a.tri[(size_t)(3 * k + c) * a.ntri + t];
-                        id = a.tri_patch[t] + 1u;
-                        CV4 poly[3];
-                        transform3(vw.mvp, vx, poly);
-                        const TriClass cl = classify_tri(poly, vw.scis);
-                        clip = cl == kTriClip && ph == 0u;
-                        have = cl == kTriIn;
-                        if (have) {
-                            A = project(poly[0], halfW);
-                            B = project(poly[1], halfW);
-                            C = project(poly[2], halfW);
-                        }
+                        for (int c = 0; c < 3; ++c)
+                            vx[k][c] = a.tri[(size_t)(3 * k + c) * a.ntri + t];
+                    id = a.tri_patch[t] + 1u;
+                    CV4 poly[3];
+                    transform3(vw.mvp, vx, poly);
+                    const TriClass cl = classify_tri(poly, vw.scis);
+                    clip = cl == kTriClip && ph == 0u;
+                    have = cl == kTriIn;
+                    if (have) {
+                        A = project(poly[0], halfW);
+                        B = project(poly[1], halfW);
+                        C = project(poly[2], halfW);
                     }
-                    qi += NW * bs;
-                    const uint64_t m = __ballot(clip);
-                    if (clip)
-                        cq[cn + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)tr;
-                    cn += (uint32_t)__popcll(m);
-                } else {
-                    const uint32_t t = t0 + cq[--cn];
-                    CV4 p;
+                }
+                qi += NW * bs;
+                const uint64_t m = __ballot(clip);
+                if (clip)
+                    cq[cn + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)tr;
+                cn += (uint32_t)__popcll(m);
+            } else {
+                const uint32_t t = tb + cq[--cn];
+                CV4 p;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    p.c[r] = 0.0f;
+                if (lane < 3) {
+                    const float tx = a.tri[(size_t)(3 * lane + 0) * a.ntri + t];
+                    const float ty = a.tri[(size_t)(3 * lane + 1) * a.ntri + t];
+                    const float tz = a.tri[(size_t)(3 * lane + 2) * a.ntri + t];
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        p.c[r] = 0.0f;
-                    if (lane < 3) {
-                        const float tx = a.tri[(size_t)(3 * lane + 0) * a.ntri + t];
-                        const float ty = a.tri[(size_t)(3 * lane + 1) * a.ntri + t];
-                        const float tz = a.tri[(size_t)(3 * lane + 2) * a.ntri + t];
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            p.c[r] = vw.mvp[0 * 4 + r] * tx + vw.mvp[1 * 4 + r] * ty +
-                                     vw.mvp[2 * 4 + r] * tz + vw.mvp[3 * 4 + r];
-                    }
-                    id = a.tri_patch[t] + 1u;
-                    const int n = clip_polygon_wave(p, lp[wv], &a.counters[kCntOverflow]);
-                    if (n >= 3)
-                        have = clip_fan(p, n, halfW, A, B, C);
+                        p.c[r] = vw.mvp[0 * 4 + r] * tx + vw.mvp[1 * 4 + r] * ty +
+                                 vw.mvp[2 * 4 + r] * tz + vw.mvp[3 * 4 + r];
                 }
-                RasterRec r;
-                int32_t bx0 = 0, by0 = 0, bx1 = -1, by1 = -1;
-                if (have) {
-                    int64_t area2;
-                    have = snapped_bbox(A, B, C, x0, y0, x1, y1, area2, bx0, by0, bx1, by1);
-                    if (have)
-                        make_record(A, B, C, area2, id, r);
-                }
-                // Small ones by their lanes, which takes as long as the
-                // largest; the others by the whole wavefront, one after the
-                // other.
-                const uint32_t nph = 1u << lph;
-                const uint32_t rows = ((uint32_t)(by1 - by0 + 1) + nph - 1u) >> lph;
-                const bool small = have && (uint32_t)(bx1 - bx0 + 1) * rows <= a.small_px &&
-                                   span_within(r, kLane32Span);
-                if (small)
-                    draw_lane32(r, 0, 0, bx0, bx1, by0, by1, ox, oy, a.tshift, tk, ph, nph);
-                for (uint64_t m = __ballot(have && !small && ph == 0u); m; m &= m - 1) {
-                    const int l = __ffsll((long long)m) - 1;
-                    RasterRec u;
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        u.x[k] = __builtin_amdgcn_readlane(r.x[k], l);
-                        u.y[k] = __builtin_amdgcn_readlane(r.y[k], l);
-                    }
-                    u.dzdx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.dzdx), l));
-                    u.dzdy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.dzdy), l));
-                    u.z0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.z0), l));
-                    u.id = (uint32_t)__builtin_amdgcn_readlane((int)r.id, l);
-                    draw_big(u, __builtin_amdgcn_readlane(bx0, l), __builtin_amdgcn_readlane(by0, l),
-                             __builtin_amdgcn_readlane(bx1, l), __builtin_amdgcn_readlane(by1, l),
-                             ox, oy, a.tshift, tk);
-                }
+                id = a.tri_patch[t] + 1u;
+                const int n = clip_polygon_wave(p, lp[wv], &a.counters[kCntOverflow]);
+                if (n >= 3)
+                    have = clip_fan(p, n, halfW, A, B, C);
             }
-            __syncthreads(); // the queues are the next groups'
+            RasterRec r;
+            int32_t bx0 = 0, by0 = 0, bx1 = -1, by1 = -1;
+            if (have) {
+                int64_t area2;
+                have = snapped_bbox(A, B, C, x0, y0, x1, y1, area2, bx0, by0, bx1, by1);
+                if (have)
+                    make_record(A, B, C, area2, id, r);
+            }
+            // Small ones by their lanes, which takes as long as the
+            // largest; the others by the whole wavefront, one after the
+            // other.
+            const uint32_t nph = 1u << lph;
+            const uint32_t rows = ((uint32_t)(by1 - by0 + 1) + nph - 1u) >> lph;
+            const bool small = have && (uint32_t)(bx1 - bx0 + 1) * rows <= a.small_px &&
+                               span_within(r, kLane32Span);
+            if (small)
+                draw_lane32(r, 0, 0, bx0, bx1, by0, by1, ox, oy, a.tshift, tk, ph, nph);
+            for (uint64_t m = __ballot(have && !small && ph == 0u); m; m &= m - 1) {
+                const int l = __ffsll((long long)m) - 1;
+                RasterRec u;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    u.x[k] = __builtin_amdgcn_readlane(r.x[k], l);
+                    u.y[k] = __builtin_amdgcn_readlane(r.y[k], l);
+                }
+                u.dzdx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.dzdx), l));
+                u.dzdy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.dzdy), l));
+                u.z0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.z0), l));
+                u.id = (uint32_t)__builtin_amdgcn_readlane((int)r.id, l);
+                draw_big(u, __builtin_amdgcn_readlane(bx0, l), __builtin_amdgcn_readlane(by0, l),
+                         __builtin_amdgcn_readlane(bx1, l), __builtin_amdgcn_readlane(by1, l),
+                         ox, oy, a.tshift, tk);
+            }
         }
+        __syncthreads(); // the queues are the next groups'
     }
 
     __syncthreads(); // the keys are complete
@@ -669,9 +659,11 @@ bool direct_wins(uint32_t k, uint32_t W, uint32_t ntri, uint32_t *T)
 {
     const uint32_t wg = k * direct_tiles(W, 32);
     *T = wg <= 64 ? 16u : 32u;
+    if (ntri > 64u * kDirMax) // what k_direct's lists hold
+        return false;
     if (wg > 256)
         return wg <= 384 && W >= 128 && ntri <= 8192;
-    return ntri <= 600u * direct_tiles(W, *T) && ntri <= (wg <= 64 ? 64 * kDirChunk : 34816u);
+    return ntri <= 600u * direct_tiles(W, *T) && (wg <= 64 || ntri <= 34816u);
 }
 
 void launch_direct(const DirectArgs &args, uint32_t T, hipStream_t st)

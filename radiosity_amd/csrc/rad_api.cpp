@@ -160,7 +160,7 @@ static uint32_t lane_limit(const rad_ctx *c, uint32_t k)
 static bool split_render(const rad_ctx *c, uint32_t k)
 {
     uint32_t T;
-    if (c->pk.nscene && c->bb.nblk * 256u <= kSplitPack)
+    if (!c->st2 || (c->pk.nscene && c->bb.nblk * 256u <= kSplitPack))
         return false;
     return k >= kSplitMin && k * c->bb.ntiles >= kSplitBins && !c->timing &&
            !use_direct(c, k, &T);
@@ -459,6 +459,22 @@ int drop_scene(rad_ctx *c, int rc)
     return rc;
 }
 
+// The stream and events of the second half of split passes, for a context
+// whose passes may be (split_render).  Most contexts are too small, and a
+// stream is the dearest part of making one: 15 to 350 us, by the hardware
+// queues in use.
+int second_stream(rad_ctx *c)
+{
+    if (c->st2 || c->K < kSplitMin || c->bb.nbins < kSplitBins)
+        return RAD_OK;
+    if (!c->ev_fork)
+        HIPCHK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
+    if (!c->ev_join)
+        HIPCHK(c, hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
+    HIPCHK(c, hipStreamCreate(&c->st2));
+    return RAD_OK;
+}
+
 // Screen tile side T (8, 16, 32) and the in-lane triangle limit; (re)sizes
 // the per-(shooter, tile) bin arrays.
 int set_tiles(rad_ctx *c, uint32_t T, uint32_t small_px)
@@ -493,8 +509,8 @@ int set_tiles(rad_ctx *c, uint32_t T, uint32_t small_px)
     c->cfg.tile_px = T;
     c->cfg.small_tri_px = small_px;
     drop_graph(c);
-    if (c->npatch && (rc = bin_lists(c)))
-        return drop_scene(c, rc); // no pass without lists
+    if ((c->npatch && (rc = bin_lists(c))) || (rc = second_stream(c)))
+        return drop_scene(c, rc); // no pass without them
     return RAD_OK;
 }
 
@@ -547,12 +563,6 @@ int rad_create(const rad_config *cfg, rad_ctx **out)
     hipError_t e = hipGetDevice(&c->device);
     if (e == hipSuccess)
         e = hipStreamCreate(&c->st);
-    if (e == hipSuccess)
-        e = hipStreamCreate(&c->st2);
-    if (e == hipSuccess)
-        e = hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming);
-    if (e == hipSuccess)
-        e = hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming);
     if (e != hipSuccess) {
         rad_destroy(c);
         return RAD_E_HIP;

@@ -16,6 +16,7 @@ size_t live_bytes, limit = SIZE_MAX;    // hipMalloc refuses what would exceed l
 size_t largest = SIZE_MAX;              // and any single one beyond largest
 std::map<const void *, std::string> kernels;
 void (*launched)(const char *name, void **args);
+size_t streams, unstreamed; // streams alive; launches on none of them
 float elapsed; // each hipEventElapsedTime reads 1 ms more than the last
 
 } // namespace
@@ -23,6 +24,8 @@ float elapsed; // each hipEventElapsedTime reads 1 ms more than the last
 extern "C" {
 
 size_t double_live(void) { return live.size(); }
+size_t double_streams(void) { return streams; }
+size_t double_unstreamed(void) { return unstreamed; }
 size_t double_live_bytes(void) { return live_bytes; }
 void double_limit(size_t bytes) { limit = bytes; }
 void double_largest(size_t bytes) { largest = bytes; }
@@ -88,10 +91,20 @@ void __hipRegisterFunction(void **, const void *host, char *, const char *name, 
 {
     kernels[host] = name;
 }
-hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
-hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t)
+static hipStream_t called_on;
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t st)
 {
+    called_on = st;
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *st)
+{
+    *st = called_on;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t st)
+{
+    unstreamed += st == nullptr;
     if (launched)
         launched(kernels[f].c_str(), args);
     return hipSuccess;
@@ -130,14 +143,22 @@ static hipError_t handle(void **h)
     *h = malloc(1);
     return hipSuccess;
 }
-hipError_t hipStreamCreate(hipStream_t *s) { return handle((void **)s); }
+hipError_t hipStreamCreate(hipStream_t *s)
+{
+    ++streams;
+    return handle((void **)s);
+}
 hipError_t hipStreamDestroy(hipStream_t s)
 {
+    --streams;
     free(s);
     return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t st, hipEvent_t e, unsigned)
+{
+    return st && e ? hipSuccess : hipErrorInvalidHandle;
+}
 hipError_t hipEventCreate(hipEvent_t *e) { return handle((void **)e); }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return handle((void **)e); }
 hipError_t hipEventDestroy(hipEvent_t e)
@@ -145,7 +166,10 @@ hipError_t hipEventDestroy(hipEvent_t e)
     free(e);
     return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t st)
+{
+    return st && e ? hipSuccess : hipErrorInvalidHandle;
+}
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)
 {

@@ -162,3 +162,29 @@ def test_autotune_times_direct_passes_with_the_limit_it_chose(on_double):
         assert s.autotune(2)[1] == 16
         assert limits == [64] + 3 * [16], limits
         """)
+
+
+def test_second_stream_where_passes_may_be_split(on_double):
+    """A context has the second half's stream from 16 shooters and 8,192 tiles
+    on, at whatever tile side it comes to that."""
+    on_double("""
+        for f in (D.double_streams, D.double_unstreamed):
+            f.restype = C.c_size_t
+        sc = R.Scene.boxes(nboxes=4, room=(5.0, 3.0, 5.0), target_tris=3000, nlights=2, seed=3)
+        def run(streams, tune=None, **kw):
+            s = R.Solver(**kw)
+            s.upload(sc)
+            s.step(3)
+            assert D.double_streams() == streams, (kw, D.double_streams())
+            if tune:
+                s.autotune(1)  # tiles of 16 and 32
+                s.step(3)
+                assert D.double_streams() == tune, (kw, D.double_streams())
+            s.close()
+            assert D.double_streams() == 0
+        run(1, hemicube=16, hemicubes=1)
+        run(1, hemicube=128, hemicubes=64, tune=2)
+        run(1, hemicube=512, hemicubes=15, tune=1)
+        run(2, hemicube=256, hemicubes=64, graph_passes=2)
+        assert D.double_unstreamed() == 0
+        """)

@@ -664,12 +664,10 @@ __device__ static uint32_t cull_faces(const float *__restrict__ sm, const float 
     // whose coordinate comes within the margin of it
     uint32_t mask = (fabsf(pb) >= T ? (pb > 0.0f ? 1u : 2u) : 0u) |
                     (fabsf(pc) >= T ? (pc > 0.0f ? 4u : 8u) : 0u) | (pa >= T ? 16u : 0u);
-    // (of one face whichever faces this workgroup looks at)
-    const bool one = (mask & (mask - 1u)) == 0u;
-    mask &= faces;
     const float l1 = fabsf(cx) + fabsf(cy) + fabsf(cz);
     const float db = fmaf(-4e-6f * l1, back.w, fmaf(cz, back.z, fmaf(cy, back.y, cx * back.x)));
-    if (db > 0.0f && one) {
+    // (one face of all five, whichever this workgroup looks at)
+    if (db > 0.0f && (mask & (mask - 1u)) == 0u) {
         const float wmin = far - rho - mq, wmax = far + rho + mq;
         const float S = __builtin_amdgcn_fmed3f(fabsf(pa), fabsf(pb), fabsf(pc)) + rho;
         const float em = 2e-6f * (fabsf(ex) + fabsf(ey) + fabsf(ez));
@@ -679,7 +677,7 @@ __device__ static uint32_t cull_faces(const float *__restrict__ sm, const float 
             a * halfW * back.w > w3 * dw)
             mask = 0u;
     }
-    return mask;
+    return mask & faces;
 }
 
 // The launch order of the bins [bin0, bin0 + n) for the tile kernel, largest

@@ -404,24 +404,23 @@ int one_pass(rad_ctx *c, bool do_select, size_t evbase, bool chain_in = false,
 
 // The bins' lists: room for 16 times the records per bin of a scene spread
 // evenly over the tiles, within 4 GiB in all, or for half of it and so on where
-// the device has no memory for that (1.6 GB for 64 shooters of 200,000
+// the device has no memory for that (0.8 GB for 64 shooters of 200,000
 // triangles at hemicube 256).  A fuller bin's workgroup makes its list in the
-// pool (whole_list), so the size is no limit.  Allocated after the buffers that
-// a scene cannot do without.
+// pool (whole_list), so the size is no limit, but each costs a walk over all
+// records: with 8 times that pass took as long as with 32 times (18.9 ms for
+// 60), with 8 times a half 24.3.  Allocated after the buffers that a scene
+// cannot do without.
 int bin_lists(rad_ctx *c)
 {
-    const uint64_t ntri = (uint64_t)c->bb.nblk * 256;
-    uint32_t cap = 256;
-    while (cap < 65536 && (uint64_t)cap * c->bb.ntiles < 16 * ntri)
-        cap *= 2;
-    while (cap > 256 && (uint64_t)c->bb.nbins * cap > (1ull << 30))
-        cap /= 2;
+    const uint64_t even = (uint64_t)c->bb.nblk * 256 / c->bb.ntiles;
+    uint64_t cap = std::min<uint64_t>(std::max<uint64_t>(16 * even, 256), 65536);
+    cap = std::min((cap + 63) / 64 * 64, std::max<uint64_t>((1ull << 30) / c->bb.nbins, 256));
     int rc;
     while ((rc = dalloc(c, &c->bb.list, (size_t)c->bb.nbins * cap)) && cap > 16) {
         c->err.clear();
         cap /= 2;
     }
-    c->bb.bin_cap = cap;
+    c->bb.bin_cap = (uint32_t)cap;
     return rc;
 }
 

@@ -227,8 +227,9 @@ int rad_face_mvps(rad_ctx *ctx, uint32_t patch, float *out80);
 
 /* Average device time (ms) per launch of each kernel of the last
  * rad_step/rad_run, measured with HIP events on the context stream:
- * out[0] select, [1] prepare+clear, [2] raster setup, [3] binning (scan +
- * fill), [4] tile raster with the fused ProcessHemicube, [5] shoot; also the
+ * out[0] select, [1] prepare+clear, [2] raster setup (records into the
+ * tiles' lists), [3] launch order of the tiles and clipped triangles, [4] tile
+ * raster with the fused ProcessHemicube, [5] shoot; also the
  * number of timed passes.  A pass drawn without bins (small passes, tile_px 0)
  * is [4] as a whole; its [2] and [3] are 0. */
 int rad_kernel_times(rad_ctx *ctx, int enable, double *out6, uint64_t *npasses);
@@ -258,8 +259,8 @@ int rad_debug_bins(rad_ctx *ctx, uint32_t *out_or_null, uint32_t *ntiles, uint32
 int rad_debug_counters(rad_ctx *ctx, uint32_t *out8, uint32_t *out_caps_or_null);
 
 /* Diagnostics (no counterpart in the reference): the candidate pool of the
- * POWER selection in captured passes.  Inside a graph, a pass's selection
- * may take the K largest keys from a pool of every receiver whose key is at
+ * POWER selection of passes in a row.  Inside a graph or a call of several
+ * passes, a pass's selection may take the K largest keys from a pool of every receiver whose key is at
  * least a bound, which the previous pass's shoot collected; it does so only
  * when the pool holds K keys (then they are exact) and at most `cap`, else
  * it scans every patch.  cap != 0 sets that most (1 .. 16384, default 16384)

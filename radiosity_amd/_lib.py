@@ -509,7 +509,7 @@ class Solver:
         return d
 
     def debug_pool(self, cap=0):
-        """Candidate pool of the POWER selection in captured passes: cap != 0
+        """Candidate pool of the POWER selection of passes in a row: cap != 0
         sets the most keys a selection takes from it (else it scans every
         patch); returns the selections taken from the pool, the full scans,
         the times its bound was set and whether it is set now."""

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 # Triangles just behind their drawn side, each on two or more faces of a shooter
 # at the origin looking along +z (up +y) and with a vertex at the near plane: on
 # some face the clipped polygon has a counter-clockwise part of some pixels
-# (found by a search over 880 million triangles near the cull's threshold).
+# (found by a search over 947 million triangles near the cull's threshold).
 # Nine coordinates each, hexadecimal.
 TRIANGLES = """
     1.a1aeecp-5 1.d83594p-5 1.a87ceap-6 1.e42f9ap-5 1.4799dp-7 1.143a4cp-7 1.319144p-4 1.c0abe2p-5 1.de960ep-6
